@@ -1,9 +1,5 @@
-// MFMA GEMM kernels for gfx950 (CDNA4).
-//
-// Block tile 128 x 128, 256 threads = 4 wave64s in a 2 x 2 arrangement, each
-// wave owning a 64 x 64 sub-tile as 4 x 4 MFMA 16x16 tiles.  Operands are
-// staged through LDS in k-chunks; the next chunk is fetched into registers
-// while the current one is multiplied.
+// MFMA GEMM launcher for gfx950 (CDNA4), the batched split-BF16x3 kernel and
+// the split-K reduction.  The FP64 / FP32 kernels are in gemm_k4.hpp.
 //
 // MFMA operand roles: the instruction's "A" operand is fed with B(k,n) and
 // its "B" operand with A(m,k), so the 16x16 result tile is C^T in MFMA
@@ -23,236 +19,10 @@
 #include "engine.hpp"
 #include "gemm.hpp"
 #include "gemm_device.hpp"
+#include "gemm_k4.hpp"
 #include "tape.hpp"
 
 namespace sisi {
-
-// ---------------------------------------------------------------------------
-// FP64 / FP32 kernel (LDS element type LT; k-chunk 16; MFMA k-step 4)
-// ---------------------------------------------------------------------------
-
-template <typename LT>
-__device__ __forceinline__ void mfma_k4(d4 &acc, double a, double b);
-
-// Body of the FP64 / FP32 kernel for output tile `pid` (of tiles_m x
-// tiles_n), k-split `ks` and batch entry `bz` (the eager kernel passes its
-// block indices, the grouped kernel of the batched solver the indices of one
-// record's blocks).
-template <int PREC, bool AK, bool BNF>
-__device__ __forceinline__ void gemm_k4_body(const GemmArgs &g, int pid, int ks, int bz) {
-  using LT = typename std::conditional<PREC == SISI_FP64, double, float>::type;
-  using AT = typename std::conditional<PREC == SISI_FP64, d4, f4>::type;
-  constexpr int BK = 16;
-  constexpr int PAD = (PREC == SISI_FP64) ? 2 : 4;
-  // result layout of the 16x16 tile: row (here n) = LSTR*(lane/16) + RSTR*reg
-  // (v_mfma_f64_16x16x4f64: lane/16 + 4*reg; the f32 form: 4*(lane/16) + reg)
-  constexpr int LSTR = (PREC == SISI_FP64) ? 1 : 4;
-  constexpr int RSTR = (PREC == SISI_FP64) ? 4 : 1;
-  __shared__ LT As[BK][BM + PAD];
-  __shared__ LT Bs[BK][BN + PAD];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: scalar branches
-  int tm, tn;
-  tile_coords(g, pid, tm, tn);
-  const int m0 = tm * BM, n0 = tn * BN;
-  const int kbeg = ks * g.kchunk;
-  const int kend = min(g.K, kbeg + g.kchunk);
-
-  const double *A = g.A + int64_t(bz) * g.bsa;
-  const double *B = g.B + int64_t(bz) * g.bsb;
-
-  double ra[8], rb[8];
-
-  // Out-of-range elements load from a clamped (in-range) address, so the
-  // loads need no branch; they are zeroed when the chunk is written to LDS
-  // (multiplying by 0.0, which the compiler cannot fold away), so the loads
-  // stay in flight across the MFMAs of the previous chunk.
-  const int mlast = g.M - 1, nlast = g.N - 1;
-  int lk0 = 0;  // k0 of the chunk held in ra/rb
-  auto load = [&](int k0) {
-    const int klast = kend - 1;
-    lk0 = k0;
-    if (!AK) {  // A m-fastest: 32 threads x 4 consecutive m, k rows t/32 and +8
-      const int mm = (tid & 31) * 4, kk = tid >> 5;
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int k = min(k0 + kk + 8 * h, klast);
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          ra[h * 4 + j] = A[int64_t(min(m0 + mm + j, mlast)) * g.sam + int64_t(k) * g.sak];
-      }
-    } else {  // A k-fastest: 16 threads along k, m = t/16 + 16 j
-      const int kk = tid & 15, mm = tid >> 4;
-      const int k = min(k0 + kk, klast);
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        ra[j] = A[int64_t(min(m0 + mm + 16 * j, mlast)) * g.sam + int64_t(k) * g.sak];
-    }
-    if (BNF) {  // B n-fastest
-      const int nn = (tid & 31) * 4, kk = tid >> 5;
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int k = min(k0 + kk + 8 * h, klast);
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          rb[h * 4 + j] = B[int64_t(k) * g.sbk + int64_t(min(n0 + nn + j, nlast)) * g.sbn];
-      }
-    } else {  // B k-fastest
-      const int kk = tid & 15, nn = tid >> 4;
-      const int k = min(k0 + kk, klast);
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        rb[j] = B[int64_t(k) * g.sbk + int64_t(min(n0 + nn + 16 * j, nlast)) * g.sbn];
-    }
-  };
-
-  auto store = [&]() {
-    auto z = [](bool ok) { return ok ? 1.0 : 0.0; };
-    if (!AK) {
-      const int mm = (tid & 31) * 4, kk = tid >> 5;
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          As[kk + 8 * h][mm + j] =
-              LT(ra[h * 4 + j] * z(m0 + mm + j <= mlast && lk0 + kk + 8 * h < kend));
-    } else {
-      const int kk = tid & 15, mm = tid >> 4;
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        As[kk][mm + 16 * j] = LT(ra[j] * z(m0 + mm + 16 * j <= mlast && lk0 + kk < kend));
-    }
-    if (BNF) {
-      const int nn = (tid & 31) * 4, kk = tid >> 5;
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          Bs[kk + 8 * h][nn + j] =
-              LT(rb[h * 4 + j] * z(n0 + nn + j <= nlast && lk0 + kk + 8 * h < kend));
-    } else {
-      const int kk = tid & 15, nn = tid >> 4;
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        Bs[kk][nn + 16 * j] = LT(rb[j] * z(n0 + nn + 16 * j <= nlast && lk0 + kk < kend));
-    }
-  };
-
-  AT acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = AT{0, 0, 0, 0};
-
-  const int wm = (wave & 1) * 64, wn = (wave >> 1) * 64;
-  const int l16 = lane & 15, lk = lane >> 4;
-  // a wave whose 64x64 sub-tile lies wholly outside the output (ragged edge
-  // tiles) skips its MFMAs; the condition is uniform per wave
-  const bool active = (m0 + wm < g.M) && (n0 + wn < g.N);
-  auto mma = [&]() {
-#pragma unroll
-    for (int kq = 0; kq < BK / 4; ++kq) {
-      const int k = kq * 4 + lk;
-      LT av[4], bv[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) av[i] = As[k][wm + i * 16 + l16];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) bv[j] = Bs[k][wn + j * 16 + l16];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          if constexpr (PREC == SISI_FP64)
-            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bv[j], av[i], acc[i][j], 0, 0, 0);
-          else
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[j], av[i], acc[i][j], 0, 0, 0);
-        }
-    }
-  };
-
-  int k0 = kbeg;
-  if (k0 < kend) load(k0);
-  while (k0 < kend) {
-    store();
-    __syncthreads();
-    const int k1 = k0 + BK;
-    if (k1 < kend) load(k1);
-    if (active) mma();
-    __syncthreads();
-    k0 = k1;
-  }
-
-  // epilogue
-  if (g.ksplit == 1) {
-    double *C = g.C + int64_t(bz) * g.bsc;
-    // row offsets once per row, each column offset once per column (the
-    // output splits cost divisions)
-    int64_t om[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int m = m0 + wm + i * 16 + l16;
-      om[i] = m < g.M ? out_off_m(g, m) : -1;
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int n = n0 + wn + j * 16 + LSTR * lk + RSTR * r;
-        if (n >= g.N) continue;
-        const int64_t on = out_off_n(g, n);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if (om[i] < 0) continue;
-          const int64_t o = om[i] + on;
-          double v = g.alpha * double(acc[i][j][r]);
-          if (g.beta != 0.0) v += g.beta * C[o];
-          C[o] = v;
-        }
-      }
-  } else {
-    double *W = g.work + (int64_t(bz) * g.ksplit + ks) * int64_t(g.M) * g.N;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int m = m0 + wm + i * 16 + l16;
-      if (m >= g.M) continue;
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int n = n0 + wn + j * 16 + LSTR * lk + RSTR * r;
-          if (n < g.N) W[m + int64_t(n) * g.M] = double(acc[i][j][r]);
-        }
-    }
-  }
-}
-
-template <int PREC, bool AK, bool BNF>
-__global__ __launch_bounds__(256, 2) void gemm_k4_kernel(GemmArgs g) {
-  gemm_k4_body<PREC, AK, BNF>(g, blockIdx.x, blockIdx.y, blockIdx.z);
-}
-
-// Grouped launch of n products (batched solver): record p owns the blocks
-// [start[p], start[p + 1]): tiles_m * tiles_n per k-split and batch entry.
-template <int PREC, bool AK, bool BNF>
-__global__ __launch_bounds__(256, 2) void gemm_k4_grouped(const GemmArgs *const *args,
-                                                          const unsigned *__restrict__ start,
-                                                          int n) {
-  int lo = 0, hi = n - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (start[mid] <= blockIdx.x) lo = mid;
-    else hi = mid - 1;
-  }
-  // the record is read in place (a copy kept the whole struct live in
-  // registers and made the kernel spill)
-  const GemmArgs &g = *args[lo];
-  const int tiles = g.tiles_m * g.tiles_n;
-  const int local = int(blockIdx.x - start[lo]);
-  const int r = local / tiles;
-  gemm_k4_body<PREC, AK, BNF>(g, local % tiles, r % g.ksplit, r / g.ksplit);
-}
 
 // ---------------------------------------------------------------------------
 // BF16x3 kernel (k-chunk 32 = one MFMA k-step; LDS rows along k)
@@ -523,14 +293,6 @@ __global__ __launch_bounds__(256) void gemm_reduce_grouped(const GemmArgs *const
 // Launcher
 // ---------------------------------------------------------------------------
 
-template <int PREC>
-static void launch_k4(GemmArgs &g, dim3 grid, hipStream_t s, bool AK, bool BNF) {
-  if (!AK && !BNF) hipLaunchKernelGGL((gemm_k4_kernel<PREC, false, false>), grid, dim3(256), 0, s, g);
-  else if (!AK && BNF) hipLaunchKernelGGL((gemm_k4_kernel<PREC, false, true>), grid, dim3(256), 0, s, g);
-  else if (AK && !BNF) hipLaunchKernelGGL((gemm_k4_kernel<PREC, true, false>), grid, dim3(256), 0, s, g);
-  else hipLaunchKernelGGL((gemm_k4_kernel<PREC, true, true>), grid, dim3(256), 0, s, g);
-}
-
 static void launch_b3(GemmArgs &g, dim3 grid, hipStream_t s, bool AK, bool BNF) {
   if (!AK && !BNF) hipLaunchKernelGGL((gemm_bf16x3_kernel<false, false>), grid, dim3(256), 0, s, g);
   else if (!AK && BNF) hipLaunchKernelGGL((gemm_bf16x3_kernel<false, true>), grid, dim3(256), 0, s, g);
@@ -562,16 +324,79 @@ int round_filling_split(int64_t groups, int64_t s, int64_t smax, int cus) {
   return int(best);
 }
 
-static int64_t env_int(const char *name, int64_t fallback) {
-  const char *v = getenv(name);
-  return v != nullptr && *v != 0 ? int64_t(atoll(v)) : fallback;
-}
-
 static void set_ksplit(GemmArgs &g, int ksplit, int kq);
 
-// Tile grid, load mappings and split-K plan of one FP64 / FP32 / batched
-// split-BF16x3 product (fields of g filled in); returns the load mappings.
-static void plan_k4(GemmArgs &g, int precision, int cus, bool &AKf, bool &BNFf) {
+// Tile and split-K of an FP64 / FP32 product, by the estimated cycles of each
+// (tile, split) pair.  What the estimate holds, fitted to a sweep of tiles and
+// splits over 21 shapes (M, N from 28 to 78400, K from 17 to 200000), where
+// it picks the fastest pair or one within 10 % of it:
+//  - a workgroup alone on its CU takes the MFMA cycles of its tile per chunk
+//    of 16 k plus kChunkLatency for the chain of LDS store, barrier and
+//    fragment reads; resident workgroups overlap these chains, and then a
+//    tile's chunk costs kTileCycles;
+//  - a split pays the launch of the reduction and its partial sums.
+// 500 x 500 x 300: 32 x 32 10.0 us, 64 x 64 16.7, 128 x 128 25.2 (each with
+// its best split); 1500^3: 157, 171, 220; 4096^3: -, 2417, 2141.
+constexpr int kResident[kNumTiles] = {2, 4, 8};
+constexpr double kTileMfma[2][kNumTiles] = {{4096, 1024, 256}, {2048, 512, 128}};
+constexpr double kTileCycles[2][kNumTiles] = {{4420, 1250, 400}, {2400, 800, 320}};
+constexpr double kChunkLatency = 700.0;
+constexpr double kBlockCycles = 3000.0;   // prologue and epilogue of a workgroup
+constexpr double kReduceCycles = 9000.0;  // launch of the split-K reduction
+constexpr double kReduceBytes = 1300.0;   // bytes per cycle of the partial sums' traffic
+
+struct TilePlan {
+  int tile = 0, ksplit = 1;
+};
+
+static double tile_cycles(const GemmArgs &g, int precision, int cus, int t, int ks) {
+  const int bt = kTiles[t], p = precision == SISI_FP64 ? 0 : 1;
+  const int64_t tiles = ((g.M + bt - 1) / bt) * int64_t((g.N + bt - 1) / bt) * g.batch;
+  const int64_t chunks = ((g.K + ks - 1) / ks + kTileK - 1) / kTileK;
+  const int64_t per_cu = (tiles * ks + cus - 1) / cus;
+  const double lone = kTileMfma[p][t] + kChunkLatency;
+  auto round = [&](int64_t n) {
+    return double(chunks) * std::max(double(n) * kTileCycles[p][t], lone) + kBlockCycles;
+  };
+  const int64_t rounds = per_cu / kResident[t], rest = per_cu % kResident[t];
+  double c = double(rounds) * round(kResident[t]) + (rest ? round(rest) : 0.0);
+  if (ks > 1)
+    c += kReduceCycles +
+         8.0 * double(2 * ks + 2) * double(g.M) * g.N * g.batch / kReduceBytes;  // W twice, C
+  return c;
+}
+
+static TilePlan choose_tile(const GemmArgs &g, int precision, int cus) {
+  static const char *const env_tile = getenv("SISI_GEMM_TILE");
+  TilePlan best;
+  double best_c = 1e300;
+  for (int t = 0; t < kNumTiles; ++t) {
+    if (env_tile && *env_tile && atoi(env_tile) != t) continue;
+    for (int ks : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64, 96, 128, 192, 256}) {
+      // at least four chunks per part, and partial sums of at most 2 GB
+      if (ks > 1 && (g.K < ks * 4 * kTileK ||
+                     double(ks) * g.M * double(g.N) * g.batch > double(int64_t(1) << 28)))
+        break;
+      const double c = tile_cycles(g, precision, cus, t, ks);
+      if (c < best_c * 0.999) {
+        best_c = c;
+        best.tile = t;
+        best.ksplit = ks;
+      }
+    }
+  }
+  return best;
+}
+
+// How a product runs: tile of the FP64 / FP32 kernels (the batched
+// split-BF16x3 kernel has one of 128 x 128) and load mapping.
+struct K4Plan {
+  int tile = 0, map = 0;
+};
+
+// Tile grid, load mapping and split-K plan of one FP64 / FP32 / batched
+// split-BF16x3 product (fields of g filled in).
+static K4Plan plan_k4(GemmArgs &g, int precision, int cus, bool taped) {
   if (g.K < 0) g.K = 0;  // K == 0 gives C = beta * C through the epilogue
   SISI_REQUIRE(g.sam == 1 || g.sak == 1 || g.K <= 1 || g.M <= 1, SISI_ERR_INVALID,
                "gemm: A needs a unit stride");
@@ -579,12 +404,8 @@ static void plan_k4(GemmArgs &g, int precision, int cus, bool &AKf, bool &BNFf) 
                "gemm: B needs a unit stride");
   // The address formula is the same for every load mapping; the mapping only
   // decides which index consecutive threads walk (coalescing).
-  AKf = (g.sak == 1) && (g.sam != 1);
-  BNFf = (g.sbn == 1) && (g.sbk != 1);
-  g.tiles_m = (g.M + BM - 1) / BM;
-  g.tiles_n = (g.N + BN - 1) / BN;
-  const int64_t tiles = int64_t(g.tiles_m) * g.tiles_n;
-  SISI_REQUIRE(tiles < (int64_t(1) << 31), SISI_ERR_INVALID, "gemm: too many tiles");
+  K4Plan p;
+  p.map = ((g.sak == 1 && g.sam != 1) ? 2 : 0) + ((g.sbn == 1 && g.sbk != 1) ? 1 : 0);
   g.split_out = !(g.dm0 >= g.M && g.dn0 >= g.N);
   {
     static const int env_map = getenv("SISI_GEMM_XCD") ? atoi(getenv("SISI_GEMM_XCD")) : 1;
@@ -592,21 +413,32 @@ static void plan_k4(GemmArgs &g, int precision, int cus, bool &AKf, bool &BNFf) 
     g.xcd_map = env_map;
     g.group = env_group > 0 ? env_group : 8;
   }
-  const int kq = (precision == SISI_BF16X3) ? 32 : 16;
-  // split-K when the tile grid alone cannot fill the 256 CUs: about `want`
-  // workgroups, each with at least `minsteps` k-chunks, at most `maxsplit`
-  // partial sums
-  static const int64_t want = env_int("SISI_GEMM_SPLIT_WANT", 1024);
-  static const int64_t minsteps = std::max<int64_t>(1, env_int("SISI_GEMM_SPLIT_MINSTEPS", 8));
-  static const int64_t maxsplit = std::max<int64_t>(1, env_int("SISI_GEMM_SPLIT_MAX", 64));
-  int ksplit = 1;
-  if (g.K > 4 * kq && tiles * g.batch < want) {
-    const int64_t tb = tiles * g.batch;
-    int64_t s = (want + tb - 1) / tb;
-    const int64_t smax = std::min<int64_t>(std::max<int64_t>(1, g.K / (minsteps * kq)), maxsplit);
-    ksplit = round_filling_split(tb, std::min(s, smax), smax, cus);
+  const int kq = (precision == SISI_BF16X3) ? 32 : kTileK;
+  int bm = BM, bn = BN, ksplit = 1;
+  if (precision == SISI_BF16X3) {
+    // the batched kernel: two rounds of its 128 x 128 tiles, at least eight
+    // k-chunks per part
+    const int64_t tb = ((g.M + bm - 1) / bm) * int64_t((g.N + bn - 1) / bn) * g.batch;
+    if (g.K > 4 * kq && tb < 1024) {
+      const int64_t smax = std::min(std::max(1, g.K / (8 * kq)), 64);
+      ksplit = round_filling_split(tb, std::min((1024 + tb - 1) / tb, smax), smax, cus);
+    }
+  } else {
+    if (taped) {
+      p.tile = kTapeTile;
+    } else {
+      const TilePlan t = choose_tile(g, precision, cus);
+      p.tile = t.tile;
+      ksplit = t.ksplit;
+    }
+    bm = bn = kTiles[p.tile];
   }
+  g.tiles_m = (g.M + bm - 1) / bm;
+  g.tiles_n = (g.N + bn - 1) / bn;
+  SISI_REQUIRE(int64_t(g.tiles_m) * g.tiles_n < (int64_t(1) << 31), SISI_ERR_INVALID,
+               "gemm: too many tiles");
   set_ksplit(g, ksplit, kq);
+  return p;
 }
 
 // Chunking of K for a split of (at most) ksplit partial sums.
@@ -621,12 +453,12 @@ static void set_ksplit(GemmArgs &g, int ksplit, int kq) {
 }
 
 // Launch of a planned product; the split-K partial sums go to g.work.
-static void launch_planned(GemmArgs &g, int precision, bool AKf, bool BNFf, hipStream_t s) {
+static void launch_planned(GemmArgs &g, int precision, const K4Plan &p, hipStream_t s) {
   SISI_REQUIRE(g.batch <= 65535 && g.ksplit <= 65535, SISI_ERR_INVALID, "gemm: grid too large");
   dim3 grid(unsigned(int64_t(g.tiles_m) * g.tiles_n), unsigned(g.ksplit), unsigned(g.batch));
-  if (precision == SISI_FP64) launch_k4<SISI_FP64>(g, grid, s, AKf, BNFf);
-  else if (precision == SISI_FP32) launch_k4<SISI_FP32>(g, grid, s, AKf, BNFf);
-  else launch_b3(g, grid, s, AKf, BNFf);
+  if (precision == SISI_FP64) launch_k4_fp64(p.tile, p.map, g, grid, s);
+  else if (precision == SISI_FP32) launch_k4_fp32(p.tile, p.map, g, grid, s);
+  else launch_b3(g, grid, s, (p.map & 2) != 0, (p.map & 1) != 0);
   SISI_HIP(hipGetLastError());
 }
 
@@ -637,30 +469,11 @@ static void launch_reduce(const GemmArgs &g, hipStream_t s) {
   SISI_HIP(hipGetLastError());
 }
 
-// Sub-kind of a taped product: precision (0 FP64, 1 FP32) * 4 + AK * 2 + BNF.
-static int tape_gemm_sub(int precision, bool AKf, bool BNFf) {
-  return (precision == SISI_FP64 ? 0 : 4) + (AKf ? 2 : 0) + (BNFf ? 1 : 0);
-}
-
+// Sub-kind of a taped product: precision (0 FP64, 1 FP32) * 4 + load mapping.
 void launch_gemm_grouped(int sub, const GemmArgs *const *args, const unsigned *start, int n,
                          unsigned total, hipStream_t s) {
-  switch (sub) {
-#define SISI_GROUPED_CASE(S, P, A, B)                                                            \
-  case S:                                                                                      \
-    hipLaunchKernelGGL((gemm_k4_grouped<P, A, B>), dim3(total), dim3(256), 0, s, args, start, n); \
-    break;
-    SISI_GROUPED_CASE(0, SISI_FP64, false, false)
-    SISI_GROUPED_CASE(1, SISI_FP64, false, true)
-    SISI_GROUPED_CASE(2, SISI_FP64, true, false)
-    SISI_GROUPED_CASE(3, SISI_FP64, true, true)
-    SISI_GROUPED_CASE(4, SISI_FP32, false, false)
-    SISI_GROUPED_CASE(5, SISI_FP32, false, true)
-    SISI_GROUPED_CASE(6, SISI_FP32, true, false)
-    SISI_GROUPED_CASE(7, SISI_FP32, true, true)
-#undef SISI_GROUPED_CASE
-    default: throw Error(SISI_ERR_INVALID, "grouped gemm: unknown sub-kind");
-  }
-  SISI_HIP(hipGetLastError());
+  if (sub < 4) launch_k4_grouped_fp64(sub, args, start, n, total, s);
+  else launch_k4_grouped_fp32(sub - 4, args, start, n, total, s);
 }
 
 void launch_gemm_reduce_grouped(const GemmArgs *const *args, const unsigned *start,
@@ -679,8 +492,7 @@ void launch_gemm_reduce_grouped(const GemmArgs *const *args, const unsigned *sta
 // otherwise run its whole K in one workgroup.
 static void tape_gemm(Engine &eng, int precision, GemmArgs g) {
   if (precision != SISI_FP64) precision = SISI_FP32;
-  bool AKf, BNFf;
-  plan_k4(g, precision, eng.cus, AKf, BNFf);
+  const K4Plan p = plan_k4(g, precision, eng.cus, true);
   const int64_t tb = int64_t(g.tiles_m) * g.tiles_n * g.batch;
   const int64_t MNb = int64_t(g.M) * g.N * g.batch;
   int64_t ks = 1;
@@ -697,7 +509,7 @@ static void tape_gemm(Engine &eng, int precision, GemmArgs g) {
   }
   TapeOp op;
   op.kind = OpKind::Gemm;
-  op.sub = tape_gemm_sub(precision, AKf, BNFf);
+  op.sub = (precision == SISI_FP64 ? 0 : 4) + p.map;
   op.gx = unsigned(g.tiles_m * g.tiles_n);
   op.gy = unsigned(g.ksplit);
   op.gz = unsigned(g.batch);
@@ -729,8 +541,7 @@ void gemm(Engine &eng, int precision, GemmArgs g, bool exact) {
     }
   }
   if (precision == SISI_BF16) precision = SISI_BF16X3;  // batched: the three-product kernel
-  bool AKf, BNFf;
-  plan_k4(g, precision, eng.cus, AKf, BNFf);
+  const K4Plan p = plan_k4(g, precision, eng.cus, false);
   DBuf work;
   if (g.ksplit > 1) {
     work = DBuf(&eng.pool, size_t(g.ksplit) * g.batch * g.M * g.N);
@@ -740,7 +551,7 @@ void gemm(Engine &eng, int precision, GemmArgs g, bool exact) {
                     : precision == SISI_FP32 ? Kind::Gemm32 : Kind::GemmB3;
   {
     Timed t(*eng.timers, kind, gemm_flops(g));
-    launch_planned(g, precision, AKf, BNFf, eng.stream);
+    launch_planned(g, precision, p, eng.stream);
   }
   if (g.ksplit > 1) gemm_reduce(eng, g);
 }
@@ -751,8 +562,7 @@ void gemm_workspace(hipStream_t stream, int cus, int precision, GemmArgs g, doub
                "gemm_workspace: FP64 or FP32 only");
   if (g.M <= 0 || g.N <= 0 || g.batch <= 0) return;
   SISI_REQUIRE(ksplit >= 0, SISI_ERR_INVALID, "gemm_workspace: negative split");
-  bool AKf, BNFf;
-  plan_k4(g, precision, cus, AKf, BNFf);
+  const K4Plan p = plan_k4(g, precision, cus, false);
   const int64_t per = int64_t(g.batch) * g.M * g.N;  // doubles per partial sum
   if (ksplit > 0) {
     set_ksplit(g, ksplit, 16);
@@ -764,7 +574,7 @@ void gemm_workspace(hipStream_t stream, int cus, int precision, GemmArgs g, doub
     set_ksplit(g, int(std::max<int64_t>(1, work_doubles / per)), 16);  // fewer partial sums
   }
   if (g.ksplit > 1) g.work = work;
-  launch_planned(g, precision, AKf, BNFf, stream);
+  launch_planned(g, precision, p, stream);
   if (g.ksplit > 1) launch_reduce(g, stream);
 }
 
