@@ -78,7 +78,8 @@ struct SegGemmArgs {
 
 class Engine;
 
-// Segmented GEMM on the engine's stream, precision SISI_FP64/_FP32/_BF16X3.
+// Segmented GEMM on the engine's stream, precision SISI_FP64/_FP32/_BF16X3
+// (FP64 and FP32: every operand k-fast, sak == sbk == 1).
 void gemm_segments(Engine &eng, int precision, SegGemmArgs a);
 
 // An operand split once into bf16 hi/lo planes for split-BF16x3: `batch`

@@ -3,106 +3,78 @@
 // same registers, so a sum of contractions into one output costs one launch
 // and one epilogue pass instead of one read-modify-write of C per product.
 //
-// Same block tile, wave layout, LDS staging and MFMA forms as the FP64/FP32
-// and on-the-fly BF16x3 kernels of gemm.hip; the operand load mapping
-// (m- or k-fastest A, k- or n-fastest B) is chosen per segment at run time
-// (uniform across the workgroup).  The k loop walks the segments' k-chunks
-// in order, prefetching the next chunk (possibly of the next segment) while
-// the current one is multiplied.
+// FP64 / FP32: the tile core of gemm_tile.hpp.  On-the-fly BF16x3: block
+// tile, LDS staging and MFMA forms of the kernel in gemm.hip, the operand
+// load mapping (m- or k-fast A, k- or n-fast B) chosen per segment at run
+// time.
 #include <cstdlib>
 
 #include "engine.hpp"
 #include "gemm.hpp"
-#include "gemm_device.hpp"
-#include "tune.hpp"
+#include "gemm_tile.hpp"
 
 namespace sisi {
 
 namespace {
 
-__device__ __forceinline__ GemmSeg seg_at(const SegGemmArgs &a, int s) {
-  return s == 0 ? a.seg[0] : s == 1 ? a.seg[1] : s == 2 ? a.seg[2] : a.seg[3];
-}
+// Block tile 64 x 64 of four waves of 32 x 32, every operand k-fast.  The
+// chunk pipeline is the one of gemm_k4.hpp; a chunk of the next segment is
+// fetched while the last one of this segment is multiplied, so the segments
+// run as one k loop.
+//
+// FP64 MFMA bounds it.  The tile: four workgroups share a CU (37 KB of LDS,
+// 94 registers), which hides the chains of a k loop of only ~30 chunks and
+// the read-modify-write of C at its end.  A (T) pass in FP64 with tiles of 64
+// x 64, 80 x 128, 96 x 128, 128 x 128: No = 12, Nv = 240 287, 324, 356, 316
+// ms; No = 14, Nv = 288 869, 1032, 891, 1118; No = 7, Nv = 95 7.1, 9.7, 10.4,
+// 12.4.  The kernel before it (element loads with bounds checks, two barriers
+// per chunk, 80 x 128 and 128 x 128 tiles) took 370, 1387 and 14.5 ms.
+constexpr int kSegTile = 64;
 
-__device__ __forceinline__ int seg_k(const SegGemmArgs &a, int s) {
-  return s == 0 ? a.seg[0].K : s == 1 ? a.seg[1].K : s == 2 ? a.seg[2].K : a.seg[3].K;
-}
-
-// TBM x TBN block tile of WGM x WGN waves (each (TBM/WGM) x (TBN/WGN), a
-// multiple of 16 in both directions: 128 x 128 as 2 x 2 waves of 64 x 64,
-// and 80 x 128 / 128 x 80 as 1 x 4 / 4 x 1 waves of 80 x 32 / 32 x 80 for
-// an output dimension of a multiple of 80 that 128-wide tiles would leave
-// ragged, such as the 400 virtuals of the (T) blocks).
-template <int PREC, int TBM, int TBN, int WGM, int WGN>
+template <int PREC>
 __global__ __launch_bounds__(256, 2) void gemm_seg_k4_kernel(SegGemmArgs a) {
-  using LT = typename std::conditional<PREC == SISI_FP64, double, float>::type;
-  using AT = typename std::conditional<PREC == SISI_FP64, d4, f4>::type;
-  constexpr int BK = 16;
-  constexpr int PAD = (PREC == SISI_FP64) ? 2 : 4;
-  constexpr int LSTR = (PREC == SISI_FP64) ? 1 : 4;
-  constexpr int RSTR = (PREC == SISI_FP64) ? 4 : 1;
+  using LT = typename TileTypes<PREC>::LT;
+  using AT = typename TileTypes<PREC>::AT;
+  constexpr int TBM = kSegTile, TBN = kSegTile, WGM = 2, WGN = 2;
   constexpr int WM = TBM / WGM, WN = TBN / WGN, TI = WM / 16, TJ = WN / 16;
-  constexpr int NA = TBM * BK / 256, NB = TBN * BK / 256;  // loads per thread
-  static_assert(WGM * WGN == 4 && TI * 16 == WM && TJ * 16 == WN, "four waves, 16-multiples");
-  static_assert(NA * 256 == TBM * BK && NB * 256 == TBN * BK, "whole loads per thread");
-  __shared__ LT As[BK][TBM + PAD];
-  __shared__ LT Bs[BK][TBN + PAD];
+  using LA = TileLds<TBM, true>;
+  using LB = TileLds<TBN, true>;
+  __shared__ __attribute__((aligned(16))) LT As[2][LA::kSize];
+  __shared__ __attribute__((aligned(16))) LT Bs[2][LB::kSize];
   const GemmArgs &g = a.g;
+  // the segments are indexed at run time: read from the argument block where
+  // it lies (a copy of it in scratch made every field a per-lane value)
+  using Args = __attribute__((address_space(4))) const SegGemmArgs;
+  Args *ka = (Args *)__builtin_amdgcn_kernarg_segment_ptr();
 
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: scalar branches
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
   int tm, tn;
   tile_coords(g, blockIdx.x, tm, tn);
   const int m0 = tm * TBM, n0 = tn * TBN;
 
-  double ra[NA], rb[NB];
-  int lak = 0, lbnf = 0;
-  // Out-of-range elements load from a clamped (in-range) address, so the
-  // loads need no branch; at the LDS store they are multiplied by zero (the
-  // segment's scale otherwise), one chunk later, so the loads stay in flight
-  // across the MFMAs of the previous chunk.  Element q of a thread is
-  // e = tid + 256 q of the tile, walked along the operand's unit-stride
-  // index (m or n fastest: e % TB, e / TB; k fastest: e / 16, e % 16).
-  const int mlast = g.M - 1, nlast = g.N - 1;
-  int lk0 = 0, lK = 0;
-  double lsc = 1.0;
-
-  auto load = [&](int s, int k0) {
-    const GemmSeg sg = seg_at(a, s);
-    const int klast = sg.K - 1;
-    lak = sg.ak;
-    lbnf = sg.bnf;
-    lk0 = k0;
-    lK = sg.K;
-    lsc = sg.scale;
-#pragma unroll
-    for (int q = 0; q < NA; ++q) {
-      const int e = tid + 256 * q;
-      const int mm = sg.ak ? e / BK : e % TBM, kk = sg.ak ? e % BK : e / TBM;
-      ra[q] = sg.A[int64_t(min(m0 + mm, mlast)) * sg.sam + int64_t(min(k0 + kk, klast)) * sg.sak];
+  TileLoader<LT, TBM, true> la;
+  TileLoader<LT, TBN, true> lb;
+  int chunks = 0;
+  for (int i = 0; i < a.nseg; ++i) chunks += (ka->seg[i].K + kTileK - 1) / kTileK;
+  int s = -1, left = 0;  // segment of the next chunk, and k left in it
+  double scale = 1.0;    // of the chunk in the registers
+  auto fetch = [&]() {
+    if (left <= 0) {
+      ++s;
+      la.init(ka->seg[s].A, ka->seg[s].sam, 1, m0, g.M - 1, 0);
+      lb.init(ka->seg[s].B, ka->seg[s].sbn, 1, n0, g.N - 1, 0);
+      scale = ka->seg[s].scale;
+      left = ka->seg[s].K;
     }
-#pragma unroll
-    for (int q = 0; q < NB; ++q) {
-      const int e = tid + 256 * q;
-      const int nn = sg.bnf ? e % TBN : e / BK, kk = sg.bnf ? e / TBN : e % BK;
-      rb[q] = sg.B[int64_t(min(k0 + kk, klast)) * sg.sbk + int64_t(min(n0 + nn, nlast)) * sg.sbn];
+    if (left >= kTileK) {
+      la.load();
+      lb.load();
+    } else {
+      la.load_tail(left);
+      lb.load_tail(left);
     }
-  };
-
-  auto store = [&]() {
-#pragma unroll
-    for (int q = 0; q < NA; ++q) {
-      const int e = tid + 256 * q;
-      const int mm = lak ? e / BK : e % TBM, kk = lak ? e % BK : e / TBM;
-      As[kk][mm] = LT(ra[q] * ((m0 + mm <= mlast && lk0 + kk < lK) ? lsc : 0.0));
-    }
-#pragma unroll
-    for (int q = 0; q < NB; ++q) {
-      const int e = tid + 256 * q;
-      const int nn = lbnf ? e % TBN : e / BK, kk = lbnf ? e / TBN : e % BK;
-      Bs[kk][nn] = LT(rb[q] * ((n0 + nn <= nlast && lk0 + kk < lK) ? 1.0 : 0.0));
-    }
+    left -= kTileK;
   };
 
   AT acc[TI][TJ];
@@ -112,51 +84,27 @@ __global__ __launch_bounds__(256, 2) void gemm_seg_k4_kernel(SegGemmArgs a) {
     for (int j = 0; j < TJ; ++j) acc[i][j] = AT{0, 0, 0, 0};
 
   const int wm = (wave % WGM) * WM, wn = (wave / WGM) * WN;
-  const int l16 = lane & 15, lk = lane >> 4;
-  // a wave whose sub-tile lies wholly outside the output skips its MFMAs
   const bool active = (m0 + wm < g.M) && (n0 + wn < g.N);
 
-  int s = 0, k0 = 0;
-  bool have = a.nseg > 0;
-  if (have) load(0, 0);
-  while (have) {
-    store();
-    __syncthreads();
-    int s1 = s, k1 = k0 + BK;
-    if (k1 >= seg_k(a, s)) {
-      s1 = s + 1;
-      k1 = 0;
+  // chunk c is multiplied in iteration c >= 0; iteration -1 fills the pipeline
+  fetch();
+  for (int c = -1; c < chunks; ++c) {
+    if (c + 1 < chunks) {
+      if (scale != 1.0) la.scale(scale);
+      la.store(As[(c + 1) & 1]);
+      lb.store(Bs[(c + 1) & 1]);
+      if (c + 2 < chunks) fetch();
     }
-    const bool more = s1 < a.nseg;
-    if (more) load(s1, k1);
-    if (active) {
-#pragma unroll
-      for (int kq = 0; kq < BK / 4; ++kq) {
-        const int k = kq * 4 + lk;
-        LT av[TI], bv[TJ];
-#pragma unroll
-        for (int i = 0; i < TI; ++i) av[i] = As[k][wm + i * 16 + l16];
-#pragma unroll
-        for (int j = 0; j < TJ; ++j) bv[j] = Bs[k][wn + j * 16 + l16];
-#pragma unroll
-        for (int i = 0; i < TI; ++i)
-#pragma unroll
-          for (int j = 0; j < TJ; ++j) {
-            if constexpr (PREC == SISI_FP64)
-              acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bv[j], av[i], acc[i][j], 0, 0, 0);
-            else
-              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[j], av[i], acc[i][j], 0, 0, 0);
-          }
-      }
-    }
+    if (active && c >= 0)
+      tile_mma<PREC, TI, TJ, LA::kRow, LA::kCol, LB::kRow, LB::kCol>(
+          As[c & 1] + wm * LA::kRow, Bs[c & 1] + wn * LB::kRow, lane, acc);
     __syncthreads();
-    s = s1;
-    k0 = k1;
-    have = more;
   }
 
   // row offsets once per row, each column offset once per column (the
   // output splits cost divisions)
+  const int l16 = lane & 15, lk = lane >> 4;
+  constexpr int LSTR = TileTypes<PREC>::kLane, RSTR = TileTypes<PREC>::kReg;
   int64_t om[TI];
 #pragma unroll
   for (int i = 0; i < TI; ++i) {
@@ -179,6 +127,14 @@ __global__ __launch_bounds__(256, 2) void gemm_seg_k4_kernel(SegGemmArgs a) {
         g.C[o] = v;
       }
     }
+}
+
+__device__ __forceinline__ GemmSeg seg_at(const SegGemmArgs &a, int s) {
+  return s == 0 ? a.seg[0] : s == 1 ? a.seg[1] : s == 2 ? a.seg[2] : a.seg[3];
+}
+
+__device__ __forceinline__ int seg_k(const SegGemmArgs &a, int s) {
+  return s == 0 ? a.seg[0].K : s == 1 ? a.seg[1].K : s == 2 ? a.seg[2].K : a.seg[3].K;
 }
 
 __global__ __launch_bounds__(256, 2) void gemm_seg_b3_kernel(SegGemmArgs a) {
@@ -376,114 +332,6 @@ __global__ __launch_bounds__(256, 2) void gemm_seg_b3_kernel(SegGemmArgs a) {
 
 }  // namespace
 
-// Tile variants of the FP64 / FP32 segmented kernel (ids of the tuning
-// cache's family 64 / 32): 128 x 128, 80 x 128, 128 x 80.
-struct SegVariant {
-  int bm, bn;
-  void (*launch)(const SegGemmArgs &, dim3, hipStream_t);
-  const char *name;
-};
-
-template <int PREC, int TBM, int TBN, int WGM, int WGN>
-static void launch_seg(const SegGemmArgs &a, dim3 grid, hipStream_t s) {
-  hipLaunchKernelGGL((gemm_seg_k4_kernel<PREC, TBM, TBN, WGM, WGN>), grid, dim3(256), 0, s, a);
-}
-
-static const SegVariant kSeg64[] = {
-    {128, 128, launch_seg<SISI_FP64, 128, 128, 2, 2>, "seg128x128"},
-    {80, 128, launch_seg<SISI_FP64, 80, 128, 1, 4>, "seg80x128"},
-    {128, 80, launch_seg<SISI_FP64, 128, 80, 4, 1>, "seg128x80"},
-    {80, 192, launch_seg<SISI_FP64, 80, 192, 1, 4>, "seg80x192"},
-    {256, 80, launch_seg<SISI_FP64, 256, 80, 4, 1>, "seg256x80"},
-};
-static const SegVariant kSeg32[] = {
-    {128, 128, launch_seg<SISI_FP32, 128, 128, 2, 2>, "seg128x128"},
-    {80, 128, launch_seg<SISI_FP32, 80, 128, 1, 4>, "seg80x128"},
-    {128, 80, launch_seg<SISI_FP32, 128, 80, 4, 1>, "seg128x80"},
-    {80, 192, launch_seg<SISI_FP32, 80, 192, 1, 4>, "seg80x192"},
-    {256, 80, launch_seg<SISI_FP32, 256, 80, 4, 1>, "seg256x80"},
-};
-constexpr int kNumSeg = 5;
-
-// Size rule when no tuning record exists: an 80-wide tile along a dimension
-// that is a multiple of 80 but not of 128, when that leaves the other at 128.
-static int default_seg_variant(const GemmArgs &g) {
-  const bool m80 = g.M % 80 == 0 && g.M % 128 != 0, n80 = g.N % 80 == 0 && g.N % 128 != 0;
-  if (m80 && !n80) return 1;
-  if (n80 && !m80) return 2;
-  return 0;
-}
-
-static void launch_seg_variant(Engine &eng, SegGemmArgs a, int precision, const SegVariant &v,
-                               int xcd, double flops) {
-  GemmArgs &g = a.g;
-  g.tiles_m = (g.M + v.bm - 1) / v.bm;
-  g.tiles_n = (g.N + v.bn - 1) / v.bn;
-  g.xcd_map = xcd;
-  const int64_t tiles = int64_t(g.tiles_m) * g.tiles_n;
-  SISI_REQUIRE(tiles < (int64_t(1) << 31), SISI_ERR_INVALID, "gemm_segments: too many tiles");
-  const Kind kind = precision == SISI_FP64 ? Kind::Gemm64 : Kind::Gemm32;
-  Timed t(*eng.timers, kind, flops);
-  v.launch(a, dim3(unsigned(tiles), 1u, 1u), eng.stream);
-  SISI_HIP(hipGetLastError());
-}
-
-// Time every tile variant (both tile walks) of one segmented product class
-// into a scratch output; the fastest is recorded for the class.
-static TuneChoice tune_seg(Engine &eng, const SegGemmArgs &a0, int precision, const TuneKey &key,
-                           double flops) {
-  const SegVariant *table = precision == SISI_FP64 ? kSeg64 : kSeg32;
-  SegGemmArgs a = a0;
-  GemmArgs &g = a.g;
-  DBuf scratch(&eng.pool, size_t(g.M) * g.N);
-  g.C = scratch.get();
-  g.cm0 = 1;
-  g.cn0 = g.M;
-  g.cm1 = g.cm2 = g.cm3 = g.cn1 = g.cn2 = g.cn3 = 0;
-  g.dm0 = g.M;
-  g.dn0 = g.N;
-  g.dm1 = g.dn1 = 1;
-  g.split_out = 0;
-  g.out_cube = 0;  // dense M x N scratch, whatever the product writes
-  g.out_planes = 0;
-  g.alpha = 1.0;
-  g.beta = 0.0;
-  const bool stats = eng.timers->enabled;
-  eng.timers->enabled = false;
-  hipEvent_t t0, t1;
-  SISI_HIP(hipEventCreate(&t0));
-  SISI_HIP(hipEventCreate(&t1));
-  TuneChoice best;
-  double best_us = 1e300;
-  for (int v = 0; v < kNumSeg; ++v)
-    for (int xcd = 1; xcd >= 0; --xcd) {
-      launch_seg_variant(eng, a, precision, table[v], xcd, flops);
-      SISI_HIP(hipEventRecord(t0, eng.stream));
-      for (int r = 0; r < 3; ++r) launch_seg_variant(eng, a, precision, table[v], xcd, flops);
-      SISI_HIP(hipEventRecord(t1, eng.stream));
-      SISI_HIP(hipEventSynchronize(t1));
-      float ms = 0.f;
-      SISI_HIP(hipEventElapsedTime(&ms, t0, t1));
-      const double us = 1e3 * double(ms) / 3;
-      if (us < best_us) {
-        best_us = us;
-        best.variant = v;
-        best.xcd = xcd;
-        best.us = us;
-      }
-    }
-  SISI_HIP(hipEventDestroy(t0));
-  SISI_HIP(hipEventDestroy(t1));
-  eng.timers->enabled = stats;
-  tune_record(key, best, table[best.variant].name);
-  return best;
-}
-
-static bool capturing(hipStream_t s) {
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
-}
-
 void gemm_segments(Engine &eng, int precision, SegGemmArgs a) {
   GemmArgs &g = a.g;
   if (g.M <= 0 || g.N <= 0) return;
@@ -492,16 +340,14 @@ void gemm_segments(Engine &eng, int precision, SegGemmArgs a) {
   SISI_REQUIRE(precision == SISI_FP64 || precision == SISI_FP32 || precision == SISI_BF16X3,
                SISI_ERR_INVALID, "gemm_segments: unknown precision");
   double flops = 0.0;
-  int64_t ktot = 0;
   for (int s = 0; s < a.nseg; ++s) {
     GemmSeg &sg = a.seg[s];
     SISI_REQUIRE(sg.K > 0 && sg.A && sg.B, SISI_ERR_INVALID,
                  "gemm_segments: every segment needs K > 0 and operands");
     // the flags only choose which index consecutive threads walk
-    sg.ak = (sg.sak == 1 && sg.sam != 1) ? 1 : 0;
     sg.bnf = (sg.sbn == 1 && sg.sbk != 1) ? 1 : 0;
+    sg.ak = (sg.sak == 1 && sg.sam != 1) ? 1 : 0;
     flops += 2.0 * double(g.M) * double(g.N) * double(sg.K);
-    ktot += sg.K;
   }
   g.batch = 1;
   g.ksplit = 1;
@@ -523,15 +369,21 @@ void gemm_segments(Engine &eng, int precision, SegGemmArgs a) {
     SISI_HIP(hipGetLastError());
     return;
   }
-  const SegVariant *table = precision == SISI_FP64 ? kSeg64 : kSeg32;
-  const TuneKey key = tune_key(precision == SISI_FP64 ? TuneFamily::Seg64 : TuneFamily::Seg32,
-                               g.M, g.N, ktot);
-  TuneChoice c = tune_lookup(key);
-  if (c.variant < 0 && tune_enabled() && !capturing(eng.stream))
-    c = tune_seg(eng, a, precision, key, flops);
-  int vid = c.variant >= 0 && c.variant < kNumSeg ? c.variant : default_seg_variant(g);
-  const int xcd = c.variant >= 0 ? c.xcd : 1;
-  launch_seg_variant(eng, a, precision, table[vid], xcd, flops);
+  for (int i = 0; i < a.nseg; ++i)
+    SISI_REQUIRE(a.seg[i].sak == 1 && a.seg[i].sbk == 1, SISI_ERR_INVALID,
+                 "gemm_segments: FP64 and FP32 segments are k-fast");
+  g.tiles_m = (g.M + kSegTile - 1) / kSegTile;
+  g.tiles_n = (g.N + kSegTile - 1) / kSegTile;
+  g.xcd_map = 1;
+  const int64_t tiles = int64_t(g.tiles_m) * g.tiles_n;
+  SISI_REQUIRE(tiles < (int64_t(1) << 31), SISI_ERR_INVALID, "gemm_segments: too many tiles");
+  Timed t(*eng.timers, precision == SISI_FP64 ? Kind::Gemm64 : Kind::Gemm32, flops);
+  const dim3 grid(unsigned(tiles), 1u, 1u);
+  if (precision == SISI_FP64)
+    hipLaunchKernelGGL(gemm_seg_k4_kernel<SISI_FP64>, grid, dim3(256), 0, eng.stream, a);
+  else
+    hipLaunchKernelGGL(gemm_seg_k4_kernel<SISI_FP32>, grid, dim3(256), 0, eng.stream, a);
+  SISI_HIP(hipGetLastError());
 }
 
 }  // namespace sisi

@@ -319,9 +319,12 @@ __global__ void sum_into_kernel(const double *part, int n, double *out) {
 
 // Operands of one (T) block, all device pointers.
 struct TriplesOps {
-  const double *T2, *T2t;      // T2[a,b,i,j] and T2t[a,b,i,j] = T2[b,a,i,j]
-  const double *Vt, *Vt2;      // Vt[d,b,c,k] = V_bdck, Vt2[d,b,c,k] = Vt[d,c,b,k]
-  const double *VP;            // VP[l,c,j,k] = V_jklc
+  const double *T2t;  // T2[a,d,x,y] as [d,a,x,y]
+  const double *T2h;  // T2[a,b,x,l] as [l,a,b,x]
+  const double *T2th;  // T2[b,a,x,l] as [l,a,b,x]
+  const double *Vt;   // V_bdck as [d,b,c,k]
+  const double *Vt2;  // V_bdck as [d,c,b,k]
+  const double *VP;   // V_jklc as [l,c,j,k]
 };
 
 // Output addressing of the W products for output index j as the GEMM row
@@ -378,9 +381,9 @@ void build_w(Engine &e, int prec, const TriplesOps &opA, const TriplesOps &opB,
       if (pi[0] == j) {
         // + sum_d T2[x_j, d, x, y] V[d, x_pi1, x_pi2, z]
         GemmSeg &sg = a.seg[a.nseg++];
-        sg.A = opA.T2 + (x + o * y) * v * v;
-        sg.sam = 1;
-        sg.sak = v;
+        sg.A = opA.T2t + (x + o * y) * v * v;
+        sg.sam = v;
+        sg.sak = 1;
         sg.B = (pi[1] == p ? opB.Vt : opB.Vt2) + z * v * v * v;
         sg.sbk = 1;
         sg.sbn = v;
@@ -393,9 +396,9 @@ void build_w(Engine &e, int prec, const TriplesOps &opA, const TriplesOps &opB,
         sg.A = opA.VP + (y + o * z) * o * v;
         sg.sam = o;
         sg.sak = 1;
-        sg.B = (pi[0] == p ? opB.T2 : opB.T2t) + x * v * v;
-        sg.sbk = v * v * o;
-        sg.sbn = 1;
+        sg.B = (pi[0] == p ? opB.T2h : opB.T2th) + x * v * v * o;
+        sg.sbk = 1;
+        sg.sbn = o;
         sg.K = int(o);
         sg.scale = -sign;
       }
@@ -586,14 +589,17 @@ double ztriples_energy(Engine &e, const double *T1, const double *T2, int prec,
     zsum(e, 1.0, zdense(e.Vaijk.get(), {v, o, o, o}), "clkj", false, 0.0,
          zdense(e.VP.get(), {o, v, o, o}), "lcjk");
   }
-  DBuf T2t(&e.pool, 2 * n2);
-  zsum(e, 1.0, zdense(const_cast<double *>(T2), {v, v, o, o}), "abij", false, 0.0,
-       zdense(T2t.get(), {v, v, o, o}), "baij");
+  DBuf T2t(&e.pool, 2 * n2), T2h(&e.pool, 2 * n2), T2th(&e.pool, 2 * n2);
+  const ZV T2v = zdense(const_cast<double *>(T2), {v, v, o, o});
+  zsum(e, 1.0, T2v, "abij", false, 0.0, zdense(T2t.get(), {v, v, o, o}), "baij");
+  zsum(e, 1.0, T2v, "abxl", false, 0.0, zdense(T2h.get(), {o, v, v, o}), "labx");
+  zsum(e, 1.0, T2v, "baxl", false, 0.0, zdense(T2th.get(), {o, v, v, o}), "labx");
   std::vector<double> eps_i(o);
   e.download(eps_i.data(), e.eps_i, size_t(o));
-  const TriplesOps re{T2, T2t.get(), e.Vt.get(), e.Vt2.get(), e.VP.get()};
-  const TriplesOps im{T2 + n2, T2t.get() + n2, e.Vt.get() + nvt, e.Vt2.get() + nvt,
-                      e.VP.get() + nvp};
+  const TriplesOps re{T2t.get(),  T2h.get(),   T2th.get(),
+                      e.Vt.get(), e.Vt2.get(), e.VP.get()};
+  const TriplesOps im{T2t.get() + n2,   T2h.get() + n2,     T2th.get() + n2,
+                      e.Vt.get() + nvt, e.Vt2.get() + nvt, e.VP.get() + nvp};
   int norbits = 0;
   DBuf orbits = orbit_codes(e, norbits);
   const int64_t v3 = w_cube_size(v);
@@ -679,7 +685,16 @@ double triples_energy(Engine &e, const double *T1, const double *T2, int prec,
       dense(T2t.get(), {v, v, o, o}), "baij");
   std::vector<double> eps_i(o);
   e.download(eps_i.data(), e.eps_i, size_t(o));
-  const TriplesOps op{T2, T2t.get(), e.Vt.get(), e.Vt2.get(), e.VP.get()};
+  // the block products read every operand along k (build_w)
+  DBuf T2h, T2th;
+  if (prec != SISI_BF16X3) {
+    T2h = DBuf(&e.pool, v * v * o * o);
+    T2th = DBuf(&e.pool, v * v * o * o);
+    const View T2v = dense(const_cast<double *>(T2), {v, v, o, o});
+    sum(e, 1.0, T2v, "abxl", 0.0, dense(T2h.get(), {o, v, v, o}), "labx");
+    sum(e, 1.0, T2v, "baxl", 0.0, dense(T2th.get(), {o, v, v, o}), "labx");
+  }
+  const TriplesOps op{T2t.get(), T2h.get(), T2th.get(), e.Vt.get(), e.Vt2.get(), e.VP.get()};
   TriplesPlanes pl{};
   if (prec == SISI_BF16X3) {
     auto pad = [](int64_t r) { return int(((r + kB3SegTile - 1) / kB3SegTile) * kB3SegTile); };
