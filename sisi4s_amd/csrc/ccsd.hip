@@ -168,24 +168,22 @@ void ccsd_residual(Engine &e, int it, bool initial_doubles, int slice_size, cons
     copy(e, dGai, Gai);
     ctr(e, -1.0, "Gil,al->Gai", Gij, T1, 1.0, dGai, prec);  // cxx:227
     ctr(e, 1.0, "Gad,di->Gai", Gab, T1, 1.0, dGai, prec);   // cxx:230
-    DBuf Xb2(&e.pool, v * o * o * v);
-    View Xakic = V4(Xb2.get(), v, o, o, v);
+    // Rings.  The reference's seven products of 2 Nv^3 No^3 flops (cxx:242-251,
+    // 283-289) are four in this form: with Y2[cbkj] = 2 T[cbkj] - T[bckj],
+    //   Xakic Y2 - Xakci T[cbkj] = (Xakic - Xakci / 2) Y2 - P / 2,
+    //   P[a,b,i,j] = Xakci[akci] T[bckj],  Xakci[bkci] T[ackj] = P[b,a,i,j],
+    // and Xakic - Xakci / 2 needs one product with T2, since its four T2 terms
+    // are (V[dclk] - V[cdlk] / 2)(T[adil] - T[dail] / 2) = U[dclk] Y2[adil] / 4;
+    // the T1 T1 part of cxx:242 contracts one T1 at a time.  No symmetry of T2
+    // or V is used.  No = 28, Nv = 280: 7 -> 4 products of 17.5 ms each.
+    // (The distinguishable variant drops single terms of these: below.)
+    DBuf Xkb(&e.pool, v * o * o * v), Xcb(&e.pool, v * o * v * o), Y2b(&e.pool, n2);
+    View Xakic = V4(Xkb.get(), v, o, o, v), Xakci = V4(Xcb.get(), v, o, v, o),
+         Y2 = V4(Y2b.get(), v, v, o, o);
     ctr(e, 1.0, "Gai,Gck->akic", dGai, Gai, 0.0, Xakic, prec);  // cxx:234
-    DBuf Yb(&e.pool, n2);
-    View Y = V4(Yb.get(), v, v, o, o);
-    add_t1t1(e, Yb.get(), T2p, T1p, 2.0, int(v), int(o));    // cxx:238-240
-    ctr(e, -0.5, "dclk,dail->akic", V, Y, 1.0, Xakic, prec);   // cxx:242
-    ctr(e, 1.0, "dclk,adil->akic", V, T2, 1.0, Xakic, prec);   // cxx:243
-    if (!e.distinguishable)
-      ctr(e, -0.5, "cdlk,adil->akic", V, T2, 1.0, Xakic, prec);  // cxx:244-246
-    e.record("Xakic", Xb2.get(), v * o * o * v);
-    // Y = 2 T[cbkj] - T[bckj] (cxx:248-249)
-    axpby(e, n2, 2.0, T2p, 0.0, Yb.get());
-    sum(e, -1.0, T2, "bckj", 1.0, Y, "cbkj");
-    ctr(e, 1.0, "akic,cbkj->abij", Xakic, Y, 1.0, R2, prec);  // cxx:251
-  }
-  {
-    // Xakci (cxx:254-290)
+    axpby(e, n2, 2.0, T2p, 0.0, Y2b.get());                     // cxx:248-249
+    sum(e, -1.0, T2, "bckj", 1.0, Y2, "cbkj");
+    // Xakci (cxx:254-278)
     DBuf dGabb(&e.pool, G * v * v), dGijb(&e.pool, G * o * o);
     View dGab = V3(dGabb.get(), G, v, v), dGij = V3(dGijb.get(), G, o, o);
     copy(e, dGab, Gab);
@@ -194,16 +192,39 @@ void ccsd_residual(Engine &e, int it, bool initial_doubles, int slice_size, cons
     ctr(e, 1.0, "Gdk,di->Gki", Gai, T1, 1.0, dGij, prec);   // cxx:273
     e.record("dGab4", dGabb.get(), G * v * v);
     e.record("dGij4", dGijb.get(), G * o * o);
-    DBuf Xb3(&e.pool, v * o * v * o);
-    View Xakci = V4(Xb3.get(), v, o, v, o);
     ctr(e, 1.0, "Gac,Gki->akci", dGab, dGij, 0.0, Xakci, prec);  // cxx:277-278
-    if (!e.distinguishable)
+    if (!e.distinguishable) {
+      e.frozen.push_back(Y2b.get());
+      DBuf Qb(&e.pool, v * o * o * o);
+      View Q = V4(Qb.get(), v, o, o, o);
+      ctr(e, 1.0, "dclk,di->clki", V, T1, 0.0, Q, prec);
+      ctr(e, -1.0, "clki,al->akic", Q, T1, 1.0, Xakic, prec);
+      sum(e, -0.5, Xakci, "akci", 1.0, Xakic, "akic");  // before its T2 term
+      ctr(e, 0.25, "dclk,adil->akic", U, Y2, 1.0, Xakic, prec);
+      e.record("Bakic", Xkb.get(), v * o * o * v);
       ctr(e, -0.5, "cdlk,dail->akci", V, T2, 1.0, Xakci, prec);  // cxx:283-285
-    e.frozen.push_back(Xb3.get());
-    e.record("Xakci", Xb3.get(), v * o * v * o);
-    ctr(e, -1.0, "akci,cbkj->abij", Xakci, T2, 1.0, R2, prec);   // cxx:288
-    ctr(e, -1.0, "bkci,ackj->abij", Xakci, T2, 1.0, R2, prec);   // cxx:289
-    e.unfreeze(Xb3.get());  // Xb3 returns to the pool at the end of this block
+      e.record("Xakci", Xcb.get(), v * o * v * o);
+      ctr(e, 1.0, "akic,cbkj->abij", Xakic, Y2, 1.0, R2, prec);
+      e.unfreeze(Y2b.get());
+      DBuf Pb(&e.pool, n2);
+      View P = V4(Pb.get(), v, v, o, o);
+      ctr(e, 1.0, "akci,bckj->abij", Xakci, T2, 0.0, P, prec);
+      axpby(e, n2, -0.5, Pb.get(), 1.0, R2p);
+      sum(e, -1.0, P, "baij", 1.0, R2, "abij");
+    } else {
+      DBuf Yb(&e.pool, n2);
+      View Y = V4(Yb.get(), v, v, o, o);
+      add_t1t1(e, Yb.get(), T2p, T1p, 2.0, int(v), int(o));     // cxx:238-240
+      ctr(e, -0.5, "dclk,dail->akic", V, Y, 1.0, Xakic, prec);  // cxx:242
+      ctr(e, 1.0, "dclk,adil->akic", V, T2, 1.0, Xakic, prec);  // cxx:243
+      e.record("Xakic", Xkb.get(), v * o * o * v);
+      e.record("Xakci", Xcb.get(), v * o * v * o);
+      ctr(e, 1.0, "akic,cbkj->abij", Xakic, Y2, 1.0, R2, prec);  // cxx:251
+      e.frozen.push_back(Xcb.get());
+      ctr(e, -1.0, "akci,cbkj->abij", Xakci, T2, 1.0, R2, prec);  // cxx:288
+      ctr(e, -1.0, "bkci,ackj->abij", Xakci, T2, 1.0, R2, prec);  // cxx:289
+      e.unfreeze(Xcb.get());  // Xcb returns to the pool at the end of this block
+    }
   }
   {
     // R_abij += R_baji (cxx:292)
@@ -592,51 +613,69 @@ void ccsd_residual_delta(Engine &e, int slice_size, const double *T1c, const dou
     ctr(e, -1.0, "bk,aikj->abij", T1A, dP, 1.0, dR2, prec);
   }
   {
-    // Xakic: (dressed Gamma_ai) Gamma_ck + V (Y, T2) terms; then Xakic Y2
+    // Rings in the form of ccsd_residual (Bakic = Xakic - Xakci / 2): changes
+    // of Bakic and Xakci, then B Y2 and P = Xakci T expanded as products
     DBuf ddGb(&e.pool, G * v * o);
     View ddG = V3(ddGb.get(), G, v, o);
     ctr(e, -1.0, "Gil,al->Gai", Gij, d1, 0.0, ddG, prec);
     ctr(e, 1.0, "Gad,di->Gai", Gab, d1, 1.0, ddG, prec);
-    DBuf dXkb(&e.pool, v * o * o * v);
-    View dXakic = V4(dXkb.get(), v, o, o, v);
+    DBuf dXkb(&e.pool, v * o * o * v), dXcb(&e.pool, v * o * v * o);
+    View dXakic = V4(dXkb.get(), v, o, o, v), dXakci = V4(dXcb.get(), v, o, v, o);
     ctr(e, 1.0, "Gai,Gck->akic", ddG, Gai, 0.0, dXakic, prec);
-    DBuf dYb(&e.pool, n2), YAb(&e.pool, n2);
-    add_t1t1(e, dYb.get(), T2p, T1p, 2.0, int(v), int(o));
-    add_t1t1(e, YAb.get(), an.T2.get(), an.T1.get(), 2.0, int(v), int(o));
-    axpby(e, n2, -1.0, YAb.get(), 1.0, dYb.get());
-    YAb.reset();
-    ctr(e, -0.5, "dclk,dail->akic", V, V4(dYb.get(), v, v, o, o), 1.0, dXakic, prec);
-    ctr(e, 1.0, "dclk,adil->akic", V, d2, 1.0, dXakic, prec);
-    if (!e.distinguishable) ctr(e, -0.5, "cdlk,adil->akic", V, d2, 1.0, dXakic, prec);
     // Y2 = 2 T2 - T2^(bc) at T and its change
-    DBuf Y2b(&e.pool, n2);
+    DBuf Y2b(&e.pool, n2), dYb(&e.pool, n2);
     View Y2 = V4(Y2b.get(), v, v, o, o), dY2 = V4(dYb.get(), v, v, o, o);
     axpby(e, n2, 2.0, T2p, 0.0, Y2b.get());
     sum(e, -1.0, T2, "bckj", 1.0, Y2, "cbkj");
     axpby(e, n2, 2.0, d2b.get(), 0.0, dYb.get());
     sum(e, -1.0, d2, "bckj", 1.0, dY2, "cbkj");
-    ctr(e, 1.0, "akic,cbkj->abij", dXakic, Y2, 1.0, dR2, prec);
-    ctr(e, 1.0, "akic,cbkj->abij", V4(A("Xakic"), v, o, o, v), dY2, 1.0, dR2, prec);
-  }
-  {
-    // Xakci = (dressed Gamma_ab)(dressed Gamma_ij) - V T2 / 2; then - Xakci T2 (two terms)
+    // Xakci = (dressed Gamma_ab)(dressed Gamma_ij) - V T2 / 2
     DBuf ddGab(&e.pool, G * v * v), ddGij(&e.pool, G * o * o), Gijn(&e.pool, G * o * o);
     ctr(e, -1.0, "Gcl,al->Gac", Gai, d1, 0.0, V3(ddGab.get(), G, v, v), prec);
     ctr(e, 1.0, "Gdk,di->Gki", Gai, d1, 0.0, V3(ddGij.get(), G, o, o), prec);
     axpby(e, G * o * o, 1.0, A("dGij4"), 0.0, Gijn.get());
     axpby(e, G * o * o, 1.0, ddGij.get(), 1.0, Gijn.get());
-    DBuf dXcb(&e.pool, v * o * v * o);
-    View dXakci = V4(dXcb.get(), v, o, v, o);
     ctr(e, 1.0, "Gac,Gki->akci", V3(ddGab.get(), G, v, v), V3(Gijn.get(), G, o, o), 0.0, dXakci,
         prec);
     ctr(e, 1.0, "Gac,Gki->akci", V3(A("dGab4"), G, v, v), V3(ddGij.get(), G, o, o), 1.0, dXakci,
         prec);
-    if (!e.distinguishable) ctr(e, -0.5, "cdlk,dail->akci", V, d2, 1.0, dXakci, prec);
     View XakciA = V4(A("Xakci"), v, o, v, o);
-    ctr(e, -1.0, "akci,cbkj->abij", dXakci, T2, 1.0, dR2, prec);
-    ctr(e, -1.0, "akci,cbkj->abij", XakciA, d2, 1.0, dR2, prec);
-    ctr(e, -1.0, "bkci,ackj->abij", dXakci, T2, 1.0, dR2, prec);
-    ctr(e, -1.0, "bkci,ackj->abij", XakciA, d2, 1.0, dR2, prec);
+    if (!e.distinguishable) {
+      e.frozen.push_back(dYb.get());
+      // change of V T1 T1: V d1 T1 + V T1_A d1
+      DBuf Qb(&e.pool, v * o * o * o);
+      View Q = V4(Qb.get(), v, o, o, o);
+      ctr(e, 1.0, "dclk,di->clki", V, d1, 0.0, Q, prec);
+      ctr(e, -1.0, "clki,al->akic", Q, T1, 1.0, dXakic, prec);
+      ctr(e, 1.0, "dclk,di->clki", V, T1A, 0.0, Q, prec);
+      ctr(e, -1.0, "clki,al->akic", Q, d1, 1.0, dXakic, prec);
+      sum(e, -0.5, dXakci, "akci", 1.0, dXakic, "akic");
+      ctr(e, 0.25, "dclk,adil->akic", U, dY2, 1.0, dXakic, prec);
+      ctr(e, -0.5, "cdlk,dail->akci", V, d2, 1.0, dXakci, prec);
+      ctr(e, 1.0, "akic,cbkj->abij", dXakic, Y2, 1.0, dR2, prec);
+      ctr(e, 1.0, "akic,cbkj->abij", V4(A("Bakic"), v, o, o, v), dY2, 1.0, dR2, prec);
+      e.unfreeze(dYb.get());
+      DBuf dPb(&e.pool, n2);
+      View dP = V4(dPb.get(), v, v, o, o);
+      ctr(e, 1.0, "akci,bckj->abij", dXakci, T2, 0.0, dP, prec);
+      ctr(e, 1.0, "akci,bckj->abij", XakciA, d2, 1.0, dP, prec);
+      axpby(e, n2, -0.5, dPb.get(), 1.0, dR2b.get());
+      sum(e, -1.0, dP, "baij", 1.0, dR2, "abij");
+    } else {
+      DBuf dYtb(&e.pool, n2), YAb(&e.pool, n2);  // change of T2 + 2 T1 T1
+      add_t1t1(e, dYtb.get(), T2p, T1p, 2.0, int(v), int(o));
+      add_t1t1(e, YAb.get(), an.T2.get(), an.T1.get(), 2.0, int(v), int(o));
+      axpby(e, n2, -1.0, YAb.get(), 1.0, dYtb.get());
+      YAb.reset();
+      ctr(e, -0.5, "dclk,dail->akic", V, V4(dYtb.get(), v, v, o, o), 1.0, dXakic, prec);
+      ctr(e, 1.0, "dclk,adil->akic", V, d2, 1.0, dXakic, prec);
+      ctr(e, 1.0, "akic,cbkj->abij", dXakic, Y2, 1.0, dR2, prec);
+      ctr(e, 1.0, "akic,cbkj->abij", V4(A("Xakic"), v, o, o, v), dY2, 1.0, dR2, prec);
+      ctr(e, -1.0, "akci,cbkj->abij", dXakci, T2, 1.0, dR2, prec);
+      ctr(e, -1.0, "akci,cbkj->abij", XakciA, d2, 1.0, dR2, prec);
+      ctr(e, -1.0, "bkci,ackj->abij", dXakci, T2, 1.0, dR2, prec);
+      ctr(e, -1.0, "bkci,ackj->abij", XakciA, d2, 1.0, dR2, prec);
+    }
   }
   {
     DBuf Rt(&e.pool, n2);
