@@ -7,6 +7,7 @@
 
 #include "contract.hpp"
 #include "gemm.hpp"
+#include "ladder.hpp"
 #include "tensor_ops.hpp"
 
 namespace sisi {
@@ -226,13 +227,28 @@ void ccsd_residual(Engine &e, int it, bool initial_doubles, int slice_size, cons
       e.unfreeze(Xcb.get());  // Xcb returns to the pool at the end of this block
     }
   }
+  // Ladder on the kept pair integrals: its T1-dressed part
+  //   - T_ak (Q[kb] - T_bl Q[kl] / 2) and the mirror of it
+  // goes in before R_abij += R_baji, the rest with V after it
+  const bool kept = e.use_kept_ladder && e.ppl && !e.recording && !e.tape;
+  DBuf Qb, Wb;
+  if (kept) {
+    Qb = DBuf(&e.pool, kept_ladder_q_size(e));
+    Wb = DBuf(&e.pool, o * o * o * o);
+    DBuf Qhb(&e.pool, o * v * o * o);
+    View Qh = V4(Qhb.get(), o, v, o, o), W = V4(Wb.get(), o, o, o, o);
+    kept_ladder_apply(e, Xb.get(), Qb.get(), Qhb.get(), Wb.get(), e.prec_ladder);
+    ctr(e, -0.5, "bl,klij->kbij", T1, W, 1.0, Qh, prec);
+    ctr(e, -1.0, "ak,kbij->abij", T1, Qh, 1.0, R2, prec);
+  }
   {
     // R_abij += R_baji (cxx:292)
     DBuf Rt(&e.pool, n2);
     copy(e, V4(Rt.get(), v, v, o, o), R2);
     sum(e, 1.0, V4(Rt.get(), v, v, o, o), "baji", 1.0, R2, "abij");
   }
-  axpby(e, n2, 1.0, e.Vabij.get(), 1.0, R2p);  // cxx:301
+  if (kept) kept_ladder_add(e, Qb.get(), e.Vabij.get(), R2p);
+  else axpby(e, n2, 1.0, e.Vabij.get(), 1.0, R2p);  // cxx:301
   {
     // Xklij (cxx:303-334)
     DBuf Xb4(&e.pool, o * o * o * o);
@@ -248,6 +264,8 @@ void ccsd_residual(Engine &e, int it, bool initial_doubles, int slice_size, cons
       axpby(e, n2, 1.0, Xb.get(), 0.0, Wb.get());
       axpby(e, n2, -1.0, T2p, 1.0, Wb.get());
       ctr(e, 1.0, "cdkl,cdij->klij", V, V4(Wb.get(), v, v, o, o), 0.0, Xklij, prec);
+    } else if (kept) {
+      copy(e, Xklij, V4(Wb.get(), o, o, o, o));  // Q[kl] is this product
     } else {
       ctr(e, 1.0, "cdkl,cdij->klij", V, X, 0.0, Xklij, prec);   // cxx:317
     }
@@ -255,7 +273,9 @@ void ccsd_residual(Engine &e, int it, bool initial_doubles, int slice_size, cons
     // ppl = 1: the T1 part of this term comes with the ladder (cxx:326-333)
     ctr(e, 1.0, "klij,abkl->abij", Xklij, e.ppl ? T2 : X, 1.0, R2, prec);
   }
-  if (e.ppl && e.NR > 0) {
+  if (kept) {
+    // added above
+  } else if (e.ppl && e.NR > 0) {
     // factor-based ladder (cxx:340-372)
     factor_ladder(e, T1p, Xb.get(), R2p, e.prec_ladder);
   } else if (e.ppl) {
@@ -1128,11 +1148,11 @@ bool graph_residual(Engine &e, int slice, const double *T1, const double *T2, do
   Engine::ResidualGraph &g = e.rgraph;
   const std::vector<int> key = {e.precision,       slice,   e.formulation,  int(e.ppl),
                                 int(e.distinguishable), e.NR, int(e.cplx), int(e.run_initial),
-                                get_b3_backend()};
-  if (g.exec && g.key != key) e.drop_residual_graph();
+                                get_b3_backend(), int(e.use_kept_ladder)};
+  if (g.exec && g.key != key) e.drop_residual_graph(true);
   const int64_t n1 = int64_t(e.n1()), n2 = int64_t(e.n2());
   if (!g.exec) {
-    e.drop_residual_graph();
+    e.drop_residual_graph(true);
     g.T1 = DBuf(&e.pool, size_t(n1));
     g.T2 = DBuf(&e.pool, size_t(n2));
     g.R1 = DBuf(&e.pool, size_t(n1));
@@ -1156,7 +1176,7 @@ bool graph_residual(Engine &e, int slice, const double *T1, const double *T2, do
         if (graph) (void)hipGraphDestroy(graph);
         (void)hipGetLastError();
         e.pool.release(e.pool.end_capture());
-        e.drop_residual_graph();
+        e.drop_residual_graph(true);
         throw;
       }
       err = hipStreamEndCapture(e.stream, &graph);
@@ -1167,7 +1187,7 @@ bool graph_residual(Engine &e, int slice, const double *T1, const double *T2, do
     if (err != hipSuccess) {
       (void)hipGetLastError();
       g.exec = nullptr;
-      e.drop_residual_graph();
+      e.drop_residual_graph(true);
       return false;
     }
     g.key = key;
@@ -1179,6 +1199,46 @@ bool graph_residual(Engine &e, int slice, const double *T1, const double *T2, do
   copy(e, V1(R1, n1), V1(g.R1.get(), n1));
   copy(e, V1(R2, n2), V1(g.R2.get(), n2));
   return true;
+}
+
+// Residual of a plain iteration.  FP64 and FP32 iterations of a symmetric run
+// contract the ladder with the kept pair integrals when at least one more
+// iteration can use them (building them costs about what one sliced ladder
+// does) and they fit; everything else, and a run that finds no memory on the
+// way, takes the sliced ladder.
+void plain_residual(Engine &e, int prec, double *R1, double *R2) {
+  const sisi_ccsd_opts &o = e.opts;
+  const bool mp2 = e.iteration == 0 && !e.run_initial;
+  auto evaluate = [&]() {
+    // graphed residual after the MP2 start (which is a copy) and with launch
+    // timing off
+    if (o.graphs != 0 && !mp2 && !e.timers->enabled &&
+        graph_residual(e, o.slice_size, e.T1.get(), e.T2.get(), R1, R2))
+      return;
+    ccsd_residual(e, e.iteration, e.run_initial, o.slice_size, e.T1.get(), e.T2.get(), R1, R2);
+  };
+  // what the run was begun with may have been changed between its iterations
+  const bool same = e.ppl && e.NR == 0 && e.formulation == SISI_FORMULATION_VERTEX && !e.cplx &&
+                    e.given_integrals == 0;
+  if (!mp2 && e.symmetric_run && same && !e.kept_ladder_failed &&
+      (prec == SISI_FP64 || prec == SISI_FP32) &&
+      (e.ladder.get() || o.max_iterations - e.iteration >= 2)) {
+    if (kept_ladder_build(e)) {
+      e.use_kept_ladder = true;
+      try {
+        evaluate();
+        e.use_kept_ladder = false;
+        return;
+      } catch (const Error &err) {
+        e.use_kept_ladder = false;
+        e.thaw();
+        if (err.code != SISI_ERR_ALLOC) throw;
+      }
+    }
+    e.drop_residual_graph();  // and the pair integrals
+    e.kept_ladder_failed = true;
+  }
+  evaluate();
 }
 
 }  // namespace
@@ -1233,6 +1293,13 @@ void ccsd_begin(Engine &e, const sisi_ccsd_opts &opts, const double *T1h, const 
   e.lin1.reset();
   e.lin2.reset();
   e.anchor = Anchor();
+  e.ladder.reset();
+  e.kept_ladder_failed = false;
+  // every residual of such a run is symmetric (T_abij = T_baji) up to
+  // rounding, whatever the vertex; uploaded classes could break that
+  e.symmetric_run = !e.cplx && e.formulation == SISI_FORMULATION_VERTEX && e.NR == 0 &&
+                    e.ppl && e.given_integrals == 0 && e.Gab.get() &&
+                    (T2h == nullptr || doubles_symmetric(e, e.T2.get()));
   if (opts.mixer == SISI_MIXER_DIIS) {
     const int N = opts.max_residua;
     e.diis.resize(N);
@@ -1289,15 +1356,7 @@ void ccsd_iterate(Engine &e, int n) {
       }
     } else {
       set_precision(e, prec);
-      // graphed residual after the MP2 start (which is a copy) and with
-      // launch timing off
-      const bool graphed = o.graphs != 0 && (e.iteration > 0 || e.run_initial) &&
-                           !e.timers->enabled &&
-                           graph_residual(e, o.slice_size, e.T1.get(), e.T2.get(), R1.get(),
-                                          R2.get());
-      if (!graphed)
-        ccsd_residual(e, e.iteration, e.run_initial, o.slice_size, e.T1.get(), e.T2.get(),
-                      R1.get(), R2.get());
+      plain_residual(e, prec, R1.get(), R2.get());
     }
     DBuf d1(&e.pool, e.n1()), d2(&e.pool, e.n2());
     estimate_amplitudes(e, 2, R1.get(), e.T1.get(), d1.get(), o.level_shift);
@@ -1363,7 +1422,9 @@ void ccsd_iterate(Engine &e, int n) {
     // precision and refinement residuals treat an antisymmetric part of T2
     // differently from the FP64 one, and DIIS lets that part grow when it is
     // not projected out
-    if (o.precision != SISI_FP64 && !e.cplx && e.formulation == SISI_FORMULATION_VERTEX)
+    // (symmetric_run: the kept ladder reads each pair once)
+    if (e.symmetric_run ||
+        (o.precision != SISI_FP64 && !e.cplx && e.formulation == SISI_FORMULATION_VERTEX))
       symmetrize_doubles(e, e.T2.get(), e.Nv, e.No);
     double E, dir, exc, Ei;
     ccsd_energy(e, e.T1.get(), e.T2.get(), E, dir, exc, &Ei);
@@ -1410,6 +1471,8 @@ void ccsd_iterate(Engine &e, int n) {
     e.prev_energy = E;
     e.prev_energy_imag = Ei;
   }
+  // a run that is over gives the pair integrals' memory back to the pool
+  if (e.converged || e.iteration >= o.max_iterations) e.ladder.reset();
 }
 
 void fill_report(const Engine &e, sisi_ccsd_report *r) {

@@ -99,12 +99,14 @@ Engine::Engine(const sisi_dims &d) {
   timers.reset(new Timers(stream));
 }
 
-void Engine::drop_residual_graph() {
+void Engine::drop_residual_graph(bool keep_ladder) {
   if (rgraph.exec) {
     (void)hipStreamSynchronize(stream);
     (void)hipGraphExecDestroy(rgraph.exec);
     rgraph.exec = nullptr;
   }
+  // the pair integrals belong to the vertex and run the graph was made for
+  if (!keep_ladder) ladder.reset();
   pool.release(rgraph.held);
   rgraph.held.clear();
   rgraph.key.clear();
@@ -122,6 +124,7 @@ Engine::~Engine() {
   // device buffers return to the pool before it is released
   T1.reset();
   T2.reset();
+  ladder.reset();
   anchor = Anchor();
   diis.clear();
   lin1.reset();

@@ -247,6 +247,12 @@ class Engine {
   bool confirm_pending = false;
   int confirm_hold = 0;
   DBuf T1, T2;
+  // Plain FP64 / FP32 iterations whose T2 is kept symmetric bit by bit (the
+  // vertex formulation started from symmetric doubles) contract the ladder
+  // with pair integrals kept for the run (ladder.hpp); use_kept_ladder is set
+  // around such a residual
+  bool symmetric_run = false, use_kept_ladder = false, kept_ladder_failed = false;
+  DBuf ladder;
   std::vector<double> energies;
   // DIIS ring (DiisMixer.cxx:48-180)
   std::vector<DiisSlot> diis;
@@ -285,7 +291,7 @@ class Engine {
     std::vector<void *> held;
     std::vector<int> key;
   } rgraph;
-  void drop_residual_graph();
+  void drop_residual_graph(bool keep_ladder = false);
 };
 
 }  // namespace sisi

@@ -3,9 +3,11 @@
 aligned pairs), split K, and values outside the operands that must not reach
 the result."""
 
+import numpy as np
 import pytest
 
 from conftest import announce
+from test_zz_no_alloc import Dev, _hip
 
 pytestmark = pytest.mark.gpu
 
@@ -19,39 +21,40 @@ SHAPES = [(1, 1, 1), (1, 37, 5), (37, 1, 19), (16, 16, 16), (17, 15, 3), (31, 33
 @pytest.mark.parametrize("prec", [0, 1])
 @pytest.mark.parametrize("shape", SHAPES)
 def test_products_at_tile_edges(shape, prec):
-    import torch
     from sisi4s_amd import engine
-    lib = engine.load()
+    lib, hip = engine.load(), _hip()
     M, N, K = shape
     # inputs rounded once to the product precision: FP32 operands are rounded
     # by the kernel, exactly representable here
     u = 2.0 ** -53 if prec == 0 else 2.0 ** -24
-    g = torch.Generator(device="cuda").manual_seed(M * 7 + N * 3 + K)
+    rng = np.random.default_rng(M * 7 + N * 3 + K)
 
     def operand(rows, cols):
-        """Column-major rows x cols inside a leading dimension of rows + 1
-        (odd for even rows), the padding NaN."""
-        full = torch.full((cols, rows + 1), float("nan"), device="cuda", dtype=torch.float64)
-        x = torch.randn(cols, rows, generator=g, device="cuda", dtype=torch.float64)
-        full[:, :rows] = x if prec == 0 else x.float().double()
-        return full, full[:, :rows].T
+        """rows x cols inside a leading dimension of rows + 1 (odd for even
+        rows), the padding NaN."""
+        full = np.full((rows + 1, cols), np.nan)
+        x = rng.standard_normal((rows, cols))
+        full[:rows] = x if prec == 0 else x.astype(np.float32)
+        return Dev(hip, full), full[:rows], rows + 1
     for ta in (0, 1):
         for tb in (0, 1):
-            fa, a = operand(K if ta else M, M if ta else K)
-            fb, b = operand(N if tb else K, K if tb else N)
+            da, a, lda = operand(*((K, M) if ta else (M, K)))
+            db, b, ldb = operand(*((N, K) if tb else (K, N)))
             a, b = (a.T if ta else a), (b.T if tb else b)
-            ref, mag = a @ b, a.abs() @ b.abs()
+            ref, mag = a @ b, np.abs(a) @ np.abs(b)
+            # standard bound of a length-K sum in the product precision, plus
+            # the FP64 epilogue (alpha, beta) and the reference's own
+            bound = (K + 2) * u * mag + (K + 4) * 2.0 ** -53 * (mag + 2.0)
             for ks in (0, 3) if K >= 48 else (0,):
                 announce("gemm tile edges M=%d N=%d K=%d ta=%d tb=%d prec=%d split=%d"
                          % (M, N, K, ta, tb, prec, ks))
-                c = torch.ones(N, M, device="cuda", dtype=torch.float64)
-                rc = lib.sisi_gemm_device_noalloc(
-                    prec, ta, tb, M, N, K, -1.0, fa.data_ptr(), fa.shape[1], fb.data_ptr(),
-                    fb.shape[1], 2.0, c.data_ptr(), M, ks,
-                    torch.cuda.current_stream().cuda_stream)
+                dc = Dev(hip, np.ones((M, N)))
+                rc = lib.sisi_gemm_device_noalloc(prec, ta, tb, M, N, K, -1.0, da.ptr, lda, db.ptr,
+                                                  ldb, 2.0, dc.ptr, M, ks, None)
                 assert rc == 0, lib.sisi_last_error()
-                torch.cuda.synchronize()
-                # standard bound of a length-K sum in the product precision,
-                # plus the FP64 epilogue (alpha, beta) and the reference's own
-                bound = (K + 2) * u * mag + (K + 4) * 2.0 ** -53 * (mag + 2.0)
-                assert bool(((c.T - (2.0 - ref)).abs() <= bound).all())
+                assert hip.hipDeviceSynchronize() == 0
+                c = dc.read().reshape((M, N), order="F")
+                dc.close()
+                assert (np.abs(c - (2.0 - ref)) <= bound).all()
+            da.close()
+            db.close()
