@@ -1129,11 +1129,6 @@ std::vector<double> diis_solve(std::vector<std::vector<double>> A, std::vector<d
 
 namespace {
 
-double fock_dot(Engine &e, const double *x1, const double *x2, const double *y1,
-                const double *y2) {
-  return dot(e, int64_t(e.n1()), x1, y1) + dot(e, int64_t(e.n2()), x2, y2);
-}
-
 // Residual replayed from a hipGraph.  The plain residual issues only kernels
 // and device copies on e.stream (no host synchronisation, no memsets), so
 // one capture per configuration serves every later iteration: T is copied
@@ -1358,6 +1353,8 @@ void ccsd_iterate(Engine &e, int n) {
       set_precision(e, prec);
       plain_residual(e, prec, R1.get(), R2.get());
     }
+    double delta_dd = 0.0;              // |dT|^2 and, in host memory, |T|^2
+    const double *delta_tt = nullptr;
     DBuf d1(&e.pool, e.n1()), d2(&e.pool, e.n2());
     estimate_amplitudes(e, 2, R1.get(), e.T1.get(), d1.get(), o.level_shift);
     estimate_amplitudes(e, 4, R2.get(), e.T2.get(), d2.get(), o.level_shift);
@@ -1369,12 +1366,26 @@ void ccsd_iterate(Engine &e, int n) {
       s.t2 = std::move(R2);
       s.d1 = std::move(d1);
       s.d2 = std::move(d2);
+      // overlaps of the new change with every slot's, read back together
+      SISI_REQUIRE(N <= Engine::kHostScalars - Engine::kDotScalars - 1, SISI_ERR_INVALID,
+                   "maxResidua too large");
+      double *h = e.host_scalars() + Engine::kDotScalars;
+      std::vector<int> filled;
+      std::vector<const double *> vs, vd;
       for (int i = 0; i < N; ++i) {
         if (!e.diis[i].d2.get()) continue;
-        const double ov = 2.0 * fock_dot(e, e.diis[i].d1.get(), e.diis[i].d2.get(), s.d1.get(),
-                                         s.d2.get());
-        e.B[e.diis_next + 1][i + 1] = ov;
-        e.B[i + 1][e.diis_next + 1] = ov;
+        filled.push_back(i);
+        vs.push_back(e.diis[i].d1.get());
+        vd.push_back(e.diis[i].d2.get());
+      }
+      overlaps_async(e, int(filled.size()), vs.data(), vd.data(), s.d1.get(), s.d2.get(), h);
+      e.sync();
+      double dd = 0.0;  // |dT|^2 of this iteration, for the test below
+      for (size_t k = 0; k < filled.size(); ++k) {
+        const int i = filled[k];
+        e.B[e.diis_next + 1][i + 1] = 2.0 * h[k];
+        e.B[i + 1][e.diis_next + 1] = 2.0 * h[k];
+        if (i == e.diis_next) dd = h[k];
       }
       if (e.diis_count < N) ++e.diis_count;
       const int dim = e.diis_count + 1;
@@ -1385,21 +1396,21 @@ void ccsd_iterate(Engine &e, int n) {
       rhs[0] = -1.0;
       std::vector<double> col = diis_solve(Bm, rhs);
       DBuf n1(&e.pool, e.n1()), n2(&e.pool, e.n2());
-      zero(e, n1.get(), int64_t(e.n1()));
-      zero(e, n2.get(), int64_t(e.n2()));
+      std::vector<double> w;
+      vs.clear();
+      vd.clear();
       for (int j = 0; j < e.diis_count; ++j) {
         const int i = (e.diis_next + N - j) % N;
-        axpby(e, int64_t(e.n1()), col[i + 1], e.diis[i].t1.get(), 1.0, n1.get());
-        axpby(e, int64_t(e.n2()), col[i + 1], e.diis[i].t2.get(), 1.0, n2.get());
+        w.push_back(col[i + 1]);
+        vs.push_back(e.diis[i].t1.get());
+        vd.push_back(e.diis[i].t2.get());
       }
+      combine_async(e, int(w.size()), w.data(), vs.data(), vd.data(), n1.get(), n2.get(), h + N);
       e.diis_next = (e.diis_next + 1) % N;
       e.T1 = std::move(n1);
       e.T2 = std::move(n2);
-      // amplitude change of this iteration, read back for the test below
-      const DiisSlot &cur = e.diis[(e.diis_next + N - 1) % N];
-      const double dd = fock_dot(e, cur.d1.get(), cur.d2.get(), cur.d1.get(), cur.d2.get());
-      const double tt = fock_dot(e, e.T1.get(), e.T2.get(), e.T1.get(), e.T2.get());
-      e.last_delta = std::sqrt(std::fabs(dd / tt));
+      delta_dd = dd;
+      delta_tt = h + N;  // read with the energy
     } else {
       // LinearMixer::append (LinearMixer.cxx:30-44)
       if (e.lin_have) {
@@ -1414,9 +1425,13 @@ void ccsd_iterate(Engine &e, int n) {
       copy(e, V1(n2.get(), int64_t(e.n2())), V1(e.lin2.get(), int64_t(e.n2())));
       e.T1 = std::move(n1);
       e.T2 = std::move(n2);
-      const double dd = fock_dot(e, d1.get(), d2.get(), d1.get(), d2.get());
-      const double tt = fock_dot(e, e.T1.get(), e.T2.get(), e.T1.get(), e.T2.get());
-      e.last_delta = std::sqrt(std::fabs(dd / tt));
+      double *h = e.host_scalars() + Engine::kDotScalars;
+      const double *x1 = d1.get(), *x2 = d2.get(), *y1 = e.T1.get(), *y2 = e.T2.get();
+      overlaps_async(e, 1, &x1, &x2, x1, x2, h);
+      overlaps_async(e, 1, &y1, &y2, y1, y2, h + 1);
+      e.sync();
+      delta_dd = h[0];
+      delta_tt = h + 1;
     }
     // mixed runs keep T2 exactly symmetric (T_abij = T_baji): the reduced-
     // precision and refinement residuals treat an antisymmetric part of T2
@@ -1427,7 +1442,8 @@ void ccsd_iterate(Engine &e, int n) {
         (o.precision != SISI_FP64 && !e.cplx && e.formulation == SISI_FORMULATION_VERTEX))
       symmetrize_doubles(e, e.T2.get(), e.Nv, e.No);
     double E, dir, exc, Ei;
-    ccsd_energy(e, e.T1.get(), e.T2.get(), E, dir, exc, &Ei);
+    ccsd_energy(e, e.T1.get(), e.T2.get(), E, dir, exc, &Ei);  // waits for the stream
+    e.last_delta = std::sqrt(std::fabs(delta_dd / *delta_tt));
     SISI_REQUIRE(std::isfinite(E) && std::isfinite(e.last_delta), SISI_ERR_NUMERIC,
                  "CCSD iteration " + std::to_string(e.iteration + 1) +
                      " diverged (non-finite energy or amplitudes)");

@@ -121,6 +121,7 @@ Engine::~Engine() {
   (void)hipStreamSynchronize(stream);
   drop_residual_graph();
   timers.reset();
+  if (scalars_) (void)hipHostFree(scalars_);
   // device buffers return to the pool before it is released
   T1.reset();
   T2.reset();
@@ -190,6 +191,15 @@ void Engine::download_t(double *dst, const DBuf &src, size_t n) {
     dst[2 * k] = planar[k];
     dst[2 * k + 1] = planar[h + k];
   }
+}
+
+double *Engine::host_scalars() {
+  if (!scalars_) {
+    std::lock_guard<std::recursive_mutex> lock(device_wide_mutex());
+    SISI_HIP(hipHostMalloc(reinterpret_cast<void **>(&scalars_), kHostScalars * sizeof(double),
+                           hipHostMallocDefault));
+  }
+  return scalars_;
 }
 
 void Engine::sync() { SISI_HIP(hipStreamSynchronize(stream)); }

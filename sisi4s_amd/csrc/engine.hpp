@@ -271,6 +271,12 @@ class Engine {
   void upload_t(DBuf &dst, const double *src, size_t n);
   void download_t(double *dst, const DBuf &src, size_t n);
   void sync();
+  // Pinned host memory that reduction kernels write their results to
+  // directly (no copy; read them after sync()).  The first kDotScalars are
+  // the single reductions', the rest the mixer's.
+  static constexpr int kHostScalars = 4096, kDotScalars = 8;
+  double *host_scalars();
+  double *scalars_ = nullptr;
   // doubles per singles / doubles amplitude tensor (both planes in complex
   // mode) and elements per plane
   size_t n1() const { return n1e() * (cplx ? 2 : 1); }

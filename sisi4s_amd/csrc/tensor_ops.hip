@@ -388,21 +388,146 @@ __global__ void sum_partials_kernel(const double *part, int n, int stride, doubl
 
 double dot(Engine &e, int64_t n, const double *x, const double *y) {
   if (n <= 0) return 0.0;
-  DBuf part(&e.pool, kRedBlocks + 1);
+  DBuf part(&e.pool, kRedBlocks);
+  double *h = e.host_scalars();
   {
     Timed t(*e.timers, Kind::Bandwidth, 16.0 * double(n));
     hipLaunchKernelGGL(dot_partial_kernel, dim3(kRedBlocks), dim3(256), 0, e.stream, n, x, y,
                        part.get());
     hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(256), 0, e.stream, part.get(),
-                       kRedBlocks, 1, part.get() + kRedBlocks);
+                       kRedBlocks, 1, h);
     SISI_HIP(hipGetLastError());
   }
-  double r = 0.0;
-  SISI_HIP(hipMemcpyAsync(&r, part.get() + kRedBlocks, sizeof(double), hipMemcpyDeviceToHost,
-                          e.stream));
   SISI_HIP(hipStreamSynchronize(e.stream));
-  return r;
+  return h[0];
 }
+
+// The mixer's reductions and combination over whole amplitude vectors
+// (singles, then doubles: element i of a vector is one of n1 + n2).  HBM
+// bound: the overlaps of a new vector with NV others read it once (NV + 1
+// streams instead of 2 NV), and a combination reads each vector once and
+// writes the result once, its norm on the way (NV + 1 streams instead of
+// 3 NV + 1, and 2 more for the norm).
+constexpr int kVecs = 8;  // vectors per launch
+
+struct VecArgs {
+  const double *s[kVecs], *d[kVecs];  // singles and doubles of each vector
+  double c[kVecs];
+  int64_t n1, n2;
+};
+
+template <int NV>
+__global__ __launch_bounds__(256) void overlaps_kernel(VecArgs g, const double *ys,
+                                                       const double *yd, double *part) {
+  double acc[NV];
+#pragma unroll
+  for (int k = 0; k < NV; ++k) acc[k] = 0.0;
+  const int64_t step = int64_t(gridDim.x) * blockDim.x;
+  const int64_t t0 = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  for (int64_t i = t0; i < g.n1; i += step) {
+    const double y = ys[i];
+#pragma unroll
+    for (int k = 0; k < NV; ++k) acc[k] += g.s[k][i] * y;
+  }
+  for (int64_t i = t0; i < g.n2; i += step) {
+    const double y = yd[i];
+#pragma unroll
+    for (int k = 0; k < NV; ++k) acc[k] += g.d[k][i] * y;
+  }
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    const double r = block_sum(acc[k]);
+    if (threadIdx.x == 0) part[int64_t(blockIdx.x) * NV + k] = r;
+  }
+}
+
+// out (+)= sum_k c_k vector_k, in the order given; part: sums of out^2
+template <int NV>
+__global__ __launch_bounds__(256) void combine_kernel(VecArgs g, double *os, double *od, int more,
+                                                      double *part) {
+  double q = 0.0;
+  const int64_t step = int64_t(gridDim.x) * blockDim.x;
+  const int64_t t0 = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  for (int64_t i = t0; i < g.n1; i += step) {
+    double v = more ? os[i] : 0.0;
+#pragma unroll
+    for (int k = 0; k < NV; ++k) v += g.c[k] * g.s[k][i];
+    os[i] = v;
+    q += v * v;
+  }
+  for (int64_t i = t0; i < g.n2; i += step) {
+    double v = more ? od[i] : 0.0;
+#pragma unroll
+    for (int k = 0; k < NV; ++k) v += g.c[k] * g.d[k][i];
+    od[i] = v;
+    q += v * v;
+  }
+  q = block_sum(q);
+  if (threadIdx.x == 0) part[blockIdx.x] = q;
+}
+
+#define SISI_VECS(NV_, CALL)                          \
+  switch (NV_) {                                      \
+    case 1: CALL(1); break;                           \
+    case 2: CALL(2); break;                           \
+    case 3: CALL(3); break;                           \
+    case 4: CALL(4); break;                           \
+    case 5: CALL(5); break;                           \
+    case 6: CALL(6); break;                           \
+    case 7: CALL(7); break;                           \
+    default: CALL(8); break;                          \
+  }
+
+void overlaps_async(Engine &e, int nv, const double *const *s, const double *const *d,
+                    const double *ys, const double *yd, double *host) {
+  for (int k0 = 0; k0 < nv; k0 += kVecs) {
+    const int m = std::min(kVecs, nv - k0);
+    VecArgs g{};
+    for (int k = 0; k < m; ++k) {
+      g.s[k] = s[k0 + k];
+      g.d[k] = d[k0 + k];
+    }
+    g.n1 = int64_t(e.n1());
+    g.n2 = int64_t(e.n2());
+    DBuf part(&e.pool, size_t(kRedBlocks) * m);
+    Timed t(*e.timers, Kind::Bandwidth, 8.0 * double(m + 1) * double(g.n1 + g.n2));
+#define SISI_CALL(NV)                                                                          \
+  hipLaunchKernelGGL(overlaps_kernel<NV>, dim3(kRedBlocks), dim3(256), 0, e.stream, g, ys, yd, \
+                     part.get())
+    SISI_VECS(m, SISI_CALL)
+#undef SISI_CALL
+    hipLaunchKernelGGL(sum_partials_kernel, dim3(m), dim3(256), 0, e.stream, part.get(),
+                       kRedBlocks, m, host + k0);
+    SISI_HIP(hipGetLastError());
+  }
+}
+
+void combine_async(Engine &e, int nv, const double *c, const double *const *s,
+                   const double *const *d, double *os, double *od, double *host) {
+  for (int k0 = 0; k0 < nv; k0 += kVecs) {
+    const int m = std::min(kVecs, nv - k0);
+    VecArgs g{};
+    for (int k = 0; k < m; ++k) {
+      g.s[k] = s[k0 + k];
+      g.d[k] = d[k0 + k];
+      g.c[k] = c[k0 + k];
+    }
+    g.n1 = int64_t(e.n1());
+    g.n2 = int64_t(e.n2());
+    DBuf part(&e.pool, kRedBlocks);
+    Timed t(*e.timers, Kind::Bandwidth, 8.0 * double(m + 1 + (k0 > 0)) * double(g.n1 + g.n2));
+#define SISI_CALL(NV)                                                                            \
+  hipLaunchKernelGGL(combine_kernel<NV>, dim3(kRedBlocks), dim3(256), 0, e.stream, g, os, od,    \
+                     int(k0 > 0), part.get())
+    SISI_VECS(m, SISI_CALL)
+#undef SISI_CALL
+    if (k0 + m >= nv)
+      hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(256), 0, e.stream, part.get(),
+                         kRedBlocks, 1, host);
+    SISI_HIP(hipGetLastError());
+  }
+}
+#undef SISI_VECS
 
 __device__ __forceinline__ void estimate_body(const ElemArgs &p, unsigned bx, unsigned gx) {
   const int order = p.i0, Nv = p.i1, No = p.i2;
@@ -569,18 +694,16 @@ __global__ void energy_partial_kernel(int Nv, int No, const double *T1, const do
 
 void energy_terms(Engine &e, const double *T1, const double *T2, double &direct,
                   double &exchange) {
-  DBuf part(&e.pool, 2 * kRedBlocks + 2);
+  DBuf part(&e.pool, 2 * kRedBlocks);
+  double *r = e.host_scalars();
   {
     Timed t(*e.timers, Kind::Bandwidth, 24.0 * double(e.n2()));
     hipLaunchKernelGGL(energy_partial_kernel, dim3(kRedBlocks), dim3(256), 0, e.stream, e.Nv,
                        e.No, T1, T2, e.Vabij.get(), e.Vbaij.get(), part.get());
     hipLaunchKernelGGL(sum_partials_kernel, dim3(2), dim3(256), 0, e.stream, part.get(),
-                       kRedBlocks, 2, part.get() + 2 * kRedBlocks);
+                       kRedBlocks, 2, r);
     SISI_HIP(hipGetLastError());
   }
-  double r[2];
-  SISI_HIP(hipMemcpyAsync(r, part.get() + 2 * kRedBlocks, 2 * sizeof(double),
-                          hipMemcpyDeviceToHost, e.stream));
   SISI_HIP(hipStreamSynchronize(e.stream));
   direct = 2.0 * r[0];
   exchange = -1.0 * r[1];

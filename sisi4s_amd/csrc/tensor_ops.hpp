@@ -39,6 +39,14 @@ void scale_pairs(Engine &e, double *C, int64_t Rx, int64_t Ry, int64_t nij, cons
 // Deterministic FP64 sum_k x[k]*y[k] (returned to the host).
 double dot(Engine &e, int64_t n, const double *x, const double *y);
 
+// Overlaps of nv amplitude vectors (singles s[k], doubles d[k]) with (ys, yd)
+// into host[k], and out = sum_k c_k vector_k with |out|^2 into *host.  host is
+// memory of e.host_scalars(), valid after e.sync().
+void overlaps_async(Engine &e, int nv, const double *const *s, const double *const *d,
+                    const double *ys, const double *yd, double *host);
+void combine_async(Engine &e, int nv, const double *c, const double *const *s,
+                   const double *const *d, double *os, double *od, double *host);
+
 // Amplitude estimate of ClusterSinglesDoublesAlgorithm.cxx:302-331 on one
 // component (order 2 for T1, 4 for T2; both planes in complex mode, the
 // denominators being real), fused with the amplitude change:

@@ -64,6 +64,12 @@ def test_split_over_calls_and_linear_mixer():
     check(*run((3, 20, 40), mixer="LinearMixer", mixing_ratio=0.7), TOL)
 
 
+def test_more_vectors_than_one_reduction_launch():
+    """Ten DIIS vectors: the overlaps and the combination take two launches of
+    at most eight."""
+    check(*run((3, 20, 40), max_residua=10, max_iterations=11), 1e-10)
+
+
 def test_distinguishable_and_no_ladder():
     check(*run((3, 20, 40), distinguishable=True), TOL)
     check(*run((3, 20, 40), ppl=False), TOL)
