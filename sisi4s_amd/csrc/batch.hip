@@ -32,6 +32,7 @@
 #include "ccsd.hpp"
 #include "engine.hpp"
 #include "tape.hpp"
+#include "ladder.hpp"
 #include "tensor_ops.hpp"
 
 namespace sisi {
@@ -374,6 +375,15 @@ void ccsd_solve_lockstep(int nsys, const sisi_dims *dims, const double *const *g
   std::vector<System> sys(static_cast<size_t>(nsys));
   const int N = o.mixer == SISI_MIXER_DIIS ? o.max_residua : 0;
   const bool bulk_run = o.precision != SISI_FP64;
+  // kept pair integrals (ladder.hpp) for every system or for none: when all of
+  // them together leave most of the memory to the recorded residuals
+  bool keep_ladders = o.ppl != 0 && o.max_iterations >= 3;
+  if (keep_ladders) {
+    size_t free_b = 0, total_b = 0;
+    double need = 0.0;
+    for (int k = 0; k < nsys; ++k) need += kept_ladder_bytes(dims[k].No, dims[k].Nv);
+    keep_ladders = hipMemGetInfo(&free_b, &total_b) == hipSuccess && need <= 0.3 * double(free_b);
+  }
   // set-up: integrals per system (eager, on the system's own stream), fixed
   // buffers, recorded residuals
   for (int k = 0; k < nsys; ++k) {
@@ -404,6 +414,8 @@ void ccsd_solve_lockstep(int nsys, const sisi_dims *dims, const double *const *g
     }
     s.cur_precision = o.precision;
     s.coarse_active = bulk_run && o.coarse_threshold > 0.0;
+    // the run starts from T = 0 and its updates keep T2 symmetric (below)
+    if (keep_ladders) e.use_kept_ladder = kept_ladder_build(e);
     if (bulk_run) record_residual(s, 1, o.slice_size, 1, s.res[1], &s.held[1], pool, stream);
     record_residual(s, 0, o.slice_size, 1, s.res[0], &s.held[0], pool, stream);
   }
@@ -535,6 +547,7 @@ void ccsd_solve_lockstep(int nsys, const sisi_dims *dims, const double *const *g
         s.lin_have = true;
         copy(e, dense(s.T1.get(), {n1}), dense(s.R1.get(), {n1}));
         copy(e, dense(s.T2.get(), {n2}), dense(s.R2.get(), {n2}));
+        if (e.use_kept_ladder) symmetrize_doubles(e, s.T2.get(), e.Nv, e.No);
         dot_into(e, n1, s.d1.get(), s.d1.get(), s.part.get(), out + 0);
         dot_into(e, n2, s.d2.get(), s.d2.get(), s.part.get(), out + 1);
         dot_into(e, n1, s.T1.get(), s.T1.get(), s.part.get(), out + 2);
@@ -595,6 +608,7 @@ void ccsd_solve_lockstep(int nsys, const sisi_dims *dims, const double *const *g
           axpby(e, n1, col[size_t(i + 1)], s.slots[size_t(i)].t1.get(), 1.0, s.T1.get());
           axpby(e, n2, col[size_t(i + 1)], s.slots[size_t(i)].t2.get(), 1.0, s.T2.get());
         }
+        if (e.use_kept_ladder) symmetrize_doubles(e, s.T2.get(), e.Nv, e.No);
         s.next = (s.next + 1) % N;
         double *out = out_of(k);
         dot_into(e, n1, s.T1.get(), s.T1.get(), s.part.get(), out + 2 * N);
@@ -689,12 +703,13 @@ void ccsd_solve_lockstep(int nsys, const sisi_dims *dims, const double *const *g
   if (!prof.empty()) {
     static const char *kinds[] = {"gemm", "copy_tiled", "copy_generic", "fill", "axpby",
                                   "add_t1t1", "estimate", "dot_partial", "sum_partials",
-                                  "energy_partial", "gemm_reduce"};
+                                  "energy_partial", "gemm_reduce", "pack_pairs",
+                                  "unpack_holes", "add_pairs", "symmetrize"};
     fprintf(stderr, "[lockstep profile] kind/variant: ms, launches, records, blocks\n");
     for (size_t k = 0; k < prof.size(); ++k)
       if (prof[k].launches > 0)
         fprintf(stderr, "[lockstep profile] %s/%d: %.1f ms, %.0f, %.0f, %.0f\n",
-                k / 16 < 11 ? kinds[k / 16] : "?", int(k % 16), prof[k].ms, prof[k].launches,
+                k / 16 < 15 ? kinds[k / 16] : "?", int(k % 16), prof[k].ms, prof[k].launches,
                 prof[k].records, prof[k].blocks);
     std::vector<std::pair<double, std::string>> top;
     for (auto &kv : prof_shapes) top.push_back({kv.second.ms, kv.first});

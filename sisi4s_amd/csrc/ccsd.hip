@@ -230,7 +230,7 @@ void ccsd_residual(Engine &e, int it, bool initial_doubles, int slice_size, cons
   // Ladder on the kept pair integrals: its T1-dressed part
   //   - T_ak (Q[kb] - T_bl Q[kl] / 2) and the mirror of it
   // goes in before R_abij += R_baji, the rest with V after it
-  const bool kept = e.use_kept_ladder && e.ppl && !e.recording && !e.tape;
+  const bool kept = e.use_kept_ladder && e.ppl && !e.recording;
   DBuf Qb, Wb;
   if (kept) {
     Qb = DBuf(&e.pool, kept_ladder_q_size(e));

@@ -4,6 +4,7 @@
 #include <algorithm>
 
 #include "contract.hpp"
+#include "tape.hpp"
 #include "tensor_ops.hpp"
 
 namespace sisi {
@@ -39,11 +40,10 @@ struct PackArgs {
 // combinations with the transposed matrix.  HBM bound: each matrix is read
 // once, tile by tile, with its mirror tile staged in LDS (both reads run along
 // c), and the packed rows are written along c.
-__global__ __launch_bounds__(256) void pack_pairs_kernel(PackArgs g) {
+__device__ __forceinline__ void pack_pairs_body(const PackArgs &g, int ct, int dt, int z) {
   const int v = g.v;
-  const int ct = int(blockIdx.x), dt = int(blockIdx.y);
   if (ct > dt) return;
-  const int p = int(blockIdx.z) % g.np, q = int(blockIdx.z) / g.np;
+  const int p = z % g.np, q = z / g.np;
   const Rows rows{v, g.o};
   int64_t row;
   if (g.mode == kParticleRows) {
@@ -55,7 +55,7 @@ __global__ __launch_bounds__(256) void pack_pairs_kernel(PackArgs g) {
     if (p > q) return;
     row = int64_t(q) * (q + 1) / 2 + p + (g.mode == kHoleRows ? rows.hh() : 0);
   }
-  const double *m = g.src + int64_t(blockIdx.z) * v * v;
+  const double *m = g.src + int64_t(z) * v * v;
   __shared__ double s0[32][33], s1[32][33];  // [d][c] of the tile, and of its mirror
   const int x = int(threadIdx.x) & 31, y0 = int(threadIdx.x) >> 5;
 #pragma unroll
@@ -79,6 +79,26 @@ __global__ __launch_bounds__(256) void pack_pairs_kernel(PackArgs g) {
   }
 }
 
+__global__ __launch_bounds__(256) void pack_pairs_kernel(PackArgs g) {
+  pack_pairs_body(g, int(blockIdx.x), int(blockIdx.y), int(blockIdx.z));
+}
+
+// The amplitudes' pack: matrices X[:, :, i, j] into rows i <= j.
+__host__ __device__ inline PackArgs amplitude_pack(const double *X, double *out, int64_t plane,
+                                                   int v, int o) {
+  PackArgs a{};
+  a.src = X;
+  a.out = out;
+  a.plane = plane;
+  a.v = v;
+  a.o = o;
+  a.mode = kAmplitudes;
+  a.np = o;
+  a.scale = 0.5;
+  a.diag = 1.0;
+  return a;
+}
+
 void pack_pairs(Engine &e, const PackArgs &g, int64_t matrices) {
   const unsigned t = unsigned((g.v + 31) / 32);
   PackArgs a = g;
@@ -97,14 +117,15 @@ void pack_pairs(Engine &e, const PackArgs &g, int64_t matrices) {
 }
 
 // Hole-particle rows to Qh[k,b,i,j] and hole rows to W[k,l,i,j].
-__global__ __launch_bounds__(256) void unpack_holes_kernel(const double *Qp, int64_t plane, int v,
-                                                           int o, double *Qh, double *W) {
+__device__ __forceinline__ void unpack_holes_body(const double *Qp, int64_t plane, int v, int o,
+                                                  double *Qh, double *W, unsigned bx,
+                                                  unsigned gx) {
   const Rows rows{v, o};
   const int64_t M = rows.count(), nij = rows.opairs();
   const int64_t hp = int64_t(o) * v, per = hp + rows.opairs();
   const int64_t total = per * nij;
-  for (int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; t < total;
-       t += int64_t(gridDim.x) * blockDim.x) {
+  for (int64_t t = int64_t(bx) * blockDim.x + threadIdx.x; t < total;
+       t += int64_t(gx) * blockDim.x) {
     const int64_t r = t % per, n = t / per;
     int j = int((sqrt(8.0 * double(n) + 1.0) - 1.0) * 0.5);
     while (int64_t(j + 1) * (j + 2) / 2 <= n) ++j;
@@ -129,19 +150,24 @@ __global__ __launch_bounds__(256) void unpack_holes_kernel(const double *Qp, int
   }
 }
 
+__global__ __launch_bounds__(256) void unpack_holes_kernel(const double *Qp, int64_t plane, int v,
+                                                           int o, double *Qh, double *W) {
+  unpack_holes_body(Qp, plane, v, o, Qh, W, blockIdx.x, gridDim.x);
+}
+
 // R2 += V + particle rows: a tile of pairs (a in ta, b in tb, ta <= tb) of one
 // i <= j is read along a, and its values go to the four places (ab,ij),
 // (ba,ji), (ab,ji), (ba,ij); the two mirrored ones through LDS, so that every
 // write runs along the first index.  HBM bound: R2 and V once, Q once.
-__global__ __launch_bounds__(256) void add_pairs_kernel(const double *Qp, int64_t plane,
-                                                        const double *V, double *R, int v, int o) {
-  const int ta = int(blockIdx.x), tb = int(blockIdx.y);
+__device__ __forceinline__ void add_pairs_body(const double *Qp, int64_t plane, const double *V,
+                                               double *R, int v, int o, int ta, int tb, int ij0,
+                                               int nij) {
   if (ta > tb) return;
   const Rows rows{v, o};
   const int64_t M = rows.count(), nv2 = int64_t(v) * v;
   __shared__ double s0[32][33], s1[32][33];
   const int x = int(threadIdx.x) & 31, y0 = int(threadIdx.x) >> 5;
-  for (int ij = int(blockIdx.z); ij < o * o; ij += int(gridDim.z)) {
+  for (int ij = ij0; ij < o * o; ij += nij) {
     const int i = ij % o, j = ij / o;
     if (i > j) continue;
     const int64_t n = int64_t(j) * (j + 1) / 2 + i;
@@ -180,6 +206,52 @@ __global__ __launch_bounds__(256) void add_pairs_kernel(const double *Qp, int64_
   }
 }
 
+__global__ __launch_bounds__(256) void add_pairs_kernel(const double *Qp, int64_t plane,
+                                                        const double *V, double *R, int v, int o) {
+  add_pairs_body(Qp, plane, V, R, v, o, int(blockIdx.x), int(blockIdx.y), int(blockIdx.z),
+                 int(gridDim.z));
+}
+
+// Grouped forms (batched solver), arguments in ElemArgs: i0 = v, i1 = o,
+// n = plane; Pack x0 -> y; Unpack x0 -> y, and W at x1; Add x0, V = x1 -> y.
+template <int KIND>
+__global__ __launch_bounds__(256) void pairs_grouped(const ElemArgs *const *args,
+                                                     const unsigned *__restrict__ start, int n) {
+  int lo = 0, hi = n - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (start[mid] <= blockIdx.x) lo = mid;
+    else hi = mid - 1;
+  }
+  const ElemArgs a = *args[lo];
+  const unsigned bx = blockIdx.x - start[lo], gx = start[lo + 1] - start[lo];
+  const int t = (a.i0 + 31) / 32, x = int(bx) % t, y = int(bx) / t % t, z = int(bx) / (t * t);
+  if constexpr (KIND == int(OpKind::PackPairs))
+    pack_pairs_body(amplitude_pack(a.x0, a.y, a.n, a.i0, a.i1), x, y, z);
+  else if constexpr (KIND == int(OpKind::UnpackHoles))
+    unpack_holes_body(a.x0, a.n, a.i0, a.i1, a.y, const_cast<double *>(a.x1), bx, gx);
+  else
+    add_pairs_body(a.x0, a.n, a.x1, a.y, a.i0, a.i1, x, y, z, a.i1 * a.i1);
+}
+
+// Record of one of them on the engine's tape.
+bool tape_pairs(Engine &e, OpKind kind, const double *x0, const double *x1, double *y,
+                int64_t plane, int64_t blocks) {
+  if (!e.tape) return false;
+  SISI_REQUIRE(blocks < (int64_t(1) << 31), SISI_ERR_INVALID, "pairs: grid too large");
+  TapeOp op;
+  op.kind = kind;
+  op.gx = unsigned(blocks);
+  op.e.x0 = x0;
+  op.e.x1 = x1;
+  op.e.y = y;
+  op.e.n = plane;
+  op.e.i0 = e.Nv;
+  op.e.i1 = e.No;
+  e.tape->ops.push_back(op);
+  return true;
+}
+
 __global__ __launch_bounds__(256) void asymmetry_kernel(const double *T, int v, int o,
                                                         double *flag) {
   const int64_t nv2 = int64_t(v) * v, total = nv2 * o * o;
@@ -208,15 +280,22 @@ bool doubles_symmetric(Engine &e, const double *T2) {
   return f == 0.0;
 }
 
+double kept_ladder_bytes(int64_t No, int64_t Nv) {
+  const Rows rows{Nv, No};
+  return 16.0 * double(rows.count()) * double(rows.pairs());
+}
+
 bool kept_ladder_build(Engine &e) {
   if (e.ladder.get()) return true;
   const int64_t o = e.No, v = e.Nv, G = e.NG, P = o + v;
   const Rows rows{v, o};
   const int64_t K = rows.pairs(), M = rows.count();
-  const double bytes = 16.0 * double(M) * double(K);
+  const double bytes = kept_ladder_bytes(o, v);
   if (o * o > 65535 || P > 65535) return false;  // grids of pack_pairs
-  // a slice of b: temporary of v^2 (o + v) doubles per b, about 2 GB
-  const int64_t nb = std::min<int64_t>(v, std::max<int64_t>(1, (int64_t(1) << 28) / (v * v * P)));
+  // a slice of b: a temporary of v^2 (o + v) doubles per b, at most an eighth
+  // of the result and 2 GB (it stays in the engine's pool)
+  const int64_t most = std::min<int64_t>(int64_t(1) << 28, M * K / 4);
+  const int64_t nb = std::min<int64_t>(v, std::max<int64_t>(1, most / (v * v * P)));
   size_t free_b = 0, total_b = 0;
   if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) return false;
   const double room = kLadderShare * (double(free_b) + double(e.pool.cached_bytes()));
@@ -287,17 +366,9 @@ void kept_ladder_apply(Engine &e, const double *X, double *Q, double *Qh, double
   const int64_t K = rows.pairs(), M = rows.count(), N = rows.opairs();
   SISI_REQUIRE(e.ladder.get(), SISI_ERR_STATE, "ladder: pair integrals not built");
   DBuf Xp(&e.pool, size_t(2 * N * K));
-  PackArgs a{};
-  a.src = X;
-  a.out = Xp.get();
-  a.plane = N * K;
-  a.v = int(v);
-  a.o = int(o);
-  a.mode = kAmplitudes;
-  a.np = int(o);
-  a.scale = 0.5;
-  a.diag = 1.0;
-  pack_pairs(e, a, o * o);
+  const int64_t t32 = (v + 31) / 32;
+  if (!tape_pairs(e, OpKind::PackPairs, X, nullptr, Xp.get(), N * K, t32 * t32 * o * o))
+    pack_pairs(e, amplitude_pack(X, Xp.get(), N * K, int(v), int(o)), o * o);
   GemmArgs g;  // both combinations as one batch
   g.A = e.ladder.get();
   g.B = Xp.get();
@@ -317,6 +388,9 @@ void kept_ladder_apply(Engine &e, const double *X, double *Q, double *Qh, double
   g.dn0 = g.N;
   gemm(e, precision, g);
   const int64_t total = (o * v + N) * N;
+  if (tape_pairs(e, OpKind::UnpackHoles, Q, W, Qh, M * N,
+                 std::min<int64_t>((total + 255) / 256, 256)))
+    return;
   Timed t(*e.timers, Kind::Bandwidth, 32.0 * double(total));
   hipLaunchKernelGGL(unpack_holes_kernel, dim3(unsigned(std::min<int64_t>((total + 255) / 256, 65536))),
                      dim3(256), 0, e.stream, Q, M * N, int(v), int(o), Qh, W);
@@ -327,9 +401,29 @@ void kept_ladder_add(Engine &e, const double *Q, const double *V, double *R2) {
   const Rows rows{e.Nv, e.No};
   const unsigned t = unsigned((e.Nv + 31) / 32);
   const unsigned gz = unsigned(std::min<int64_t>(int64_t(e.No) * e.No, 65535));
+  if (tape_pairs(e, OpKind::AddPairs, Q, V, R2, rows.count() * rows.opairs(),
+                 int64_t(t) * t * e.No * e.No))
+    return;
   Timed tm(*e.timers, Kind::Bandwidth, 28.0 * double(e.n2e()));
   hipLaunchKernelGGL(add_pairs_kernel, dim3(t, t, gz), dim3(256), 0, e.stream, Q,
                      rows.count() * rows.opairs(), V, R2, e.Nv, e.No);
+  SISI_HIP(hipGetLastError());
+}
+
+void launch_pairs_grouped(OpKind kind, const ElemArgs *const *args, const unsigned *start, int n,
+                          unsigned total, hipStream_t s) {
+  switch (kind) {
+#define SISI_PAIRS_CASE(K)                                                                      \
+  case OpKind::K:                                                                               \
+    hipLaunchKernelGGL(pairs_grouped<int(OpKind::K)>, dim3(total), dim3(256), 0, s, args, start, \
+                       n);                                                                      \
+    break;
+    SISI_PAIRS_CASE(PackPairs)
+    SISI_PAIRS_CASE(UnpackHoles)
+    SISI_PAIRS_CASE(AddPairs)
+#undef SISI_PAIRS_CASE
+    default: throw Error(SISI_ERR_INVALID, "grouped launch: unknown kind");
+  }
   SISI_HIP(hipGetLastError());
 }
 

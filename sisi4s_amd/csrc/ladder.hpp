@@ -24,6 +24,8 @@ bool doubles_symmetric(Engine &e, const double *T2);
 // fit (more than kLadderShare of the memory that is free or cached in the
 // pool, or an allocation fails).
 bool kept_ladder_build(Engine &e);
+// Device memory of an engine's pair integrals.
+double kept_ladder_bytes(int64_t No, int64_t Nv);
 
 // Q of X: Qp (kept_ladder_rows x pairs, + and - parts), its hole-particle
 // rows expanded to Qh[k,b,i,j] and its hole rows to W[k,l,i,j].

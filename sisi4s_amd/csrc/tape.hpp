@@ -62,6 +62,10 @@ enum class OpKind : int {
                  // Vabij = x2, Vbaij = x3, i0 = Nv, i1 = No
   GemmReduce,    // GemmArgs: split-K reduction of the preceding Gemm record, gx per
                  // batch entry
+  PackPairs,     // ladder pairs (ladder.hip): X -> pair combinations
+  UnpackHoles,   // ... hole rows of Q
+  AddPairs,      // ... R2 += V + particle rows of Q
+  Symmetrize,    // y = symmetrized doubles, i0 = Nv, i1 = No
 };
 
 struct TapeOp {
@@ -107,6 +111,10 @@ void launch_copy_grouped(OpKind kind, const CopyArgs *const *args, const unsigne
                          unsigned total, hipStream_t s);
 void launch_elem_grouped(OpKind kind, const ElemArgs *const *args, const unsigned *start, int n,
                          unsigned total, hipStream_t s);
+
+// (the pair kinds, ladder.hip)
+void launch_pairs_grouped(OpKind kind, const ElemArgs *const *args, const unsigned *start, int n,
+                          unsigned total, hipStream_t s);
 
 // Lockstep schedule of several tapes (one per system): the i-th launches of
 // the tapes are merged greedily into grouped launches of one (kind, variant)

@@ -583,13 +583,13 @@ __global__ void estimate_kernel(int order, int Nv, int No, double *R, const doub
 // taken by the block with i < j, or i == j and ta <= tb (the others exit):
 // both tiles are staged in LDS, then each element and its partner get the
 // same average (an addition of the same two values in either order).
-__global__ __launch_bounds__(256) void symmetrize_doubles_kernel(double *T, int Nv, int No) {
-  const int ta = int(blockIdx.x), tb = int(blockIdx.y);
+__device__ __forceinline__ void symmetrize_body(double *T, int Nv, int No, int ta, int tb, int ij0,
+                                                int nij) {
   const int x = int(threadIdx.x) & 31, y0 = int(threadIdx.x) >> 5;
   const int64_t nv2 = int64_t(Nv) * Nv;
   __shared__ double s0[32][33], s1[32][33];
   // (i, j) pairs strided by the grid's z extent (block-uniform skips)
-  for (int ij = int(blockIdx.z); ij < No * No; ij += int(gridDim.z)) {
+  for (int ij = ij0; ij < No * No; ij += nij) {
     const int i = ij % No, j = ij / No;
     if (i > j || (i == j && ta > tb)) continue;
     double *P = T + nv2 * (i + int64_t(No) * j);  // [a, b] of (i, j) at a + Nv b
@@ -614,11 +614,26 @@ __global__ __launch_bounds__(256) void symmetrize_doubles_kernel(double *T, int 
   }
 }
 
+__global__ __launch_bounds__(256) void symmetrize_doubles_kernel(double *T, int Nv, int No) {
+  symmetrize_body(T, Nv, No, int(blockIdx.x), int(blockIdx.y), int(blockIdx.z), int(gridDim.z));
+}
+
 void symmetrize_doubles(Engine &e, double *T2, int Nv, int No) {
   SISI_REQUIRE(Nv > 0 && No > 0 && int64_t(No) * No < (int64_t(1) << 31), SISI_ERR_INVALID,
                "symmetrize_doubles: bad shape");
   const unsigned tiles = unsigned((Nv + 31) / 32);
   const unsigned gz = unsigned(std::min<int64_t>(int64_t(No) * No, 65535));
+  if (e.tape) {
+    TapeOp op;
+    op.kind = OpKind::Symmetrize;
+    op.gx = tiles * tiles;
+    op.gy = gz;
+    op.e.y = T2;
+    op.e.i0 = Nv;
+    op.e.i1 = No;
+    e.tape->ops.push_back(op);
+    return;
+  }
   Timed t(*e.timers, Kind::Bandwidth, 16.0 * double(Nv) * Nv * No * No);
   hipLaunchKernelGGL(symmetrize_doubles_kernel, dim3(tiles, tiles, gz), dim3(256), 0, e.stream,
                      T2, Nv, No);
@@ -802,6 +817,10 @@ __global__ __launch_bounds__(256) void elem_grouped(const ElemArgs *const *args,
   else if constexpr (KIND == int(OpKind::DotPartial)) dot_partial_body(a, bx, gx);
   else if constexpr (KIND == int(OpKind::SumPartials)) sum_partials_body(a, bx);
   else if constexpr (KIND == int(OpKind::EnergyPartial)) energy_partial_body(a, bx, gx);
+  else if constexpr (KIND == int(OpKind::Symmetrize)) {
+    const int t = (a.i0 + 31) / 32, tt = t * t;
+    symmetrize_body(a.y, a.i0, a.i1, int(bx) % t, int(bx) / t % t, int(bx) / tt, int(gx) / tt);
+  }
 }
 
 void launch_copy_grouped(OpKind kind, const CopyArgs *const *args, const unsigned *start, int n,
@@ -828,8 +847,9 @@ void launch_elem_grouped(OpKind kind, const ElemArgs *const *args, const unsigne
     SISI_ELEM_CASE(DotPartial)
     SISI_ELEM_CASE(SumPartials)
     SISI_ELEM_CASE(EnergyPartial)
+    SISI_ELEM_CASE(Symmetrize)
 #undef SISI_ELEM_CASE
-    default: throw Error(SISI_ERR_INVALID, "grouped launch: not an element-wise kind");
+    default: return launch_pairs_grouped(kind, args, start, n, total, s);
   }
   SISI_HIP(hipGetLastError());
 }
