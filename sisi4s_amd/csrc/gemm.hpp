@@ -105,10 +105,16 @@ struct B3Seg {
   const unsigned short *Ah = nullptr, *Al = nullptr, *Bh = nullptr, *Bl = nullptr;
   int Kp = 0;
 };
+// out_f: the FP32 accumulators themselves go to out_f (alpha 1, beta 0; g.C
+// unused), at the offsets of C; add0, add1: such results of earlier products
+// are added to this one's in FP64 as C is written (beta 0), which gives the
+// bits that accumulating them in C would.
 struct B3SegArgs {
   GemmArgs g;
   int nseg = 0;
   B3Seg seg[kMaxSegs];
+  float *out_f = nullptr;
+  const float *add0 = nullptr, *add1 = nullptr;
 };
 constexpr int kB3SegTile = 128;  // rows of A and B planes must cover the tile-padded M, N
 void gemm_b3_segments(Engine &e, B3SegArgs a);

@@ -595,10 +595,21 @@ __device__ __forceinline__ B3Seg b3seg_at(const B3SegArgs &a, int s) {
   return s == 0 ? a.seg[0] : s == 1 ? a.seg[1] : s == 2 ? a.seg[2] : a.seg[3];
 }
 
+//
+// Bound by HBM (B's planes and W) and by the MFMAs together, about half each
+// at Nv = 288, so three things count: W (FP64, 8 Nv^3 bytes) is not read and
+// written again by each of a block's three products (out_f, add0, add1: 5
+// passes of 8 Nv^3 bytes become 3), the tile leaves little of the short side
+// ragged (96 or 128 rows of it: Nv = 288 is 3 x 96), and three workgroups per
+// CU overlap one's epilogue with another's products.  Split-BF16x3 (T) pass
+// at No = 14, Nv = 288: 398 -> 348 ms.
+template <int BM, int BN>
 __global__ __launch_bounds__(256) void gemm_b3p_seg_kernel(B3SegArgs p) {
-  constexpr int BM = 128, BN = 128, WM = 64, WN = 64;
+  constexpr int WM = BM / 2, WN = BN / 2;
   constexpr int BK = 32, RS = BK + 8;
-  constexpr int NA = BM * 4 / 256, NB = BN * 4 / 256;
+  constexpr int NA = (BM * 4 + 255) / 256, NB = (BN * 4 + 255) / 256;
+  const bool lastA = BM * 4 % 256 == 0 || threadIdx.x < BM * 4 % 256;
+  const bool lastB = BN * 4 % 256 == 0 || threadIdx.x < BN * 4 % 256;
   __shared__ __attribute__((aligned(16))) u16 Ah[BM * RS];
   __shared__ __attribute__((aligned(16))) u16 Al[BM * RS];
   __shared__ __attribute__((aligned(16))) u16 Bh[BN * RS];
@@ -623,6 +634,7 @@ __global__ __launch_bounds__(256) void gemm_b3p_seg_kernel(B3SegArgs p) {
     const int kb = c * BK;
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
+      if (i == NA - 1 && !lastA) break;
       const int q = tid + 256 * i, row = q >> 2, kq = (q & 3) * 8;
       const int64_t off = int64_t(m0 + row) * Kp + kb + kq;
       ra[i] = *reinterpret_cast<const U128 *>(sg.Ah + off);
@@ -630,6 +642,7 @@ __global__ __launch_bounds__(256) void gemm_b3p_seg_kernel(B3SegArgs p) {
     }
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
+      if (i == NB - 1 && !lastB) break;
       const int q = tid + 256 * i, row = q >> 2, kq = (q & 3) * 8;
       const int64_t off = int64_t(n0 + row) * Kp + kb + kq;
       rb[i] = *reinterpret_cast<const U128 *>(sg.Bh + off);
@@ -639,12 +652,14 @@ __global__ __launch_bounds__(256) void gemm_b3p_seg_kernel(B3SegArgs p) {
   auto store = [&]() {
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
+      if (i == NA - 1 && !lastA) break;
       const int q = tid + 256 * i, row = q >> 2, kq = (q & 3) * 8;
       *reinterpret_cast<U128 *>(&Ah[row * RS + kq]) = ra[i];
       *reinterpret_cast<U128 *>(&Al[row * RS + kq]) = ra[NA + i];
     }
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
+      if (i == NB - 1 && !lastB) break;
       const int q = tid + 256 * i, row = q >> 2, kq = (q & 3) * 8;
       *reinterpret_cast<U128 *>(&Bh[row * RS + kq]) = rb[i];
       *reinterpret_cast<U128 *>(&Bl[row * RS + kq]) = rb[NB + i];
@@ -723,8 +738,18 @@ __global__ __launch_bounds__(256) void gemm_b3p_seg_kernel(B3SegArgs p) {
       for (int i = 0; i < TI; ++i) {
         if (om[i] < 0) continue;
         const int64_t o = om[i] + on;
+        if (p.out_f) {
+          p.out_f[o] = acc[i][j][r];
+          continue;
+        }
         double v = g.alpha * double(acc[i][j][r]);
-        if (g.beta != 0.0) v += g.beta * g.C[o];
+        if (p.add0) {
+          double w = double(p.add0[o]);
+          if (p.add1) w = double(p.add1[o]) + w;
+          v += w;
+        } else if (g.beta != 0.0) {
+          v += g.beta * g.C[o];
+        }
         g.C[o] = v;
       }
     }
@@ -1155,14 +1180,26 @@ void gemm_b3_segments(Engine &e, B3SegArgs a) {
   }
   g.batch = 1;
   g.ksplit = 1;
-  g.tiles_m = (g.M + kB3SegTile - 1) / kB3SegTile;
-  g.tiles_n = (g.N + kB3SegTile - 1) / kB3SegTile;
+  SISI_REQUIRE(!a.out_f || (g.alpha == 1.0 && !a.add0), SISI_ERR_INVALID,
+               "gemm_b3_segments: FP32 output takes no alpha and no addends");
+  // 96-row tiles along the short side where they leave less of it ragged (and
+  // so stay inside the planes, which are padded to 128 rows)
+  auto padded = [](int x, int t) { return (x + t - 1) / t * t; };
+  const int side = std::min(g.M, g.N);
+  const bool t96 = padded(side, 96) < padded(side, 128);
+  const int bm = t96 && g.M == side ? 96 : 128, bn = t96 && bm == 128 ? 96 : 128;
+  g.tiles_m = (g.M + bm - 1) / bm;
+  g.tiles_n = (g.N + bn - 1) / bn;
   g.split_out = !(g.dm0 >= g.M && g.dn0 >= g.N);
   g.xcd_map = 1;
   const int64_t tiles = int64_t(g.tiles_m) * g.tiles_n;
   SISI_REQUIRE(tiles < (int64_t(1) << 31), SISI_ERR_INVALID, "gemm_b3_segments: too many tiles");
   Timed t(*e.timers, Kind::GemmB3, flops);
-  hipLaunchKernelGGL(gemm_b3p_seg_kernel, dim3(unsigned(tiles)), dim3(256), 0, e.stream, a);
+  const dim3 grid(static_cast<unsigned>(tiles));
+  if (bm == 96) hipLaunchKernelGGL((gemm_b3p_seg_kernel<96, 128>), grid, dim3(256), 0, e.stream, a);
+  else if (bn == 96)
+    hipLaunchKernelGGL((gemm_b3p_seg_kernel<128, 96>), grid, dim3(256), 0, e.stream, a);
+  else hipLaunchKernelGGL((gemm_b3p_seg_kernel<128, 128>), grid, dim3(256), 0, e.stream, a);
   SISI_HIP(hipGetLastError());
 }
 

@@ -442,9 +442,10 @@ struct TriplesPlanes {
 
 // build_w on pre-split planes (split-BF16x3, FP32 accumulation).
 void build_w_b3(Engine &e, const TriplesPlanes &pl, const std::array<int, 3> &ib,
-                const std::array<std::array<int, 3>, 6> &perms, const bool *use, double *W) {
+                const std::array<std::array<int, 3>, 6> &perms, const bool *use, double *W, float *W0, float *W1) {
   const int64_t o = e.No, v = e.Nv;
-  bool first = true;
+  B3SegArgs last;  // every product but the last keeps its FP32 sums in W0, W1
+  int done = 0;
   for (int j = 0; j < 3; ++j) {
     const int p = j == 0 ? 1 : 0, q = j == 2 ? 1 : 2;
     B3SegArgs a;
@@ -475,8 +476,7 @@ void build_w_b3(Engine &e, const TriplesPlanes &pl, const std::array<int, 3> &ib
     GemmArgs &g = a.g;
     g.C = W;
     g.alpha = 1.0;
-    g.beta = first ? 0.0 : 1.0;
-    first = false;
+    g.beta = 0.0;
     if (j == 0) {
       g.M = int(v);
       g.N = int(v * v);
@@ -490,8 +490,15 @@ void build_w_b3(Engine &e, const TriplesPlanes &pl, const std::array<int, 3> &ib
       g.N = int(v);
     }
     w_cube_addressing(g, int(v), j, p, q);
-    gemm_b3_segments(e, a);
+    if (last.nseg > 0) {
+      last.out_f = done++ == 0 ? W0 : W1;
+      gemm_b3_segments(e, last);
+    }
+    last = a;
   }
+  if (done > 0) last.add0 = W0;
+  if (done > 1) last.add1 = W1;
+  gemm_b3_segments(e, last);
 }
 
 // The permutations of a block: tup[p] = i.pi_p and whether pi_p gives a
@@ -716,7 +723,13 @@ double triples_energy(Engine &e, const double *T1, const double *T2, int prec,
 
   int norbits = 0;
   DBuf orbits_buf = orbit_codes(e, norbits);
-  DBuf W(&e.pool, w_cube_size(v));
+  DBuf W(&e.pool, w_cube_size(v)), Wf;
+  float *Wf0 = nullptr, *Wf1 = nullptr;
+  if (prec == SISI_BF16X3) {
+    Wf = DBuf(&e.pool, w_cube_size(v));
+    Wf0 = reinterpret_cast<float *>(Wf.get());
+    Wf1 = Wf0 + w_cube_size(v);
+  }
   DBuf part(&e.pool, norbits), Eb(&e.pool, blocks.size());
   zero(e, Eb.get(), blocks.size());
   std::array<std::array<int, 3>, 6> perms;
@@ -728,7 +741,7 @@ double triples_energy(Engine &e, const double *T1, const double *T2, int prec,
     bool distinct[6];
     std::array<int, 3> tup[6];
     block_perms(ib, perms, tup, distinct);
-    if (prec == SISI_BF16X3) build_w_b3(e, pl, ib, perms, distinct, W.get());
+    if (prec == SISI_BF16X3) build_w_b3(e, pl, ib, perms, distinct, W.get(), Wf0, Wf1);
     else build_w(e, prec, op, op, ib, perms, distinct, W.get());
 
     EnergyArgs g{};
