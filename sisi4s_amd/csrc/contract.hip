@@ -89,9 +89,18 @@ bool operand_ok(const Operand &o, const std::string &g1, const std::string &g2,
   return u1 || u2;
 }
 
-// Dense copy of an operand in label order `order`.
+// A view with the imaginary plane as one more index.
+View with_plane(View v, int64_t plane) {
+  v.len[v.order] = 2;
+  v.stride[v.order] = plane;
+  ++v.order;
+  return v;
+}
+
+// Dense copy of an operand in label order `order`; plane != 0: of both planes
+// of a complex operand, and plane becomes the copy's.
 View densify(Engine &e, const Operand &o, const std::string &order,
-             const std::map<char, int64_t> &len, DBuf &store) {
+             const std::map<char, int64_t> &len, DBuf &store, int64_t *plane) {
   int64_t n = 1;
   for (char c : order) n *= len.at(c);
   // Constant operands keep their permuted copies for the whole residual.
@@ -100,6 +109,7 @@ View densify(Engine &e, const Operand &o, const std::string &order,
   if (cached) {
     key = std::to_string(reinterpret_cast<uintptr_t>(o.v->p));
     for (char c : order) key += ":" + std::to_string(len.at(c)) + "/" + std::to_string(o.stride.at(c));
+    if (plane) key += ":z" + std::to_string(*plane);
   }
   View d;
   d.order = int(order.size());
@@ -113,10 +123,11 @@ View densify(Engine &e, const Operand &o, const std::string &order,
         d.stride[k] = st;
         st *= d.len[k];
       }
+      if (plane) *plane = n;
       return d;
     }
   }
-  store = DBuf(&e.pool, size_t(std::max<int64_t>(n, 1)));
+  store = DBuf(&e.pool, size_t(std::max<int64_t>(n, 1) * (plane ? 2 : 1)));
   d.p = store.get();
   View s;
   s.p = o.v->p;
@@ -134,7 +145,12 @@ View densify(Engine &e, const Operand &o, const std::string &order,
     d.len[0] = s.len[0] = 1;
     d.stride[0] = s.stride[0] = 1;
   }
-  copy(e, d, s);
+  if (plane) {
+    copy(e, with_plane(d, n), with_plane(s, *plane));
+    *plane = n;
+  } else {
+    copy(e, d, s);
+  }
   if (cached) e.perm_cache[key] = std::move(store);
   return d;
 }
@@ -151,7 +167,7 @@ Operand operand_from_dense(const View &d, const std::string &order) {
 
 void contract(Engine &e, double alpha, const View &Av, const std::string &ia, const View &Bv,
               const std::string &ib, double beta, const View &Cv, const std::string &ic,
-              int precision) {
+              int precision, const ZPlanes *z) {
   if (precision < 0) precision = e.precision;
   std::map<char, int64_t> len;
   Operand A = make_operand(Av, ia, len);
@@ -174,6 +190,8 @@ void contract(Engine &e, double alpha, const View &Av, const std::string &ia, co
                                         " must appear in two of the three operands (" + ia +
                                         "," + ib + "->" + ic + ")");
   }
+  ZPlanes zp = z ? *z : ZPlanes{0, 0, 0, 1.0, 1.0};
+  SISI_REQUIRE(!z || gB.empty(), SISI_ERR_INVALID, "contract: complex product with a batch label");
   std::string Mord = in_order(A, gM), Nord = in_order(B, gN), Bord = in_order(C, gB);
   std::string KA = in_order(A, gK), KB = in_order(B, gK), Kord;
   // The epilogue's lanes run along the first M (or, swapped, N) label.  When
@@ -218,11 +236,11 @@ void contract(Engine &e, double alpha, const View &Av, const std::string &ia, co
     permA = permB = true;
   }
   if (permA) {
-    dA = densify(e, A, Mord + Kord + Bord, len, storeA);
+    dA = densify(e, A, Mord + Kord + Bord, len, storeA, z ? &zp.a : nullptr);
     A = operand_from_dense(dA, Mord + Kord + Bord);
   }
   if (permB) {
-    dB = densify(e, B, Kord + Nord + Bord, len, storeB);
+    dB = densify(e, B, Kord + Nord + Bord, len, storeB, z ? &zp.b : nullptr);
     B = operand_from_dense(dB, Kord + Nord + Bord);
   }
 
@@ -235,7 +253,8 @@ void contract(Engine &e, double alpha, const View &Av, const std::string &ia, co
   if (!c_direct) {
     const std::string order = Mord + Nord + Bord;
     int64_t n = prod(order, len);
-    storeC = DBuf(&e.pool, size_t(n));
+    storeC = DBuf(&e.pool, size_t(z ? 2 * n : n));
+    zp.c = n;
     tmpC.p = storeC.get();
     tmpC.order = int(order.size());
     int64_t st = 1;
@@ -323,6 +342,15 @@ void contract(Engine &e, double alpha, const View &Av, const std::string &ia, co
   g.C = Cw.v->p;
   g.alpha = alpha;
   g.beta = c_direct ? beta : 0.0;
+  if (z) {
+    g.cplx = 1;
+    g.batch = 2;
+    g.za = swap ? zp.b : zp.a;
+    g.zb = swap ? zp.a : zp.b;
+    g.sa = swap ? zp.sb : zp.sa;
+    g.sb = swap ? zp.sa : zp.sb;
+    g.bsc = zp.c;
+  }
   gemm(e, precision, g);
 
   if (!c_direct) {
@@ -336,6 +364,10 @@ void contract(Engine &e, double alpha, const View &Av, const std::string &ia, co
       src.len[k] = dst.len[k] = tmpC.len[k];
       src.stride[k] = tmpC.stride[k];
       dst.stride[k] = C.stride.at(order[k]);
+    }
+    if (z) {
+      dst = with_plane(dst, z->c);
+      src = with_plane(src, zp.c);
     }
     copy(e, dst, src, 1.0, beta);
   }

@@ -18,9 +18,17 @@ namespace sisi {
 
 // C[ic] = alpha * A[ia] * B[ib] + beta * C[ic].  precision < 0 uses the
 // engine's current precision.
+// Imaginary planes of planar complex operands: elements from each real plane
+// to its imaginary one, and the signs of the operands (-1: conjugated).  With
+// them a contraction is complex, in one launch (FP64 or FP32, no batch label).
+struct ZPlanes {
+  int64_t a, b, c;
+  double sa, sb;
+};
+
 void contract(Engine &e, double alpha, const View &A, const std::string &ia,
               const View &B, const std::string &ib, double beta, const View &C,
-              const std::string &ic, int precision = -1);
+              const std::string &ic, int precision = -1, const ZPlanes *z = nullptr);
 
 // einsum-style spelling: ctr(e, alpha, "cdkl,adkl->ac", A, B, beta, C).
 void ctr(Engine &e, double alpha, const char *spec, const View &A, const View &B,

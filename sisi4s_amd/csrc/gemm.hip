@@ -427,7 +427,9 @@ static K4Plan plan_k4(GemmArgs &g, int precision, int cus, bool taped) {
     if (taped) {
       p.tile = kTapeTile;
     } else {
-      const TilePlan t = choose_tile(g, precision, cus);
+      GemmArgs c = g;  // a complex part is two plane products
+      if (g.cplx) c.K = int(std::min<int64_t>(2 * int64_t(g.K), (int64_t(1) << 31) - 1));
+      const TilePlan t = choose_tile(c, precision, cus);
       p.tile = t.tile;
       ksplit = t.ksplit;
     }
@@ -456,7 +458,11 @@ static void set_ksplit(GemmArgs &g, int ksplit, int kq) {
 static void launch_planned(GemmArgs &g, int precision, const K4Plan &p, hipStream_t s) {
   SISI_REQUIRE(g.batch <= 65535 && g.ksplit <= 65535, SISI_ERR_INVALID, "gemm: grid too large");
   dim3 grid(unsigned(int64_t(g.tiles_m) * g.tiles_n), unsigned(g.ksplit), unsigned(g.batch));
-  if (precision == SISI_FP64) launch_k4_fp64(p.tile, p.map, g, grid, s);
+  if (g.cplx) {
+    SISI_REQUIRE(g.batch == 2 && (precision == SISI_FP64 || precision == SISI_FP32),
+                 SISI_ERR_INVALID, "gemm: complex products are FP64 or FP32, batch 2");
+    (precision == SISI_FP64 ? launch_k4z_fp64 : launch_k4z_fp32)(p.tile, p.map, g, grid, s);
+  } else if (precision == SISI_FP64) launch_k4_fp64(p.tile, p.map, g, grid, s);
   else if (precision == SISI_FP32) launch_k4_fp32(p.tile, p.map, g, grid, s);
   else launch_b3(g, grid, s, (p.map & 2) != 0, (p.map & 1) != 0);
   SISI_HIP(hipGetLastError());
@@ -527,6 +533,7 @@ static void tape_gemm(Engine &eng, int precision, GemmArgs g) {
 
 void gemm(Engine &eng, int precision, GemmArgs g, bool exact) {
   if (g.M <= 0 || g.N <= 0 || g.batch <= 0) return;
+  SISI_REQUIRE(!g.cplx || !eng.tape, SISI_ERR_INVALID, "gemm: complex products are not recorded");
   if (eng.tape) return tape_gemm(eng, precision, g);
   // split-BF16x3 splits both operands first (a bandwidth pass over each); a
   // product too small to amortise that runs on FP32 MFMA instead

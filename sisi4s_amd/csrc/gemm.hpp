@@ -52,6 +52,13 @@ struct GemmArgs {
   // (cn* for n).  This writes tensors stored as contiguous 8 x 8 x 8 cubes.
   int out_cube = 0;
   int64_t cm3 = 0, cn3 = 0;
+  // cplx = 1 (FP64 / FP32, batch = 2): one product of planar complex operands,
+  // the imaginary planes za, zb elements after the real ones (C's: bsc);
+  // batch entry 0 is Re C = Re A Re B - sa sb Im A Im B, entry 1 is Im C =
+  // sb Re A Im B + sa Im A Re B (sa, sb = -1: conjugated operand)
+  int cplx = 0;
+  int64_t za = 0, zb = 0;
+  double sa = 1.0, sb = 1.0;
 };
 
 // One product of a segmented GEMM: A(m,k) = A[m*sam + k*sak],
@@ -185,9 +192,9 @@ void gemm_reduce(Engine &eng, const GemmArgs &g);
 // for (the split's extra pass over the operands would dominate).
 constexpr double kB3MinFlops = 1e10;
 
-// Algorithmic flops of one call (2*M*N*K*batch).
+// Algorithmic flops of one call (2*M*N*K*batch; twice that in complex).
 inline double gemm_flops(const GemmArgs &g) {
-  return 2.0 * double(g.M) * double(g.N) * double(g.K) * double(g.batch);
+  return 2.0 * double(g.M) * double(g.N) * double(g.K) * double(g.batch) * (g.cplx ? 2.0 : 1.0);
 }
 
 }  // namespace sisi

@@ -18,6 +18,9 @@ constexpr int kNumTiles = 3;
 // Load mappings: 0: A m-fast, B k-fast; +1: B n-fast; +2: A k-fast.
 void launch_k4_fp64(int tile, int map, const GemmArgs &g, dim3 grid, hipStream_t s);
 void launch_k4_fp32(int tile, int map, const GemmArgs &g, dim3 grid, hipStream_t s);
+// The same for planar complex operands (g.cplx).
+void launch_k4z_fp64(int tile, int map, const GemmArgs &g, dim3 grid, hipStream_t s);
+void launch_k4z_fp32(int tile, int map, const GemmArgs &g, dim3 grid, hipStream_t s);
 // Grouped launch of n products (batched solver): record p owns the blocks
 // [start[p], start[p + 1]): tiles_m * tiles_n per k-split and batch entry.
 // The systems of a grouped launch fill the device together, and one tile for
@@ -30,8 +33,11 @@ void launch_k4_grouped_fp32(int map, const GemmArgs *const *args, const unsigned
 
 #ifdef __HIPCC__
 
-// Output tile `pid`, k-split `ks`, batch entry `bz` of one product.
-template <int PREC, int TBM, int TBN, int WGM, int WGN, bool AK, bool BNF>
+// Output tile `pid`, k-split `ks`, batch entry `bz` of one product.  CPLX: the
+// part bz (0 Re, 1 Im) of a planar complex product, its two plane products as
+// one k loop (a separate launch and a read-modify-write of C for each of the
+// four took a 9-orbital complex CCSD iteration 590 launches).
+template <int PREC, int TBM, int TBN, int WGM, int WGN, bool AK, bool BNF, bool CPLX = false>
 __device__ __forceinline__ void gemm_k4_body(const GemmArgs &g, int pid, int ks, int bz) {
   using LT = typename TileTypes<PREC>::LT;
   using AT = typename TileTypes<PREC>::AT;
@@ -49,13 +55,30 @@ __device__ __forceinline__ void gemm_k4_body(const GemmArgs &g, int pid, int ks,
   const int m0 = tm * TBM, n0 = tn * TBN;
   const int kbeg = ks * g.kchunk;
   const int kend = min(g.K, kbeg + g.kchunk);
-  const int chunks = (kend - kbeg + kTileK - 1) / kTileK;
+  const int half = (kend - kbeg + kTileK - 1) / kTileK;  // chunks of one plane product
+  const int chunks = CPLX ? 2 * half : half;
 
   TileLoader<LT, TBM, AK> la;
   TileLoader<LT, TBN, !BNF> lb;
-  la.init(g.A + int64_t(bz) * g.bsa, g.sam, g.sak, m0, g.M - 1, kbeg);
-  lb.init(g.B + int64_t(bz) * g.bsb, g.sbn, g.sbk, n0, g.N - 1, kbeg);
+  // second plane product of a complex part: Im A with Im B (Re C) or Re B (Im C)
+  double scale = 1.0;  // of the chunk in the registers
+  if constexpr (CPLX) {
+    la.init(g.A, g.sam, g.sak, m0, g.M - 1, kbeg);
+    lb.init(g.B + (bz ? g.zb : 0), g.sbn, g.sbk, n0, g.N - 1, kbeg);
+    scale = bz ? g.sb : 1.0;
+  } else {
+    la.init(g.A + int64_t(bz) * g.bsa, g.sam, g.sak, m0, g.M - 1, kbeg);
+    lb.init(g.B + int64_t(bz) * g.bsb, g.sbn, g.sbk, n0, g.N - 1, kbeg);
+  }
   auto load = [&](int c) {
+    if constexpr (CPLX) {
+      if (c == half) {
+        la.init(g.A + g.za, g.sam, g.sak, m0, g.M - 1, kbeg);
+        lb.init(g.B + (bz ? 0 : g.zb), g.sbn, g.sbk, n0, g.N - 1, kbeg);
+        scale = bz ? g.sa : -g.sa * g.sb;
+      }
+      if (c >= half) c -= half;
+    }
     const int nk = kend - kbeg - c * kTileK;
     if (nk >= kTileK) {
       la.load();
@@ -78,6 +101,7 @@ __device__ __forceinline__ void gemm_k4_body(const GemmArgs &g, int pid, int ks,
 
   if (chunks > 0) {
     load(0);
+    if (CPLX && scale != 1.0) la.scale(scale);
     la.store(As[0]);
     lb.store(Bs[0]);
     if (chunks > 1) load(1);
@@ -85,6 +109,7 @@ __device__ __forceinline__ void gemm_k4_body(const GemmArgs &g, int pid, int ks,
     for (int c = 0; c < chunks; ++c) {
       // buffer (c + 1) & 1 was last read before the barrier just passed
       if (c + 1 < chunks) {
+        if (CPLX && scale != 1.0) la.scale(scale);
         la.store(As[(c + 1) & 1]);
         lb.store(Bs[(c + 1) & 1]);
         if (c + 2 < chunks) load(c + 2);
@@ -141,9 +166,9 @@ __device__ __forceinline__ void gemm_k4_body(const GemmArgs &g, int pid, int ks,
   }
 }
 
-template <int PREC, int TBM, int TBN, int WGM, int WGN, bool AK, bool BNF>
+template <int PREC, int TBM, int TBN, int WGM, int WGN, bool AK, bool BNF, bool CPLX>
 __global__ __launch_bounds__(256, 2) void gemm_k4_kernel(GemmArgs g) {
-  gemm_k4_body<PREC, TBM, TBN, WGM, WGN, AK, BNF>(g, blockIdx.x, blockIdx.y, blockIdx.z);
+  gemm_k4_body<PREC, TBM, TBN, WGM, WGN, AK, BNF, CPLX>(g, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
 template <int PREC, int TBM, int TBN, int WGM, int WGN, bool AK, bool BNF>
@@ -165,13 +190,13 @@ __global__ __launch_bounds__(256, 2) void gemm_k4_grouped(const GemmArgs *const 
   gemm_k4_body<PREC, TBM, TBN, WGM, WGN, AK, BNF>(g, local % tiles, r % g.ksplit, r / g.ksplit);
 }
 
-template <int PREC>
+template <int PREC, bool CPLX>
 void launch_k4_tiles(int tile, int map, const GemmArgs &g, dim3 grid, hipStream_t s) {
   switch (tile * 4 + map) {
 #define SISI_K4_ONE(T, MAP, AK_, BNF_)                                                          \
   case T * 4 + MAP:                                                                             \
-    hipLaunchKernelGGL((gemm_k4_kernel<PREC, kTiles[T], kTiles[T], 2, 2, AK_, BNF_>), grid,     \
-                       dim3(256), 0, s, g);                                                     \
+    hipLaunchKernelGGL((gemm_k4_kernel<PREC, kTiles[T], kTiles[T], 2, 2, AK_, BNF_, CPLX>),     \
+                       grid, dim3(256), 0, s, g);                                               \
     break;
 #define SISI_K4_ALL(T)             \
   SISI_K4_ONE(T, 0, false, false)  \

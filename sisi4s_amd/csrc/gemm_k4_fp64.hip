@@ -4,7 +4,7 @@
 namespace sisi {
 
 void launch_k4_fp64(int tile, int map, const GemmArgs &g, dim3 grid, hipStream_t s) {
-  launch_k4_tiles<SISI_FP64>(tile, map, g, grid, s);
+  launch_k4_tiles<SISI_FP64, false>(tile, map, g, grid, s);
 }
 
 void launch_k4_grouped_fp64(int map, const GemmArgs *const *args, const unsigned *start, int n,

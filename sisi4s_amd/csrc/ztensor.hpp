@@ -27,10 +27,26 @@ inline ZV zsub(const ZV &v, std::initializer_list<int64_t> lo, std::initializer_
   return {subview(v.re, lo, hi), subview(v.im, lo, hi)};
 }
 
-// C = alpha * op(A) op(B) + beta * C, op = conj when the flag is set.
+// C = alpha * op(A) op(B) + beta * C, op = conj when the flag is set.  FP64 and
+// FP32 products without a batch label run as one complex product; the
+// split-BF16x3 kernels and batched products take the planes one by one.
 inline void zctr(Engine &e, double alpha, const char *spec, const ZV &A, bool ca, const ZV &B, bool cb,
           double beta, const ZV &C, int prec) {
   const double sa = ca ? -1.0 : 1.0, sb = cb ? -1.0 : 1.0;
+  const std::string s(spec);
+  const size_t comma = s.find(','), arrow = s.find("->");
+  const std::string ia = s.substr(0, comma), ib = s.substr(comma + 1, arrow - comma - 1),
+                    ic = s.substr(arrow + 2);
+  bool batch = false;
+  for (size_t k = 0; k < ia.size(); ++k)
+    batch = batch || (A.re.len[k] > 1 && ib.find(ia[k]) != std::string::npos &&
+                      ic.find(ia[k]) != std::string::npos);
+  const int p = prec < 0 ? e.precision : prec;
+  if (!batch && (p == SISI_FP64 || p == SISI_FP32)) {
+    const ZPlanes z{A.im.p - A.re.p, B.im.p - B.re.p, C.im.p - C.re.p, sa, sb};
+    contract(e, alpha, A.re, ia, B.re, ib, beta, C.re, ic, p, &z);
+    return;
+  }
   ctr(e, alpha, spec, A.re, B.re, beta, C.re, prec);
   ctr(e, -alpha * sa * sb, spec, A.im, B.im, 1.0, C.re, prec);
   ctr(e, alpha * sb, spec, A.re, B.im, beta, C.im, prec);
