@@ -101,6 +101,16 @@ void ccsd_residual(Engine &e, int it, bool initial_doubles, int slice_size, cons
   e.frozen = {T1p, T2p, e.Vabij.get(), e.Uabij.get(), e.Vaibj.get(), e.Vijka.get(),
               e.Gij.get(), e.Gai.get(), e.Gab.get()};
 
+  // The first anchor of a run is at T = 0: a product with an amplitude is zero
+  // and is not run (every call below through tctr has one, directly or through
+  // an intermediate); what is left are the vertex products, the ladder's kept
+  // planes and R2 = V.  No = 30, Nv = 300, six mixed iterations: 557 -> 474 ms.
+  const bool zt = e.zero_amplitudes;
+  auto tctr = [&](double alpha, const char *spec, const View &A, const View &B, double beta,
+                  const View &C, int p) {
+    if (!zt) ctr(e, alpha, spec, A, B, beta, C, p);
+    else if (beta == 0.0) zero(e, C.p, C.size());
+  };
   DBuf Xb(&e.pool, n2);
   View X = V4(Xb.get(), v, v, o, o);
   add_t1t1(e, Xb.get(), T2p, T1p, 1.0, int(v), int(o));  // cxx:136-138
@@ -111,64 +121,64 @@ void ccsd_residual(Engine &e, int it, bool initial_doubles, int slice_size, cons
        Lki = V2(Lkib.get(), o, o);
   {
     // Kac = -2 V[cdkl] X[adkl] + V[dckl] X[adkl] = -U[cdkl] X[adkl] (cxx:146-147)
-    ctr(e, -1.0, "cdkl,adkl->ac", U, X, 0.0, Kac, prec);
+    tctr(-1.0, "cdkl,adkl->ac", U, X, 0.0, Kac, prec);
     // distinguishable: Lac = -V[cdkl] Y[adkl] + V[dckl] Y[adkl] / 2
     // = -U[cdkl] Y[adkl] / 2 with Y = T2 + 2 T1 T1 (cxx:150-160)
     DBuf Ydb;
     if (e.distinguishable) {
       Ydb = DBuf(&e.pool, n2);
       add_t1t1(e, Ydb.get(), T2p, T1p, 2.0, int(v), int(o));
-      ctr(e, -0.5, "cdkl,adkl->ac", U, V4(Ydb.get(), v, v, o, o), 0.0, Lac, prec);
+      tctr(-0.5, "cdkl,adkl->ac", U, V4(Ydb.get(), v, v, o, o), 0.0, Lac, prec);
     } else {
       copy(e, Lac, Kac);  // cxx:151
     }
     // + 2 Gamma_Gca Gamma_Gdk T_dk (cxx:162-165)
     DBuf Zb(&e.pool, G);
-    ctr(e, 1.0, "Gdk,dk->G", Gai, T1, 0.0, V1(Zb.get(), G), prec);
-    ctr(e, 2.0, "Gca,G->ac", Gab, V1(Zb.get(), G), 1.0, Lac, prec);
+    tctr(1.0, "Gdk,dk->G", Gai, T1, 0.0, V1(Zb.get(), G), prec);
+    tctr(2.0, "Gca,G->ac", Gab, V1(Zb.get(), G), 1.0, Lac, prec);
     // - Gamma_Gck Gamma_Gda T_dk (cxx:166-169)
     DBuf Yb(&e.pool, G * v * o);
-    ctr(e, 1.0, "Gda,dk->Gak", Gab, T1, 0.0, V3(Yb.get(), G, v, o), prec);
-    ctr(e, -1.0, "Gck,Gak->ac", Gai, V3(Yb.get(), G, v, o), 1.0, Lac, prec);
+    tctr(1.0, "Gda,dk->Gak", Gab, T1, 0.0, V3(Yb.get(), G, v, o), prec);
+    tctr(-1.0, "Gck,Gak->ac", Gai, V3(Yb.get(), G, v, o), 1.0, Lac, prec);
     // Kki = 2 V[cdkl] X[cdil] - V[dckl] X[cdil] = U[cdkl] X[cdil] (cxx:172-173)
-    ctr(e, 1.0, "cdkl,cdil->ki", U, X, 0.0, Kki, prec);
+    tctr(1.0, "cdkl,cdil->ki", U, X, 0.0, Kki, prec);
     if (e.distinguishable)  // Lki = U[cdkl] Y[cdil] / 2 (cxx:176-186)
-      ctr(e, 0.5, "cdkl,cdil->ki", U, V4(Ydb.get(), v, v, o, o), 0.0, Lki, prec);
+      tctr(0.5, "cdkl,cdil->ki", U, V4(Ydb.get(), v, v, o, o), 0.0, Lki, prec);
     else
       copy(e, Lki, Kki);  // cxx:177
-    ctr(e, 2.0, "klic,cl->ki", Vijka, T1, 1.0, Lki, prec);   // cxx:188
-    ctr(e, -1.0, "lkic,cl->ki", Vijka, T1, 1.0, Lki, prec);  // cxx:189
+    tctr(2.0, "klic,cl->ki", Vijka, T1, 1.0, Lki, prec);   // cxx:188
+    tctr(-1.0, "lkic,cl->ki", Vijka, T1, 1.0, Lki, prec);  // cxx:189
     e.record("Kac", Kacb.get(), v * v);
     e.record("Lac", Lacb.get(), v * v);
     e.record("Kki", Kkib.get(), o * o);
     e.record("Lki", Lkib.get(), o * o);
-    ctr(e, 1.0, "ac,cbij->abij", Lac, T2, 1.0, R2, prec);    // cxx:192
-    ctr(e, -1.0, "ki,abkj->abij", Lki, T2, 1.0, R2, prec);   // cxx:195
+    tctr(1.0, "ac,cbij->abij", Lac, T2, 1.0, R2, prec);    // cxx:192
+    tctr(-1.0, "ki,abkj->abij", Lki, T2, 1.0, R2, prec);   // cxx:195
   }
   {
     // dressed Gamma_ai and its terms (cxx:198-216)
     DBuf dGb(&e.pool, G * v * o), Qb(&e.pool, G * v * o);
     View dGai = V3(dGb.get(), G, v, o), Q = V3(Qb.get(), G, v, o);
     copy(e, dGai, Gai);
-    ctr(e, -1.0, "Gki,ak->Gai", Gij, T1, 1.0, dGai, prec);   // cxx:205
-    ctr(e, 1.0, "Gbc,cj->Gbj", Gab, T1, 0.0, Q, prec);       // cxx:208 (Gamma_Gbc T_cj)
+    tctr(-1.0, "Gki,ak->Gai", Gij, T1, 1.0, dGai, prec);   // cxx:205
+    tctr(1.0, "Gbc,cj->Gbj", Gab, T1, 0.0, Q, prec);       // cxx:208 (Gamma_Gbc T_cj)
     e.record("dGai2b", dGb.get(), G * v * o);
     e.record("Q", Qb.get(), G * v * o);
-    ctr(e, 1.0, "Gai,Gbj->abij", dGai, Q, 1.0, R2, prec);    // cxx:208-209
-    ctr(e, -1.0, "jika,bk->abij", Vijka, T1, 1.0, R2, prec); // cxx:213
+    tctr(1.0, "Gai,Gbj->abij", dGai, Q, 1.0, R2, prec);    // cxx:208-209
+    tctr(-1.0, "jika,bk->abij", Vijka, T1, 1.0, R2, prec); // cxx:213
     DBuf Pb(&e.pool, v * o * o * o);
     View P = V4(Pb.get(), v, o, o, o);
-    ctr(e, 1.0, "acik,cj->aikj", V, T1, 0.0, P, prec);       // cxx:214-215
+    tctr(1.0, "acik,cj->aikj", V, T1, 0.0, P, prec);       // cxx:214-215
     e.record("P", Pb.get(), v * o * o * o);
-    ctr(e, -1.0, "bk,aikj->abij", T1, P, 1.0, R2, prec);
+    tctr(-1.0, "bk,aikj->abij", T1, P, 1.0, R2, prec);
   }
   {
     // Xakic (cxx:218-252)
     DBuf dGb(&e.pool, G * v * o);
     View dGai = V3(dGb.get(), G, v, o);
     copy(e, dGai, Gai);
-    ctr(e, -1.0, "Gil,al->Gai", Gij, T1, 1.0, dGai, prec);  // cxx:227
-    ctr(e, 1.0, "Gad,di->Gai", Gab, T1, 1.0, dGai, prec);   // cxx:230
+    tctr(-1.0, "Gil,al->Gai", Gij, T1, 1.0, dGai, prec);  // cxx:227
+    tctr(1.0, "Gad,di->Gai", Gab, T1, 1.0, dGai, prec);   // cxx:230
     // Rings.  The reference's seven products of 2 Nv^3 No^3 flops (cxx:242-251,
     // 283-289) are four in this form: with Y2[cbkj] = 2 T[cbkj] - T[bckj],
     //   Xakic Y2 - Xakci T[cbkj] = (Xakic - Xakci / 2) Y2 - P / 2,
@@ -189,8 +199,8 @@ void ccsd_residual(Engine &e, int it, bool initial_doubles, int slice_size, cons
     View dGab = V3(dGabb.get(), G, v, v), dGij = V3(dGijb.get(), G, o, o);
     copy(e, dGab, Gab);
     copy(e, dGij, Gij);
-    ctr(e, -1.0, "Gcl,al->Gac", Gai, T1, 1.0, dGab, prec);  // cxx:270
-    ctr(e, 1.0, "Gdk,di->Gki", Gai, T1, 1.0, dGij, prec);   // cxx:273
+    tctr(-1.0, "Gcl,al->Gac", Gai, T1, 1.0, dGab, prec);  // cxx:270
+    tctr(1.0, "Gdk,di->Gki", Gai, T1, 1.0, dGij, prec);   // cxx:273
     e.record("dGab4", dGabb.get(), G * v * v);
     e.record("dGij4", dGijb.get(), G * o * o);
     ctr(e, 1.0, "Gac,Gki->akci", dGab, dGij, 0.0, Xakci, prec);  // cxx:277-278
@@ -198,32 +208,32 @@ void ccsd_residual(Engine &e, int it, bool initial_doubles, int slice_size, cons
       e.frozen.push_back(Y2b.get());
       DBuf Qb(&e.pool, v * o * o * o);
       View Q = V4(Qb.get(), v, o, o, o);
-      ctr(e, 1.0, "dclk,di->clki", V, T1, 0.0, Q, prec);
-      ctr(e, -1.0, "clki,al->akic", Q, T1, 1.0, Xakic, prec);
+      tctr(1.0, "dclk,di->clki", V, T1, 0.0, Q, prec);
+      tctr(-1.0, "clki,al->akic", Q, T1, 1.0, Xakic, prec);
       sum(e, -0.5, Xakci, "akci", 1.0, Xakic, "akic");  // before its T2 term
-      ctr(e, 0.25, "dclk,adil->akic", U, Y2, 1.0, Xakic, prec);
+      tctr(0.25, "dclk,adil->akic", U, Y2, 1.0, Xakic, prec);
       e.record("Bakic", Xkb.get(), v * o * o * v);
-      ctr(e, -0.5, "cdlk,dail->akci", V, T2, 1.0, Xakci, prec);  // cxx:283-285
+      tctr(-0.5, "cdlk,dail->akci", V, T2, 1.0, Xakci, prec);  // cxx:283-285
       e.record("Xakci", Xcb.get(), v * o * v * o);
-      ctr(e, 1.0, "akic,cbkj->abij", Xakic, Y2, 1.0, R2, prec);
+      tctr(1.0, "akic,cbkj->abij", Xakic, Y2, 1.0, R2, prec);
       e.unfreeze(Y2b.get());
       DBuf Pb(&e.pool, n2);
       View P = V4(Pb.get(), v, v, o, o);
-      ctr(e, 1.0, "akci,bckj->abij", Xakci, T2, 0.0, P, prec);
+      tctr(1.0, "akci,bckj->abij", Xakci, T2, 0.0, P, prec);
       axpby(e, n2, -0.5, Pb.get(), 1.0, R2p);
       sum(e, -1.0, P, "baij", 1.0, R2, "abij");
     } else {
       DBuf Yb(&e.pool, n2);
       View Y = V4(Yb.get(), v, v, o, o);
       add_t1t1(e, Yb.get(), T2p, T1p, 2.0, int(v), int(o));     // cxx:238-240
-      ctr(e, -0.5, "dclk,dail->akic", V, Y, 1.0, Xakic, prec);  // cxx:242
-      ctr(e, 1.0, "dclk,adil->akic", V, T2, 1.0, Xakic, prec);  // cxx:243
+      tctr(-0.5, "dclk,dail->akic", V, Y, 1.0, Xakic, prec);  // cxx:242
+      tctr(1.0, "dclk,adil->akic", V, T2, 1.0, Xakic, prec);  // cxx:243
       e.record("Xakic", Xkb.get(), v * o * o * v);
       e.record("Xakci", Xcb.get(), v * o * v * o);
-      ctr(e, 1.0, "akic,cbkj->abij", Xakic, Y2, 1.0, R2, prec);  // cxx:251
+      tctr(1.0, "akic,cbkj->abij", Xakic, Y2, 1.0, R2, prec);  // cxx:251
       e.frozen.push_back(Xcb.get());
-      ctr(e, -1.0, "akci,cbkj->abij", Xakci, T2, 1.0, R2, prec);  // cxx:288
-      ctr(e, -1.0, "bkci,ackj->abij", Xakci, T2, 1.0, R2, prec);  // cxx:289
+      tctr(-1.0, "akci,cbkj->abij", Xakci, T2, 1.0, R2, prec);  // cxx:288
+      tctr(-1.0, "bkci,ackj->abij", Xakci, T2, 1.0, R2, prec);  // cxx:289
       e.unfreeze(Xcb.get());  // Xcb returns to the pool at the end of this block
     }
   }
@@ -238,8 +248,8 @@ void ccsd_residual(Engine &e, int it, bool initial_doubles, int slice_size, cons
     DBuf Qhb(&e.pool, o * v * o * o);
     View Qh = V4(Qhb.get(), o, v, o, o), W = V4(Wb.get(), o, o, o, o);
     kept_ladder_apply(e, Xb.get(), Qb.get(), Qhb.get(), Wb.get(), e.prec_ladder);
-    ctr(e, -0.5, "bl,klij->kbij", T1, W, 1.0, Qh, prec);
-    ctr(e, -1.0, "ak,kbij->abij", T1, Qh, 1.0, R2, prec);
+    tctr(-0.5, "bl,klij->kbij", T1, W, 1.0, Qh, prec);
+    tctr(-1.0, "ak,kbij->abij", T1, Qh, 1.0, R2, prec);
   }
   {
     // R_abij += R_baji (cxx:292)
@@ -254,24 +264,24 @@ void ccsd_residual(Engine &e, int it, bool initial_doubles, int slice_size, cons
     DBuf Xb4(&e.pool, o * o * o * o);
     View Xklij = V4(Xb4.get(), o, o, o, o);
     copy(e, Xklij, Vijkl);
-    ctr(e, 1.0, "klic,cj->klij", Vijka, T1, 1.0, Xklij, prec);  // cxx:308
-    ctr(e, 1.0, "lkjc,ci->klij", Vijka, T1, 1.0, Xklij, prec);  // cxx:309
+    tctr(1.0, "klic,cj->klij", Vijka, T1, 1.0, Xklij, prec);  // cxx:308
+    tctr(1.0, "lkjc,ci->klij", Vijka, T1, 1.0, Xklij, prec);  // cxx:309
     e.record("Xklij1", Xb4.get(), o * o * o * o);
-    ctr(e, 1.0, "klij,abkl->abij", Xklij, X, 1.0, R2, prec);    // cxx:313
+    tctr(1.0, "klij,abkl->abij", Xklij, X, 1.0, R2, prec);    // cxx:313
     if (e.distinguishable) {
       // Xklij = T[ci] V[cdkl] T[dj] (cxx:319): V contracted with X - T2
       DBuf Wb(&e.pool, n2);
       axpby(e, n2, 1.0, Xb.get(), 0.0, Wb.get());
       axpby(e, n2, -1.0, T2p, 1.0, Wb.get());
-      ctr(e, 1.0, "cdkl,cdij->klij", V, V4(Wb.get(), v, v, o, o), 0.0, Xklij, prec);
+      tctr(1.0, "cdkl,cdij->klij", V, V4(Wb.get(), v, v, o, o), 0.0, Xklij, prec);
     } else if (kept) {
       copy(e, Xklij, V4(Wb.get(), o, o, o, o));  // Q[kl] is this product
     } else {
-      ctr(e, 1.0, "cdkl,cdij->klij", V, X, 0.0, Xklij, prec);   // cxx:317
+      tctr(1.0, "cdkl,cdij->klij", V, X, 0.0, Xklij, prec);   // cxx:317
     }
     e.record("Xklij2", Xb4.get(), o * o * o * o);
     // ppl = 1: the T1 part of this term comes with the ladder (cxx:326-333)
-    ctr(e, 1.0, "klij,abkl->abij", Xklij, e.ppl ? T2 : X, 1.0, R2, prec);
+    tctr(1.0, "klij,abkl->abij", Xklij, e.ppl ? T2 : X, 1.0, R2, prec);
   }
   if (kept) {
     // added above
@@ -284,7 +294,7 @@ void ccsd_residual(Engine &e, int it, bool initial_doubles, int slice_size, cons
     DBuf dGabb(&e.pool, G * v * v);
     View dGab = V3(dGabb.get(), G, v, v);
     copy(e, dGab, Gab);
-    ctr(e, -1.0, "Gbk,ak->Gab", Gai, T1, 1.0, dGab, prec);  // cxx:397-400
+    tctr(-1.0, "Gbk,ak->Gab", Gai, T1, 1.0, dGab, prec);  // cxx:397-400
     e.record("dGabP", dGabb.get(), G * v * v);
     const int nslices = int((v + slice_size - 1) / slice_size);
     std::vector<DBuf> sl(nslices);
@@ -374,7 +384,7 @@ void ccsd_residual(Engine &e, int it, bool initial_doubles, int slice_size, cons
                         (pl == SISI_BF16X3 || pl == SISI_BF16) && get_b3_backend() == 0 &&
                         2.0 * double(smin * smin) * double(v * v) * double(std::min(G, o * o)) >=
                             kB3MinFlops;
-    if (planes) {
+    if (planes && !zt) {
       const int64_t Kp = (v * v + 31) / 32 * 32;
       const int64_t Mmax = (smax * smax + 255) / 256 * 256;
       std::vector<DBuf> slt(nslices);
@@ -461,7 +471,7 @@ void ccsd_residual(Engine &e, int it, bool initial_doubles, int slice_size, cons
       an.ladder_stack = DBuf(&e.pool, size_t((2 * rows * Kp_k * 2 + 7) / 8));
       stack_hi = reinterpret_cast<uint16_t *>(an.ladder_stack.get());
     }
-    for (int m = 0, pair = 0; m < nslices && !planes; ++m)
+    for (int m = 0, pair = 0; m < nslices && !planes && (keep_planes || !zt); ++m)
       for (int n = m; n < nslices; ++n, ++pair) {  // cxx:418-451
         const int64_t Nx = hi[n] - lo[n], Ny = hi[m] - lo[m];
         View Vxycd = V4(Vxy.get(), Nx, Ny, v, v);
@@ -486,7 +496,8 @@ void ccsd_residual(Engine &e, int it, bool initial_doubles, int slice_size, cons
             b3_freeze_a(e, Vxy.get(), 1, Nx * Ny, int(Nx * Ny), int(v * v), fz);
           }
         }
-        ctr(e, 1.0, "xycd,cdij->xyij", Vxycd, X, 0.0, Rxyij, e.prec_ladder);  // cxx:443
+        tctr(1.0, "xycd,cdij->xyij", Vxycd, X, 0.0, Rxyij, e.prec_ladder);  // cxx:443
+        if (zt) continue;  // the planes only
         // sliceIntoResiduum (ClusterSinglesDoublesAlgorithm.cxx:887-915)
         const int64_t a = lo[n], b = lo[m];
         copy(e, subview(R2, {a, b, 0, 0}, {a + Nx, b + Ny, o, o}), Rxyij, 1.0, 1.0);
@@ -495,27 +506,27 @@ void ccsd_residual(Engine &e, int it, bool initial_doubles, int slice_size, cons
   }
   {
     // T1 equations (cxx:457-492)
-    ctr(e, 1.0, "ac,ci->ai", Kac, T1, 1.0, R1, prec);    // cxx:466
-    ctr(e, -1.0, "ki,ak->ai", Kki, T1, 1.0, R1, prec);   // cxx:467
+    tctr(1.0, "ac,ci->ai", Kac, T1, 1.0, R1, prec);    // cxx:466
+    tctr(-1.0, "ki,ak->ai", Kki, T1, 1.0, R1, prec);   // cxx:467
     DBuf Kckb(&e.pool, v * o), Skib(&e.pool, o * o);
     View Kck = V2(Kckb.get(), v, o);
-    ctr(e, 1.0, "cdkl,dl->ck", U, T1, 0.0, Kck, prec);   // cxx:470-471
+    tctr(1.0, "cdkl,dl->ck", U, T1, 0.0, Kck, prec);   // cxx:470-471
     e.record("Kck", Kckb.get(), v * o);
-    ctr(e, 2.0, "ck,caki->ai", Kck, T2, 1.0, R1, prec);  // cxx:474
-    ctr(e, -1.0, "ck,caik->ai", Kck, T2, 1.0, R1, prec); // cxx:475
-    ctr(e, 1.0, "ck,ci->ki", Kck, T1, 0.0, V2(Skib.get(), o, o), prec);  // cxx:476
+    tctr(2.0, "ck,caki->ai", Kck, T2, 1.0, R1, prec);  // cxx:474
+    tctr(-1.0, "ck,caik->ai", Kck, T2, 1.0, R1, prec); // cxx:475
+    tctr(1.0, "ck,ci->ki", Kck, T1, 0.0, V2(Skib.get(), o, o), prec);  // cxx:476
     e.record("Ski", Skib.get(), o * o);
-    ctr(e, 1.0, "ak,ki->ai", T1, V2(Skib.get(), o, o), 1.0, R1, prec);
-    ctr(e, 2.0, "acik,ck->ai", V, T1, 1.0, R1, prec);      // cxx:477
-    ctr(e, -1.0, "ciak,ck->ai", Vaibj, T1, 1.0, R1, prec); // cxx:478
+    tctr(1.0, "ak,ki->ai", T1, V2(Skib.get(), o, o), 1.0, R1, prec);
+    tctr(2.0, "acik,ck->ai", V, T1, 1.0, R1, prec);      // cxx:477
+    tctr(-1.0, "ciak,ck->ai", Vaibj, T1, 1.0, R1, prec); // cxx:478
     DBuf Ygb(&e.pool, G * v * o);
     View Yg = V3(Ygb.get(), G, v, o);
-    ctr(e, 1.0, "Gdk,cdik->Gci", Gai, X, 0.0, Yg, prec);  // cxx:480-481
-    ctr(e, 2.0, "Gca,Gci->ai", Gab, Yg, 1.0, R1, prec);
-    ctr(e, 1.0, "Gck,cdik->Gdi", Gai, X, 0.0, Yg, prec);  // cxx:484-485
-    ctr(e, -1.0, "Gda,Gdi->ai", Gab, Yg, 1.0, R1, prec);
-    ctr(e, -2.0, "klic,ackl->ai", Vijka, X, 1.0, R1, prec);  // cxx:489
-    ctr(e, 1.0, "lkic,ackl->ai", Vijka, X, 1.0, R1, prec);   // cxx:490
+    tctr(1.0, "Gdk,cdik->Gci", Gai, X, 0.0, Yg, prec);  // cxx:480-481
+    tctr(2.0, "Gca,Gci->ai", Gab, Yg, 1.0, R1, prec);
+    tctr(1.0, "Gck,cdik->Gdi", Gai, X, 0.0, Yg, prec);  // cxx:484-485
+    tctr(-1.0, "Gda,Gdi->ai", Gab, Yg, 1.0, R1, prec);
+    tctr(-2.0, "klic,ackl->ai", Vijka, X, 1.0, R1, prec);  // cxx:489
+    tctr(1.0, "lkic,ackl->ai", Vijka, X, 1.0, R1, prec);   // cxx:490
   }
   e.thaw();
 }
@@ -1328,7 +1339,14 @@ void ccsd_iterate(Engine &e, int n) {
       if (!e.anchor.valid || e.anchor.precision != prec ||
           e.anchor.age >= o.bulk_refine_interval) {
         set_precision(e, prec);
-        ccsd_residual_anchor(e, o.slice_size, e.T1.get(), e.T2.get(), R1.get(), R2.get(), prec);
+        e.zero_amplitudes = e.iteration == 0 && !e.run_initial;
+        try {
+          ccsd_residual_anchor(e, o.slice_size, e.T1.get(), e.T2.get(), R1.get(), R2.get(), prec);
+        } catch (...) {
+          e.zero_amplitudes = false;
+          throw;
+        }
+        e.zero_amplitudes = false;
       } else {
         set_precision(e, o.refine_precision);
         ccsd_residual_delta(e, o.slice_size, e.T1.get(), e.T2.get(), R1.get(), R2.get());

@@ -227,6 +227,7 @@ class Engine {
   // refinement anchor (recorded by an FP64 residual when `recording` is set)
   Anchor anchor;
   bool recording = false;
+  bool zero_amplitudes = false;  // the residual in progress is at T = 0
   void record(const std::string &name, const double *p, size_t n);
 
   // CCSD run state
