@@ -337,9 +337,9 @@ static void set_ksplit(GemmArgs &g, int ksplit, int kq);
 //  - a split pays the launch of the reduction and its partial sums.
 // 500 x 500 x 300: 32 x 32 10.0 us, 64 x 64 16.7, 128 x 128 25.2 (each with
 // its best split); 1500^3: 157, 171, 220; 4096^3: -, 2417, 2141.
-constexpr int kResident[kNumTiles] = {2, 4, 8};
+constexpr int kResident[kNumTiles] = {2, 4, 4};
 constexpr double kTileMfma[2][kNumTiles] = {{4096, 1024, 256}, {2048, 512, 128}};
-constexpr double kTileCycles[2][kNumTiles] = {{4420, 1250, 400}, {2400, 800, 320}};
+constexpr double kTileCycles[2][kNumTiles] = {{4420, 1250, 360}, {2400, 800, 300}};
 constexpr double kChunkLatency = 700.0;
 constexpr double kBlockCycles = 3000.0;   // prologue and epilogue of a workgroup
 constexpr double kReduceCycles = 9000.0;  // launch of the split-K reduction
@@ -352,9 +352,10 @@ struct TilePlan {
 static double tile_cycles(const GemmArgs &g, int precision, int cus, int t, int ks) {
   const int bt = kTiles[t], p = precision == SISI_FP64 ? 0 : 1;
   const int64_t tiles = ((g.M + bt - 1) / bt) * int64_t((g.N + bt - 1) / bt) * g.batch;
-  const int64_t chunks = ((g.K + ks - 1) / ks + kTileK - 1) / kTileK;
+  const int64_t kc = tile_k(bt);  // counted in chunks of 16
+  const int64_t chunks = ((g.K + ks - 1) / ks + kc - 1) / kc * (kc / kTileK);
   const int64_t per_cu = (tiles * ks + cus - 1) / cus;
-  const double lone = kTileMfma[p][t] + kChunkLatency;
+  const double lone = kTileMfma[p][t] + kChunkLatency * kTileK / tile_k(bt);
   auto round = [&](int64_t n) {
     return double(chunks) * std::max(double(n) * kTileCycles[p][t], lone) + kBlockCycles;
   };
@@ -413,7 +414,7 @@ static K4Plan plan_k4(GemmArgs &g, int precision, int cus, bool taped) {
     g.xcd_map = env_map;
     g.group = env_group > 0 ? env_group : 8;
   }
-  const int kq = (precision == SISI_BF16X3) ? 32 : kTileK;
+  int kq = (precision == SISI_BF16X3) ? 32 : kTileK;
   int bm = BM, bn = BN, ksplit = 1;
   if (precision == SISI_BF16X3) {
     // the batched kernel: two rounds of its 128 x 128 tiles, at least eight
@@ -434,6 +435,7 @@ static K4Plan plan_k4(GemmArgs &g, int precision, int cus, bool taped) {
       ksplit = t.ksplit;
     }
     bm = bn = kTiles[p.tile];
+    kq = tile_k(bm);
   }
   g.tiles_m = (g.M + bm - 1) / bm;
   g.tiles_n = (g.N + bn - 1) / bn;

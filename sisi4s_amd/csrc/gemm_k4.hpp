@@ -14,6 +14,11 @@ namespace sisi {
 // and were best at no size by more than 5 %.
 constexpr int kTiles[] = {128, 64, 32};
 constexpr int kNumTiles = 3;
+// k per chunk: a wave of the 32 x 32 tile has four MFMAs per 16 k between two
+// barriers, too few to cover the chain of store, barrier and reads; with 32 k
+// 250^3 takes 8.9 -> 7.6 us, 500^3 14.9 -> 13.0, 777 x 640 x 1531 47 -> 40
+// (FP32: 500^3 12.9 -> 10.2, 810^3 29 -> 22)
+constexpr int tile_k(int tile) { return tile == 32 ? 32 : kTileK; }
 
 // Load mappings: 0: A m-fast, B k-fast; +1: B n-fast; +2: A k-fast.
 void launch_k4_fp64(int tile, int map, const GemmArgs &g, dim3 grid, hipStream_t s);
@@ -43,8 +48,9 @@ __device__ __forceinline__ void gemm_k4_body(const GemmArgs &g, int pid, int ks,
   using AT = typename TileTypes<PREC>::AT;
   constexpr int WM = TBM / WGM, WN = TBN / WGN, TI = WM / 16, TJ = WN / 16;
   static_assert(WGM * WGN == 4 && TI * 16 == WM && TJ * 16 == WN, "four waves, 16-multiples");
-  using LA = TileLds<TBM, AK>;
-  using LB = TileLds<TBN, !BNF>;
+  constexpr int KC = tile_k(TBM);
+  using LA = TileLds<TBM, AK, KC>;
+  using LB = TileLds<TBN, !BNF, KC>;
   __shared__ __attribute__((aligned(16))) LT As[2][LA::kSize];
   __shared__ __attribute__((aligned(16))) LT Bs[2][LB::kSize];
 
@@ -55,11 +61,11 @@ __device__ __forceinline__ void gemm_k4_body(const GemmArgs &g, int pid, int ks,
   const int m0 = tm * TBM, n0 = tn * TBN;
   const int kbeg = ks * g.kchunk;
   const int kend = min(g.K, kbeg + g.kchunk);
-  const int half = (kend - kbeg + kTileK - 1) / kTileK;  // chunks of one plane product
+  const int half = (kend - kbeg + KC - 1) / KC;  // chunks of one plane product
   const int chunks = CPLX ? 2 * half : half;
 
-  TileLoader<LT, TBM, AK> la;
-  TileLoader<LT, TBN, !BNF> lb;
+  TileLoader<LT, TBM, AK, KC> la;
+  TileLoader<LT, TBN, !BNF, KC> lb;
   // second plane product of a complex part: Im A with Im B (Re C) or Re B (Im C)
   double scale = 1.0;  // of the chunk in the registers
   if constexpr (CPLX) {
@@ -79,8 +85,8 @@ __device__ __forceinline__ void gemm_k4_body(const GemmArgs &g, int pid, int ks,
       }
       if (c >= half) c -= half;
     }
-    const int nk = kend - kbeg - c * kTileK;
-    if (nk >= kTileK) {
+    const int nk = kend - kbeg - c * KC;
+    if (nk >= KC) {
       la.load();
       lb.load();
     } else {
@@ -115,7 +121,7 @@ __device__ __forceinline__ void gemm_k4_body(const GemmArgs &g, int pid, int ks,
         if (c + 2 < chunks) load(c + 2);
       }
       if (active)
-        tile_mma<PREC, TI, TJ, LA::kRow, LA::kCol, LB::kRow, LB::kCol>(
+        tile_mma<PREC, TI, TJ, LA::kRow, LA::kCol, LB::kRow, LB::kCol, KC>(
             As[c & 1] + wm * LA::kRow, Bs[c & 1] + wn * LB::kRow, lane, acc);
       __syncthreads();
     }

@@ -20,24 +20,24 @@ typedef float f2 __attribute__((ext_vector_type(2)));
 // two doubles at any element address (odd leading dimensions)
 typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
 
-constexpr int kTileK = 16;  // k per chunk
+constexpr int kTileK = 16;  // k per chunk, where not stated otherwise
 
-// LDS layout of R rows by 16 k: k-fast rows of 18 elements (144 bytes: the 16
-// rows of a fragment read fall on distinct banks) or m-fast rows of R + 4.
+// LDS layout of R rows by KC k: k-fast rows of KC + 2 elements (144 bytes: the
+// 16 rows of a fragment read fall on distinct banks) or m-fast rows of R + 4.
 // Both measure no bank conflicts at 2560^3 (m-fast rows of R + 16 cost four
 // cycles per fragment read).
-template <int R, bool KF>
+template <int R, bool KF, int KC = kTileK>
 struct TileLds {
-  static constexpr int kRow = KF ? 18 : 1;
+  static constexpr int kRow = KF ? KC + 2 : 1;
   static constexpr int kCol = KF ? 1 : R + 4;
-  static constexpr int kSize = KF ? R * 18 : kTileK * (R + 4);
+  static constexpr int kSize = KF ? R * (KC + 2) : KC * (R + 4);
 };
 
-// One operand's tile rows [r0, r0 + R): global loads of a 16-k chunk into
+// One operand's tile rows [r0, r0 + R): global loads of a KC-k chunk into
 // registers, and the store into LDS.  KF: k is the index the threads walk.
-template <typename LT, int R, bool KF>
+template <typename LT, int R, bool KF, int KC = kTileK>
 struct TileLoader {
-  static constexpr int kGran = R * kTileK / 2;  // two-element granules per chunk
+  static constexpr int kGran = R * KC / 2;  // two-element granules per chunk
   static constexpr int kQ = (kGran + 255) / 256;
   static constexpr bool kWhole = kGran % 256 == 0;
   using L2 = typename std::conditional<sizeof(LT) == 8, d2, f2>::type;
@@ -51,8 +51,8 @@ struct TileLoader {
   d2 v[kQ];
 
   static __device__ __forceinline__ void place(int e, int &row, int &k) {
-    row = KF ? e / (kTileK / 2) : 2 * (e % (R / 2));
-    k = KF ? 2 * (e % (kTileK / 2)) : e / (R / 2);
+    row = KF ? e / (KC / 2) : 2 * (e % (R / 2));
+    k = KF ? 2 * (e % (KC / 2)) : e / (R / 2);
   }
 
   __device__ __forceinline__ void init(const double *p, int64_t s_row, int64_t s_k, int r0,
@@ -60,7 +60,7 @@ struct TileLoader {
     sr = s_row;
     sk = s_k;
     base = p + int64_t(r0) * sr + int64_t(k0) * sk;
-    step = kTileK * sk;
+    step = KC * sk;
     last = rlast - r0;
     // 16-byte loads need the walked index at unit stride; along the rows
     // also every row of the tile in range
@@ -94,7 +94,7 @@ struct TileLoader {
     base += step;
   }
 
-  // the last chunk, nk < 16: elements past nk are zero (loaded from a clamped k)
+  // the last chunk, nk < KC: elements past nk are zero (loaded from a clamped k)
   __device__ __forceinline__ void load_tail(int nk) {
 #pragma unroll
     for (int q = 0; q < kQ; ++q)
@@ -132,7 +132,7 @@ struct TileLoader {
         w.x = LT(v[q].x);
         w.y = LT(v[q].y);
         *reinterpret_cast<L2 *>(
-            lds + row * TileLds<R, KF>::kRow + k * TileLds<R, KF>::kCol) = w;
+            lds + row * TileLds<R, KF, KC>::kRow + k * TileLds<R, KF, KC>::kCol) = w;
       }
   }
 };
@@ -149,7 +149,7 @@ struct TileTypes {
 
 // One LDS chunk into a wave's accumulators.  a and b point at the wave's
 // first row of each operand.
-template <int PREC, int TI, int TJ, int AROW, int ACOL, int BROW, int BCOL>
+template <int PREC, int TI, int TJ, int AROW, int ACOL, int BROW, int BCOL, int KC = kTileK>
 __device__ __forceinline__ void tile_mma(const typename TileTypes<PREC>::LT *a,
                                          const typename TileTypes<PREC>::LT *b, int lane,
                                          typename TileTypes<PREC>::AT (&acc)[TI][TJ]) {
@@ -157,7 +157,7 @@ __device__ __forceinline__ void tile_mma(const typename TileTypes<PREC>::LT *a,
   const int l16 = lane & 15, lk = lane >> 4;
   const LT *pa = a + l16 * AROW + lk * ACOL, *pb = b + l16 * BROW + lk * BCOL;
 #pragma unroll
-  for (int kq = 0; kq < kTileK / 4; ++kq) {
+  for (int kq = 0; kq < KC / 4; ++kq) {
     LT av[TI], bv[TJ];
 #pragma unroll
     for (int i = 0; i < TI; ++i) av[i] = pa[i * 16 * AROW + kq * 4 * ACOL];
