@@ -39,7 +39,10 @@ def slice_pairs(Nv, s):
 def ccsd_iteration_flops(No, Nv, NG, s):
     """Algorithmic flops of one CCSD iteration (real arithmetic, 2*M*N*K per
     term): ladder 2 P(s) Nv^2 (NG + No^2), seven O(No^3 Nv^3) ring products,
-    five K=NG products and the O(No^4 Nv^2) hole ladder."""
+    five K=NG products and the O(No^4 Nv^2) hole ladder.  This is the
+    reference's term count, a fixed unit of work: the engine's regrouped rings
+    and kept pair ladder execute fewer, so a rate on it may exceed the peak
+    (the roofline entry counts the launched products)."""
     return (2.0 * slice_pairs(Nv, s) * Nv ** 2 * (NG + No ** 2) + 14.0 * Nv ** 3 * No ** 3
             + 10.0 * NG * Nv ** 2 * No ** 2 + 6.0 * Nv ** 2 * No ** 4)
 

@@ -47,7 +47,7 @@ void set_last_error(const std::string &msg);
 // the first iteration.  Buffers up to kSlabMax are carved out of slabs of
 // growing size (8 to 256 MB): hipMalloc and hipFree cost 50 to 100 us each
 // whatever the size, and a small system's engine holds a few hundred buffers
-// (the batch of 16 systems with No about 10, Nv about 70: 433 -> 270 ms, most
+// (the batch of 16 systems with No about 10, Nv about 70: 433 -> 264 ms, most
 // of it the frees at the end).  Not thread-safe (one engine, one host thread).
 // Device-wide operations (hipDeviceSynchronize, hipFree, stream creation and
 // destruction) are not allowed while another thread captures its stream into

@@ -335,8 +335,8 @@ static void set_ksplit(GemmArgs &g, int ksplit, int kq);
 //    fragment reads; resident workgroups overlap these chains, and then a
 //    tile's chunk costs kTileCycles;
 //  - a split pays the launch of the reduction and its partial sums.
-// 500 x 500 x 300: 32 x 32 10.0 us, 64 x 64 16.7, 128 x 128 25.2 (each with
-// its best split); 1500^3: 157, 171, 220; 4096^3: -, 2417, 2141.
+// 500 x 500 x 300: 32 x 32 9.0 us, 64 x 64 16.7, 128 x 128 25.2 (each with
+// its best split); 1500^3: 150, 171, 220; 4096^3: -, 2417, 2141.
 constexpr int kResident[kNumTiles] = {2, 4, 4};
 constexpr double kTileMfma[2][kNumTiles] = {{4096, 1024, 256}, {2048, 512, 128}};
 constexpr double kTileCycles[2][kNumTiles] = {{4420, 1250, 360}, {2400, 800, 300}};
@@ -368,11 +368,9 @@ static double tile_cycles(const GemmArgs &g, int precision, int cus, int t, int 
 }
 
 static TilePlan choose_tile(const GemmArgs &g, int precision, int cus) {
-  static const char *const env_tile = getenv("SISI_GEMM_TILE");
   TilePlan best;
   double best_c = 1e300;
   for (int t = 0; t < kNumTiles; ++t) {
-    if (env_tile && *env_tile && atoi(env_tile) != t) continue;
     for (int ks : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64, 96, 128, 192, 256}) {
       // at least four chunks per part, and partial sums of at most 2 GB
       if (ks > 1 && (g.K < ks * 4 * kTileK ||
