@@ -415,7 +415,12 @@ void ccsd_solve_lockstep(int nsys, const sisi_dims *dims, const double *const *g
     s.cur_precision = o.precision;
     s.coarse_active = bulk_run && o.coarse_threshold > 0.0;
     // the run starts from T = 0 and its updates keep T2 symmetric (below)
-    if (keep_ladders) e.use_kept_ladder = kept_ladder_build(e);
+    if (keep_ladders) {
+      e.use_kept_ladder = kept_ladder_build(e);
+      // the recorded launches run on `stream`, in buffers that the build's
+      // temporaries may give to them: it ends first (like the integrals)
+      e.sync();
+    }
     if (bulk_run) record_residual(s, 1, o.slice_size, 1, s.res[1], &s.held[1], pool, stream);
     record_residual(s, 0, o.slice_size, 1, s.res[0], &s.held[0], pool, stream);
   }

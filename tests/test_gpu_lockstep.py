@@ -146,3 +146,21 @@ def test_lockstep_64_systems_config():
                                       st["plans"], float(np.max(np.abs(emx - e64)))), flush=True)
     assert all(r["converged"] for r in rmx)
     assert float(np.max(np.abs(emx - e64))) <= 1e-6
+
+
+def test_lockstep_large_last_system():
+    """The pair integrals of a system whose build outlasts the rest of the
+    set-up (about 60 ms, the last in the list) are whole before the recorded
+    residuals read them: energies as from single-system runs."""
+    from sisi4s_amd import engine
+    specs = [(61, 3, 20, 80), (62, 4, 250, 1000)]
+    systems = [engine.generate_system(*sp) for sp in specs]
+    kw = dict(mixer="DiisMixer", max_residua=4, max_iterations=4, level_shift=2.0,
+              amplitudes_convergence=0.0, energy_convergence=0.0)
+    announce("lockstep, large last system")
+    E, reps, _ = engine.ccsd_solve_lockstep(systems, engine.default_opts(**kw))
+    for sp, (g, ei, ea), x in zip(specs, systems, E):
+        with engine.Engine(*sp[1:]) as e:
+            e.set_system(g, ei, ea)
+            ref = e.ccsd_solve(engine.default_opts(**kw))
+        assert abs(x - ref["energy"]) <= 1e-10 * abs(ref["energy"]), (sp, x, ref["energy"])
