@@ -335,6 +335,8 @@ static void set_ksplit(GemmArgs &g, int ksplit, int kq);
 //    fragment reads; resident workgroups overlap these chains, and then a
 //    tile's chunk costs kTileCycles;
 //  - a split pays the launch of the reduction and its partial sums.
+// In FP32 the 128 x 128 tile sums a part in one chain, so it takes at least
+// `least` parts (the smaller tiles sum in two levels, gemm_k4.hpp).
 // 500 x 500 x 300: 32 x 32 9.0 us, 64 x 64 16.7, 128 x 128 25.2 (each with
 // its best split); 1500^3: 150, 171, 220; 4096^3: -, 2417, 2141.
 constexpr int kResident[kNumTiles] = {2, 4, 4};
@@ -367,11 +369,21 @@ static double tile_cycles(const GemmArgs &g, int precision, int cus, int t, int 
   return c;
 }
 
-static TilePlan choose_tile(const GemmArgs &g, int precision, int cus) {
+// Parts of a product's K that fill the device with 128 x 128 tiles: about 1024
+// workgroups of at least eight chunks of kq, 64 parts at most.
+static int filling_parts(const GemmArgs &g, int kq, int cus) {
+  const int64_t tb = ((g.M + BM - 1) / BM) * int64_t((g.N + BN - 1) / BN) * g.batch;
+  if (g.K <= 4 * kq || tb >= 1024) return 1;
+  const int64_t smax = std::min(std::max(1, g.K / (8 * kq)), 64);
+  return round_filling_split(tb, std::min((1024 + tb - 1) / tb, smax), smax, cus);
+}
+
+static TilePlan choose_tile(const GemmArgs &g, int precision, int cus, int least) {
   TilePlan best;
   double best_c = 1e300;
-  for (int t = 0; t < kNumTiles; ++t) {
+  for (int t = g.cplx ? first_tile_z(precision) : 0; t < kNumTiles; ++t) {
     for (int ks : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64, 96, 128, 192, 256}) {
+      if (t == 0 && ks < least) continue;
       // at least four chunks per part, and partial sums of at most 2 GB
       if (ks > 1 && (g.K < ks * 4 * kTileK ||
                      double(ks) * g.M * double(g.N) * g.batch > double(int64_t(1) << 28)))
@@ -415,20 +427,15 @@ static K4Plan plan_k4(GemmArgs &g, int precision, int cus, bool taped) {
   int kq = (precision == SISI_BF16X3) ? 32 : kTileK;
   int bm = BM, bn = BN, ksplit = 1;
   if (precision == SISI_BF16X3) {
-    // the batched kernel: two rounds of its 128 x 128 tiles, at least eight
-    // k-chunks per part
-    const int64_t tb = ((g.M + bm - 1) / bm) * int64_t((g.N + bn - 1) / bn) * g.batch;
-    if (g.K > 4 * kq && tb < 1024) {
-      const int64_t smax = std::min(std::max(1, g.K / (8 * kq)), 64);
-      ksplit = round_filling_split(tb, std::min((1024 + tb - 1) / tb, smax), smax, cus);
-    }
+    ksplit = filling_parts(g, kq, cus);
   } else {
     if (taped) {
       p.tile = kTapeTile;
     } else {
       GemmArgs c = g;  // a complex part is two plane products
       if (g.cplx) c.K = int(std::min<int64_t>(2 * int64_t(g.K), (int64_t(1) << 31) - 1));
-      const TilePlan t = choose_tile(c, precision, cus);
+      const int least = precision == SISI_FP32 ? filling_parts(g, kTileK, cus) : 1;
+      const TilePlan t = choose_tile(c, precision, cus, least);
       p.tile = t.tile;
       ksplit = t.ksplit;
     }

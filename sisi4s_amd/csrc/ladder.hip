@@ -15,6 +15,8 @@ namespace {
 // integrals may take: 124 GB of about 240 free at No = 40, Nv = 400.
 constexpr double kLadderShare = 0.55;
 
+constexpr int64_t kSlab = 4096;  // pairs per FP32 product of the ladder
+
 // Rows of a pair tensor: particle pairs a <= b at b(b+1)/2 + a, then (k, b) at
 // k + No b, then hole pairs k <= l at l(l+1)/2 + k.
 struct Rows {
@@ -386,7 +388,21 @@ void kept_ladder_apply(Engine &e, const double *X, double *Q, double *Qh, double
   g.cn0 = M;
   g.dm0 = g.M;
   g.dn0 = g.N;
-  gemm(e, precision, g);
+  // FP32: sums over the pairs in slabs of about kSlab, added in FP64, as the
+  // 128 tile sums a launch in one FP32 chain and the sliced ladder's chains
+  // are no longer than a slab.  (Recorded products run on the 64 tile, whose
+  // sums have two levels.)
+  const int64_t slabs = e.tape || precision == SISI_FP64
+                            ? 1
+                            : std::max<int64_t>(1, (K + kSlab / 2) / kSlab);
+  const int64_t step = ((K + slabs - 1) / slabs + 15) / 16 * 16;
+  for (int64_t k = 0; k < K; k += step) {
+    g.A = e.ladder.get() + k;
+    g.B = Xp.get() + k;
+    g.K = int(std::min(step, K - k));
+    g.beta = k == 0 ? 0.0 : 1.0;
+    gemm(e, precision, g);
+  }
   const int64_t total = (o * v + N) * N;
   if (tape_pairs(e, OpKind::UnpackHoles, Q, W, Qh, M * N,
                  std::min<int64_t>((total + 255) / 256, 256)))

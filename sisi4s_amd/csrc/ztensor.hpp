@@ -29,7 +29,9 @@ inline ZV zsub(const ZV &v, std::initializer_list<int64_t> lo, std::initializer_
 
 // C = alpha * op(A) op(B) + beta * C, op = conj when the flag is set.  FP64 and
 // FP32 products without a batch label run as one complex product; the
-// split-BF16x3 kernels and batched products take the planes one by one.
+// split-BF16x3 kernels, batched products and FP32 outputs of 1024 tiles of
+// 128 x 128 (which one launch for both planes cannot take in FP32) take the
+// planes one by one.
 inline void zctr(Engine &e, double alpha, const char *spec, const ZV &A, bool ca, const ZV &B, bool cb,
           double beta, const ZV &C, int prec) {
   const double sa = ca ? -1.0 : 1.0, sb = cb ? -1.0 : 1.0;
@@ -42,7 +44,8 @@ inline void zctr(Engine &e, double alpha, const char *spec, const ZV &A, bool ca
     batch = batch || (A.re.len[k] > 1 && ib.find(ia[k]) != std::string::npos &&
                       ic.find(ia[k]) != std::string::npos);
   const int p = prec < 0 ? e.precision : prec;
-  if (!batch && (p == SISI_FP64 || p == SISI_FP32)) {
+  const bool large = p == SISI_FP32 && C.re.size() >= (int64_t(1) << 24);
+  if (!batch && !large && (p == SISI_FP64 || p == SISI_FP32)) {
     const ZPlanes z{A.im.p - A.re.p, B.im.p - B.re.p, C.im.p - C.re.p, sa, sb};
     contract(e, alpha, A.re, ia, B.re, ib, beta, C.re, ic, p, &z);
     return;
