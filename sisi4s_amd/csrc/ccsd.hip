@@ -1279,6 +1279,7 @@ void ccsd_begin(Engine &e, const sisi_ccsd_opts &opts, const double *T1h, const 
   e.T1 = DBuf(&e.pool, e.n1());
   e.T2 = DBuf(&e.pool, e.n2());
   e.run_initial = (T2h != nullptr);
+  e.zero_start = T1h == nullptr && T2h == nullptr;
   if (T1h) e.upload_t(e.T1, T1h, e.n1());
   else zero(e, e.T1.get(), int64_t(e.n1()));
   if (T2h) e.upload_t(e.T2, T2h, e.n2());
@@ -1339,7 +1340,7 @@ void ccsd_iterate(Engine &e, int n) {
       if (!e.anchor.valid || e.anchor.precision != prec ||
           e.anchor.age >= o.bulk_refine_interval) {
         set_precision(e, prec);
-        e.zero_amplitudes = e.iteration == 0 && !e.run_initial;
+        e.zero_amplitudes = e.iteration == 0 && e.zero_start;
         try {
           ccsd_residual_anchor(e, o.slice_size, e.T1.get(), e.T2.get(), R1.get(), R2.get(), prec);
         } catch (...) {

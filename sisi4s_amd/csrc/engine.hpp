@@ -233,7 +233,8 @@ class Engine {
   // CCSD run state
   sisi_ccsd_opts opts{};
   bool run_active = false;
-  bool run_initial = false;
+  bool run_initial = false;  // given doubles
+  bool zero_start = false;   // neither singles nor doubles given
   int iteration = 0;
   int fp64_iterations = 0;
   int cur_precision = SISI_FP64;
