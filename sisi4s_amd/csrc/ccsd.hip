@@ -1207,6 +1207,13 @@ bool graph_residual(Engine &e, int slice, const double *T1, const double *T2, do
   return true;
 }
 
+// Whether every residual as the engine stands now keeps T_abij = T_baji up to
+// rounding, whatever the vertex; uploaded classes could break that.
+bool symmetric_residual(const Engine &e) {
+  return !e.cplx && e.formulation == SISI_FORMULATION_VERTEX && e.NR == 0 && e.ppl &&
+         e.given_integrals == 0;
+}
+
 // Residual of a plain iteration.  FP64 and FP32 iterations of a symmetric run
 // contract the ladder with the kept pair integrals when at least one more
 // iteration can use them (building them costs about what one sliced ladder
@@ -1223,10 +1230,7 @@ void plain_residual(Engine &e, int prec, double *R1, double *R2) {
       return;
     ccsd_residual(e, e.iteration, e.run_initial, o.slice_size, e.T1.get(), e.T2.get(), R1, R2);
   };
-  // what the run was begun with may have been changed between its iterations
-  const bool same = e.ppl && e.NR == 0 && e.formulation == SISI_FORMULATION_VERTEX && !e.cplx &&
-                    e.given_integrals == 0;
-  if (!mp2 && e.symmetric_run && same && !e.kept_ladder_failed &&
+  if (!mp2 && e.symmetric_run && !e.kept_ladder_failed &&
       (prec == SISI_FP64 || prec == SISI_FP32) &&
       (e.ladder.get() || o.max_iterations - e.iteration >= 2)) {
     if (kept_ladder_build(e)) {
@@ -1302,10 +1306,7 @@ void ccsd_begin(Engine &e, const sisi_ccsd_opts &opts, const double *T1h, const 
   e.anchor = Anchor();
   e.ladder.reset();
   e.kept_ladder_failed = false;
-  // every residual of such a run is symmetric (T_abij = T_baji) up to
-  // rounding, whatever the vertex; uploaded classes could break that
-  e.symmetric_run = !e.cplx && e.formulation == SISI_FORMULATION_VERTEX && e.NR == 0 &&
-                    e.ppl && e.given_integrals == 0 && e.Gab.get() &&
+  e.symmetric_run = symmetric_residual(e) && e.Gab.get() &&
                     (T2h == nullptr || doubles_symmetric(e, e.T2.get()));
   if (opts.mixer == SISI_MIXER_DIIS) {
     const int N = opts.max_residua;
@@ -1324,6 +1325,9 @@ void ccsd_iterate(Engine &e, int n) {
   SISI_REQUIRE(e.run_active, SISI_ERR_STATE, "ccsd: no run (call begin first)");
   const sisi_ccsd_opts &o = e.opts;
   for (int step = 0; step < n && !e.converged && e.iteration < o.max_iterations; ++step) {
+    // what the run was begun with may have been changed since: from then on
+    // its doubles are not projected, and the kept ladder cannot read them
+    if (!symmetric_residual(e)) e.symmetric_run = false;
     // precision schedule: coarse precision until |dT|/|T| <= coarse_threshold
     // (if set), bulk precision until |dT|/|T| <= switch_threshold, FP64
     // afterwards (and FP64 throughout for the plain path)
