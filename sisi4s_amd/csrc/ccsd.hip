@@ -1390,9 +1390,6 @@ void ccsd_iterate(Engine &e, int n) {
       s.d1 = std::move(d1);
       s.d2 = std::move(d2);
       // overlaps of the new change with every slot's, read back together
-      SISI_REQUIRE(N <= Engine::kHostScalars - Engine::kDotScalars - 1, SISI_ERR_INVALID,
-                   "maxResidua too large");
-      double *h = e.host_scalars() + Engine::kDotScalars;
       std::vector<int> filled;
       std::vector<const double *> vs, vd;
       for (int i = 0; i < N; ++i) {
@@ -1401,7 +1398,9 @@ void ccsd_iterate(Engine &e, int n) {
         vs.push_back(e.diis[i].d1.get());
         vd.push_back(e.diis[i].d2.get());
       }
-      overlaps_async(e, int(filled.size()), vs.data(), vd.data(), s.d1.get(), s.d2.get(), h);
+      const size_t nf = filled.size();
+      double *h = e.host_scalars(nf + 1) + Engine::kDotScalars;
+      overlaps_async(e, int(nf), vs.data(), vd.data(), s.d1.get(), s.d2.get(), h);
       e.sync();
       double dd = 0.0;  // |dT|^2 of this iteration, for the test below
       for (size_t k = 0; k < filled.size(); ++k) {
@@ -1428,12 +1427,12 @@ void ccsd_iterate(Engine &e, int n) {
         vs.push_back(e.diis[i].t1.get());
         vd.push_back(e.diis[i].t2.get());
       }
-      combine_async(e, int(w.size()), w.data(), vs.data(), vd.data(), n1.get(), n2.get(), h + N);
+      combine_async(e, int(w.size()), w.data(), vs.data(), vd.data(), n1.get(), n2.get(), h + nf);
       e.diis_next = (e.diis_next + 1) % N;
       e.T1 = std::move(n1);
       e.T2 = std::move(n2);
       delta_dd = dd;
-      delta_tt = h + N;  // read with the energy
+      delta_tt = h + nf;  // read with the energy
     } else {
       // LinearMixer::append (LinearMixer.cxx:30-44)
       if (e.lin_have) {
@@ -1448,7 +1447,7 @@ void ccsd_iterate(Engine &e, int n) {
       copy(e, V1(n2.get(), int64_t(e.n2())), V1(e.lin2.get(), int64_t(e.n2())));
       e.T1 = std::move(n1);
       e.T2 = std::move(n2);
-      double *h = e.host_scalars() + Engine::kDotScalars;
+      double *h = e.host_scalars(2) + Engine::kDotScalars;
       const double *x1 = d1.get(), *x2 = d2.get(), *y1 = e.T1.get(), *y2 = e.T2.get();
       overlaps_async(e, 1, &x1, &x2, x1, x2, h);
       overlaps_async(e, 1, &y1, &y2, y1, y2, h + 1);

@@ -193,11 +193,17 @@ void Engine::download_t(double *dst, const DBuf &src, size_t n) {
   }
 }
 
-double *Engine::host_scalars() {
-  if (!scalars_) {
+double *Engine::host_scalars(size_t more) {
+  if (scalars_n_ < kDotScalars + more) {
     std::lock_guard<std::recursive_mutex> lock(device_wide_mutex());
-    SISI_HIP(hipHostMalloc(reinterpret_cast<void **>(&scalars_), kHostScalars * sizeof(double),
+    sync();  // kernels that write to the present ones
+    if (scalars_) (void)hipHostFree(scalars_);
+    scalars_ = nullptr;
+    scalars_n_ = 0;
+    const size_t n = kDotScalars + std::max<size_t>(more, 64);
+    SISI_HIP(hipHostMalloc(reinterpret_cast<void **>(&scalars_), n * sizeof(double),
                            hipHostMallocDefault));
+    scalars_n_ = n;
   }
   return scalars_;
 }

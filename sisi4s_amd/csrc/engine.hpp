@@ -275,10 +275,12 @@ class Engine {
   void sync();
   // Pinned host memory that reduction kernels write their results to
   // directly (no copy; read them after sync()).  The first kDotScalars are
-  // the single reductions', the rest the mixer's.
-  static constexpr int kHostScalars = 4096, kDotScalars = 8;
-  double *host_scalars();
+  // the single reductions', `more` behind them the mixer's (asking for more
+  // than there are waits for the stream and moves them).
+  static constexpr size_t kDotScalars = 8;
+  double *host_scalars(size_t more = 0);
   double *scalars_ = nullptr;
+  size_t scalars_n_ = 0;
   // doubles per singles / doubles amplitude tensor (both planes in complex
   // mode) and elements per plane
   size_t n1() const { return n1e() * (cplx ? 2 : 1); }

@@ -71,3 +71,19 @@ def test_integrals_replaced_between_iterations():
             assert np.abs(T1 - O1).max() <= 1e-12 * np.abs(O1).max()
             assert np.abs(T2 - O2).max() <= 1e-12 * np.abs(O2).max()
             assert np.abs(T2 - T2.transpose(1, 0, 3, 2)).max() > 1e-4
+
+
+def test_any_number_of_residua():
+    """maxResidua above what a run can fill is no bound."""
+    from oracle import ccsd
+    from sisi4s_amd import engine
+    g, ei, ea, _ = system()
+    kw = dict(mixer="DiisMixer", max_iterations=5, level_shift=1.5, energy_convergence=0.0,
+              amplitudes_convergence=1e-12)
+    announce("maxResidua 4500")
+    with engine.Engine(*SIZE) as e:
+        e.set_system(g, ei, ea)
+        e.ccsd_solve(engine.default_opts(max_residua=4500, **kw))
+        E = e.energies()
+    ref = ccsd.solve(g, ei, ea, max_residua=6, **kw)
+    assert np.abs(E - np.array(ref["energies"])).max() <= 1e-11 * abs(ref["energy"])
