@@ -134,11 +134,15 @@ class Pool {
       }
     }
   }
-  // Bytes held in the free lists (device memory the pool can hand out
-  // again, or give back with trim()).
+  // Device memory that trim() gives back: the free lists, of slabs those none
+  // of whose buffers is in use.
   size_t cached_bytes() const {
     size_t b = 0;
-    for (const auto &kv : free_) b += kv.first * kv.second.size();
+    for (const auto &kv : free_)
+      for (void *p : kv.second)
+        if (!slab_of_.count(p)) b += kv.first;
+    for (const auto &s : slabs_)
+      if (s.base && s.held == 0) b += s.size;
     return b;
   }
   void trim() {
@@ -190,12 +194,13 @@ class Pool {
     size_t size = 0, used = 0;
     int held = 0;  // its buffers outside the free lists
   };
-  // A buffer from the newest slab, or from a new one; null when it is too
-  // large or no slab can be had.
+  // A buffer from the first slab with room, or from a new one; null when it
+  // is too large or no slab can be had.
   void *carve(size_t bytes) {
     if (bytes > kSlabMax) return nullptr;
-    if (slabs_.empty() || !slabs_.back().base ||
-        slabs_.back().size - slabs_.back().used < bytes) {
+    size_t i = 0;
+    while (i < slabs_.size() && (!slabs_[i].base || slabs_[i].size - slabs_[i].used < bytes)) ++i;
+    if (i == slabs_.size()) {
       Slab s;
       s.size = std::max(next_slab_, 2 * bytes);
       void *p = nullptr;
@@ -207,10 +212,10 @@ class Pool {
       slabs_.push_back(s);
       next_slab_ = std::min(2 * next_slab_, kSlabLast);
     }
-    Slab &s = slabs_.back();
+    Slab &s = slabs_[i];
     void *p = s.base + s.used;
     s.used += bytes;
-    slab_of_[p] = slabs_.size() - 1;
+    slab_of_[p] = i;
     hold(p, 1);
     return p;
   }
