@@ -300,6 +300,16 @@ struct System {
   double prev_energy = 0.0, energy = 0.0, direct = 0.0, exchange = 0.0, delta = 1.0;
   int status = SISI_OK;
   std::string error;
+  // the recorded residuals read the pair integrals for as long as there are any
+  bool ladder_in_use = false;
+  void use_ladder() {
+    e->pool.begin_use();
+    ladder_in_use = true;
+  }
+  System() = default;
+  ~System() {
+    if (ladder_in_use) e->pool.end_use();
+  }
 };
 
 constexpr int kOutSlots = 64;  // doubles of reduction results per system
@@ -416,6 +426,7 @@ void ccsd_solve_lockstep(int nsys, const sisi_dims *dims, const double *const *g
     s.coarse_active = bulk_run && o.coarse_threshold > 0.0;
     // the run starts from T = 0 and its updates keep T2 symmetric (below)
     if (keep_ladders) {
+      s.use_ladder();
       e.use_kept_ladder = kept_ladder_build(e);
       // the recorded launches run on `stream`, in buffers that the build's
       // temporaries may give to them: it ends first (like the integrals)

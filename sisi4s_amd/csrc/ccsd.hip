@@ -1214,11 +1214,23 @@ bool symmetric_residual(const Engine &e) {
          e.given_integrals == 0;
 }
 
+// The pair integrals are in use by an iteration: no other allocation takes
+// their memory, which any may do between the iterations.
+struct LadderUse {
+  Engine &e;
+  explicit LadderUse(Engine &e_) : e(e_) { e.pool.begin_use(); }
+  ~LadderUse() {
+    e.use_kept_ladder = false;
+    e.pool.end_use();
+  }
+};
+
 // Residual of a plain iteration.  FP64 and FP32 iterations of a symmetric run
 // contract the ladder with the kept pair integrals when at least one more
 // iteration can use them (building them costs about what one sliced ladder
 // does) and they fit; everything else, and a run that finds no memory on the
-// way, takes the sliced ladder.
+// way or whose pair integrals were taken by another allocation, takes the
+// sliced ladder.
 void plain_residual(Engine &e, int prec, double *R1, double *R2) {
   const sisi_ccsd_opts &o = e.opts;
   const bool mp2 = e.iteration == 0 && !e.run_initial;
@@ -1232,17 +1244,17 @@ void plain_residual(Engine &e, int prec, double *R1, double *R2) {
   };
   if (!mp2 && e.symmetric_run && !e.kept_ladder_failed &&
       (prec == SISI_FP64 || prec == SISI_FP32) &&
-      (e.ladder.get() || o.max_iterations - e.iteration >= 2)) {
-    if (kept_ladder_build(e)) {
-      e.use_kept_ladder = true;
-      try {
-        evaluate();
-        e.use_kept_ladder = false;
-        return;
-      } catch (const Error &err) {
-        e.use_kept_ladder = false;
-        e.thaw();
-        if (err.code != SISI_ERR_ALLOC) throw;
+      (e.ladder || o.max_iterations - e.iteration >= 2)) {
+    {
+      LadderUse use(e);
+      if (!e.pool.block_lost() && kept_ladder_build(e)) {
+        e.use_kept_ladder = true;
+        try {
+          return evaluate();
+        } catch (const Error &err) {
+          e.thaw();
+          if (err.code != SISI_ERR_ALLOC) throw;
+        }
       }
     }
     e.drop_residual_graph();  // and the pair integrals
@@ -1304,7 +1316,6 @@ void ccsd_begin(Engine &e, const sisi_ccsd_opts &opts, const double *T1h, const 
   e.lin1.reset();
   e.lin2.reset();
   e.anchor = Anchor();
-  e.ladder.reset();
   e.kept_ladder_failed = false;
   e.symmetric_run = symmetric_residual(e) && e.Gab.get() &&
                     (T2h == nullptr || doubles_symmetric(e, e.T2.get()));
@@ -1509,8 +1520,8 @@ void ccsd_iterate(Engine &e, int n) {
     e.prev_energy = E;
     e.prev_energy_imag = Ei;
   }
-  // a run that is over gives the pair integrals' memory back to the pool
-  if (e.converged || e.iteration >= o.max_iterations) e.ladder.reset();
+  // a run that is over no longer needs the pair integrals
+  if (e.converged || e.iteration >= o.max_iterations) e.drop_ladder();
 }
 
 void fill_report(const Engine &e, sisi_ccsd_report *r) {

@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
+#include <chrono>
 #include <cstdint>
 #include <cstdio>
 #include <map>
@@ -12,6 +14,7 @@
 #include <set>
 #include <stdexcept>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/sisi_engine.h"
@@ -57,9 +60,33 @@ inline std::recursive_mutex &device_wide_mutex() {
   return m;
 }
 
+//
+// A pool also holds at most one block: a large buffer whose contents its owner
+// can do without (the pair integrals of the ladder, 124 GB at No = 40, Nv =
+// 400).  It is there for whoever needs memory.  While it is not lent, the
+// pool's own buffers are carved out of it once hipMalloc fails; and an
+// allocation that would fail takes the block of its own pool or of another
+// pool of the process, lent or not, back to the device (block_lost() then
+// tells the owner), except while the owner has work in hand that reads it
+// (begin_use() to end_use()).  Carving comes before freeing since pages that
+// were freed are wiped at about 33 GB/s before they can be had again: a mixed
+// run after an FP64 run at that size waited 3.1 s for them.
 class Pool {
  public:
-  ~Pool() { release_all(); }
+  Pool() {
+    std::lock_guard<std::mutex> lock(registry_mutex());
+    registry().push_back(this);
+  }
+  Pool(const Pool &) = delete;
+  Pool &operator=(const Pool &) = delete;
+  ~Pool() {
+    {
+      std::lock_guard<std::mutex> lock(registry_mutex());
+      auto &r = registry();
+      r.erase(std::find(r.begin(), r.end(), this));
+    }
+    release_all();
+  }
   void *get(size_t bytes) {
     if (bytes == 0) bytes = 8;
     bytes = (bytes + 255) & ~size_t(255);
@@ -73,21 +100,65 @@ class Pool {
       return p;
     }
     if (void *p = carve(bytes)) return handed_out(p, bytes);
-    void *p = nullptr;
-    hipError_t err = hipMalloc(&p, bytes);
-    if (err != hipSuccess) {
-      (void)hipGetLastError();
-      // Drop cached buffers and retry once.
+    void *p = device_malloc(bytes);
+    if (!p) p = carve_block(bytes);
+    if (!p) {
+      // Drop cached buffers and retry, then take blocks.
       trim();
-      err = hipMalloc(&p, bytes);
-      if (err != hipSuccess) {
-        (void)hipGetLastError();
-        throw Error(SISI_ERR_ALLOC, "device allocation of " +
-                                        std::to_string(bytes) + " bytes failed");
+      p = device_malloc(bytes);
+      int waits = 0;
+      while (!p) {
+        bool busy = false;  // a block in use, which may soon be had
+        if (!reclaim(busy)) {
+          if (!busy || ++waits > kWaits)
+            throw Error(SISI_ERR_ALLOC, "device allocation of " +
+                                            std::to_string(bytes) + " bytes failed");
+          std::this_thread::sleep_for(std::chrono::milliseconds(20));
+        }
+        p = device_malloc(bytes);
       }
     }
     return handed_out(p, bytes);
   }
+  // The block, of `bytes` bytes: the one kept from an earlier use or a new
+  // one; null when it cannot be had.
+  void *take_block(size_t bytes) {
+    {
+      std::lock_guard<std::mutex> lock(block_m_);
+      if (block_.base && (block_.lent || block_.held > 0)) return nullptr;
+      if (block_.base && block_.size >= bytes) {
+        block_.lent = true;
+        return block_.base;
+      }
+    }
+    free_idle_block();  // too small
+    void *p = device_malloc(bytes);
+    if (!p) {
+      trim();
+      p = device_malloc(bytes);
+    }
+    if (!p) return nullptr;
+    std::lock_guard<std::mutex> lock(block_m_);
+    block_ = Block();
+    block_.base = static_cast<char *>(p);
+    block_.size = bytes;
+    block_.lent = true;
+    (void)hipGetDevice(&block_.device);
+    return p;
+  }
+  // Its owner no longer needs what is in it.
+  void return_block() {
+    std::lock_guard<std::mutex> lock(block_m_);
+    block_.lent = false;
+    lost_ = false;
+  }
+  // A lent block was taken by another allocation.
+  bool block_lost() const { return lost_; }
+  // The owner issues work that reads or writes the block.
+  void begin_use() {
+    while (busy_.exchange(true)) std::this_thread::yield();  // a reclaim frees it
+  }
+  void end_use() { busy_ = false; }
   void put(void *p) {
     if (!p) return;
     auto it = size_.find(p);
@@ -122,6 +193,8 @@ class Pool {
         }
     }
     captured_.clear();
+    std::lock_guard<std::mutex> lock(block_m_);
+    if (block_.held == 0) make_block_whole();
     return held;
   }
   void release(const std::vector<void *> &held) {
@@ -135,14 +208,16 @@ class Pool {
     }
   }
   // Device memory that trim() gives back: the free lists, of slabs those none
-  // of whose buffers is in use.
+  // of whose buffers is in use, and so the block when it is not lent.
   size_t cached_bytes() const {
     size_t b = 0;
     for (const auto &kv : free_)
       for (void *p : kv.second)
-        if (!slab_of_.count(p)) b += kv.first;
+        if (!slab_of_.count(p) && !in_block_.count(p)) b += kv.first;
     for (const auto &s : slabs_)
       if (s.base && s.held == 0) b += s.size;
+    std::lock_guard<std::mutex> lock(block_m_);
+    if (block_.base && !block_.lent && block_.held == 0) b += block_.size;
     return b;
   }
   void trim() {
@@ -153,7 +228,7 @@ class Pool {
       std::vector<void *> keep;
       for (void *p : kv.second) {
         auto it = slab_of_.find(p);
-        if (it != slab_of_.end() && slabs_[it->second].held > 0) {
+        if ((it != slab_of_.end() && slabs_[it->second].held > 0) || in_block_.count(p)) {
           keep.push_back(p);
           continue;
         }
@@ -168,14 +243,21 @@ class Pool {
         (void)hipFree(s.base);
         s = Slab();
       }
+    free_idle_block();
   }
   void release_all() {
     std::lock_guard<std::recursive_mutex> lock(device_wide_mutex());
     (void)hipDeviceSynchronize();
     for (auto &kv : size_)
-      if (!slab_of_.count(kv.first)) (void)hipFree(kv.first);
+      if (!slab_of_.count(kv.first) && !in_block_.count(kv.first)) (void)hipFree(kv.first);
     for (auto &s : slabs_)
       if (s.base) (void)hipFree(s.base);
+    {
+      std::lock_guard<std::mutex> block_lock(block_m_);
+      if (block_.base) (void)hipFree(block_.base);
+      block_ = Block();
+    }
+    in_block_.clear();
     slabs_.clear();
     slab_of_.clear();
     next_slab_ = kSlabFirst;
@@ -222,6 +304,95 @@ class Pool {
   void hold(void *p, int d) {
     auto it = slab_of_.find(p);
     if (it != slab_of_.end()) slabs_[it->second].held += d;
+    if (!in_block_.count(p)) return;
+    std::lock_guard<std::mutex> lock(block_m_);
+    block_.held += d;
+    if (block_.held == 0 && !capturing_) make_block_whole();
+  }
+  // With the last of its buffers back (during a capture not before its end:
+  // the captured launches may use them) the block is one again.
+  void make_block_whole() {
+    for (void *q : in_block_) {
+      auto &fl = free_[size_[q]];
+      fl.erase(std::remove(fl.begin(), fl.end(), q), fl.end());
+      size_.erase(q);
+    }
+    in_block_.clear();
+    block_.used = 0;
+  }
+  static void *device_malloc(size_t bytes) {
+    void *p = nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  struct Block {
+    char *base = nullptr;
+    size_t size = 0, used = 0;
+    int held = 0, device = 0;
+    bool lent = false;
+  };
+  static constexpr int kWaits = 50;  // of 20 ms, for blocks in use
+  static std::mutex &registry_mutex() {
+    static std::mutex m;
+    return m;
+  }
+  static std::vector<Pool *> &registry() {
+    static auto *r = new std::vector<Pool *>;  // outlives every pool
+    return *r;
+  }
+  void *carve_block(size_t bytes) {
+    std::lock_guard<std::mutex> lock(block_m_);
+    if (!block_.base || block_.lent || block_.size - block_.used < bytes) return nullptr;
+    void *p = block_.base + block_.used;
+    block_.used += bytes;
+    ++block_.held;
+    in_block_.insert(p);
+    return p;
+  }
+  void free_idle_block() {
+    std::lock_guard<std::recursive_mutex> device_lock(device_wide_mutex());
+    std::lock_guard<std::mutex> lock(block_m_);
+    if (!block_.base || block_.lent || block_.held > 0) return;
+    (void)hipDeviceSynchronize();
+    (void)hipFree(block_.base);
+    block_ = Block();
+  }
+  // Frees the block if nothing is carved out of it; by a thread that holds
+  // busy_ (so that its owner is not using it) and the device-wide lock.
+  bool surrender(int device) {
+    std::lock_guard<std::mutex> lock(block_m_);
+    if (!block_.base || block_.held > 0 || block_.device != device) return false;
+    (void)hipDeviceSynchronize();
+    (void)hipFree(block_.base);
+    lost_ = block_.lent;
+    block_ = Block();
+    return true;
+  }
+  // One block of this pool or another is freed.  busy: another's is in use.
+  bool reclaim(bool &busy) {
+    if (capturing_) return false;
+    int device = 0;
+    (void)hipGetDevice(&device);
+    std::lock_guard<std::recursive_mutex> device_lock(device_wide_mutex());
+    std::lock_guard<std::mutex> lock(registry_mutex());
+    auto attempt = [&](Pool *q) {
+      if (q->busy_.exchange(true)) {
+        busy = busy || (q != this && q->block_in_use(device));
+        return false;
+      }
+      const bool freed = q->surrender(device);
+      q->busy_ = false;
+      return freed;
+    };
+    if (attempt(this)) return true;
+    for (Pool *q : registry())
+      if (q != this && attempt(q)) return true;
+    return false;
+  }
+  bool block_in_use(int device) {
+    std::lock_guard<std::mutex> lock(block_m_);
+    return block_.base && block_.lent && block_.device == device;
   }
   void *handed_out(void *p, size_t bytes) {
     size_[p] = bytes;
@@ -229,6 +400,11 @@ class Pool {
     if (capturing_) captured_.push_back(p);
     return p;
   }
+  mutable std::mutex block_m_;     // block_: another pool may take it
+  Block block_;
+  std::set<void *> in_block_;      // buffers carved out of it
+  std::atomic<bool> busy_{false};  // in use by its owner, or about to be freed
+  std::atomic<bool> lost_{false};
   std::vector<Slab> slabs_;
   std::map<void *, size_t> slab_of_;
   size_t next_slab_ = kSlabFirst;

@@ -106,7 +106,7 @@ void Engine::drop_residual_graph(bool keep_ladder) {
     rgraph.exec = nullptr;
   }
   // the pair integrals belong to the vertex and run the graph was made for
-  if (!keep_ladder) ladder.reset();
+  if (!keep_ladder) drop_ladder();
   pool.release(rgraph.held);
   rgraph.held.clear();
   rgraph.key.clear();
@@ -114,6 +114,11 @@ void Engine::drop_residual_graph(bool keep_ladder) {
   rgraph.T2.reset();
   rgraph.R1.reset();
   rgraph.R2.reset();
+}
+
+void Engine::drop_ladder() {
+  if (ladder) pool.return_block();
+  ladder = nullptr;
 }
 
 Engine::~Engine() {
@@ -125,7 +130,6 @@ Engine::~Engine() {
   // device buffers return to the pool before it is released
   T1.reset();
   T2.reset();
-  ladder.reset();
   anchor = Anchor();
   diis.clear();
   lin1.reset();

@@ -254,7 +254,8 @@ class Engine {
   // with pair integrals kept for the run (ladder.hpp); use_kept_ladder is set
   // around such a residual
   bool symmetric_run = false, use_kept_ladder = false, kept_ladder_failed = false;
-  DBuf ladder;
+  double *ladder = nullptr;  // in the pool's block
+  void drop_ladder();
   std::vector<double> energies;
   // DIIS ring (DiisMixer.cxx:48-180)
   std::vector<DiisSlot> diis;

@@ -288,7 +288,7 @@ double kept_ladder_bytes(int64_t No, int64_t Nv) {
 }
 
 bool kept_ladder_build(Engine &e) {
-  if (e.ladder.get()) return true;
+  if (e.ladder) return true;
   const int64_t o = e.No, v = e.Nv, G = e.NG, P = o + v;
   const Rows rows{v, o};
   const int64_t K = rows.pairs(), M = rows.count();
@@ -303,15 +303,17 @@ bool kept_ladder_build(Engine &e) {
   const double room = kLadderShare * (double(free_b) + double(e.pool.cached_bytes()));
   if (bytes + 8.0 * double(v * v * P * nb + G * v * P) > room || M >= (int64_t(1) << 31))
     return false;
+  double *out = static_cast<double *>(e.pool.take_block(16 * size_t(M) * size_t(K)));
+  if (!out) return false;
+  e.ladder = out;
   try {
     // Gt[G, c, p]: Gamma_pc with c next to G, p over the holes, then the particles
-    DBuf Gt(&e.pool, size_t(G * v * P)), tmp(&e.pool, size_t(v * v * P * nb)),
-        out(&e.pool, size_t(2 * M * K));
+    DBuf Gt(&e.pool, size_t(G * v * P)), tmp(&e.pool, size_t(v * v * P * nb));
     copy(e, dense(Gt.get(), {G, v, o}), dense(e.Gai.get(), {G, v, o}));
     sum(e, 1.0, dense(e.Gab.get(), {G, v, v}), "Gac", 0.0,
         dense(Gt.get() + G * v * o, {G, v, v}), "Gca");
     PackArgs a{};
-    a.out = out.get();
+    a.out = out;
     a.plane = M * K;
     a.v = int(v);
     a.o = int(o);
@@ -348,8 +350,8 @@ bool kept_ladder_build(Engine &e) {
     a.np = int(o);
     a.b0 = 0;
     pack_pairs(e, a, o * o);
-    e.ladder = std::move(out);
   } catch (const Error &err) {
+    e.drop_ladder();
     if (err.code != SISI_ERR_ALLOC) throw;
     return false;
   }
@@ -366,13 +368,13 @@ void kept_ladder_apply(Engine &e, const double *X, double *Q, double *Qh, double
   const int64_t o = e.No, v = e.Nv;
   const Rows rows{v, o};
   const int64_t K = rows.pairs(), M = rows.count(), N = rows.opairs();
-  SISI_REQUIRE(e.ladder.get(), SISI_ERR_STATE, "ladder: pair integrals not built");
+  SISI_REQUIRE(e.ladder, SISI_ERR_STATE, "ladder: pair integrals not built");
   DBuf Xp(&e.pool, size_t(2 * N * K));
   const int64_t t32 = (v + 31) / 32;
   if (!tape_pairs(e, OpKind::PackPairs, X, nullptr, Xp.get(), N * K, t32 * t32 * o * o))
     pack_pairs(e, amplitude_pack(X, Xp.get(), N * K, int(v), int(o)), o * o);
   GemmArgs g;  // both combinations as one batch
-  g.A = e.ladder.get();
+  g.A = e.ladder;
   g.B = Xp.get();
   g.C = Q;
   g.sam = g.sbn = K;
@@ -397,7 +399,7 @@ void kept_ladder_apply(Engine &e, const double *X, double *Q, double *Qh, double
                             : std::max<int64_t>(1, (K + kSlab / 2) / kSlab);
   const int64_t step = ((K + slabs - 1) / slabs + 15) / 16 * 16;
   for (int64_t k = 0; k < K; k += step) {
-    g.A = e.ladder.get() + k;
+    g.A = e.ladder + k;
     g.B = Xp.get() + k;
     g.K = int(std::min(step, K - k));
     g.beta = k == 0 ? 0.0 : 1.0;

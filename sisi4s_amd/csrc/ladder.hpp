@@ -20,9 +20,10 @@ namespace sisi {
 // Whether T2 (device) equals its transpose T_baji bit by bit.
 bool doubles_symmetric(Engine &e, const double *T2);
 
-// Build the pair integrals if the engine has none; false when they do not
-// fit (more than kLadderShare of the memory that is free or cached in the
-// pool, or an allocation fails).
+// Build the pair integrals (in the pool's block) if the engine has none; false
+// when they do not fit (more than kLadderShare of the memory that is free or
+// cached in the pool, or an allocation fails).  Between begin_use() and
+// end_use() of the pool.
 bool kept_ladder_build(Engine &e);
 // Device memory of an engine's pair integrals.
 double kept_ladder_bytes(int64_t No, int64_t Nv);

@@ -93,12 +93,187 @@ static int slab_tails_are_used() {
   return 0;
 }
 
+static bool fails(Pool &pool, size_t bytes) {
+  try {
+    pool.get(bytes);
+  } catch (const sisi::Error &e) {
+    return e.code == SISI_ERR_ALLOC;
+  }
+  return false;
+}
+
+// The block is kept for the next use; a larger one replaces it.
+static int block_is_kept() {
+  device_size = 1000 * MB;
+  Pool pool;
+  void *a = pool.take_block(600 * MB);
+  CHECK(a && !pool.take_block(1 * MB));
+  pool.return_block();
+  CHECK(pool.cached_bytes() == 600 * MB);
+  CHECK(pool.take_block(500 * MB) == a && frees == 0);
+  pool.return_block();
+  CHECK(pool.take_block(700 * MB) && device_used == 700 * MB);
+  return 0;
+}
+
+// An allocation of the same pool takes the lent block, but not one in use.
+static int block_yields_to_its_pool() {
+  device_size = 1000 * MB;
+  Pool pool;
+  CHECK(pool.take_block(600 * MB));
+  pool.begin_use();
+  CHECK(fails(pool, 500 * MB) && !pool.block_lost());
+  pool.end_use();
+  CHECK(pool.get(500 * MB) && pool.block_lost());
+  pool.return_block();
+  CHECK(!pool.block_lost() && device_used == 500 * MB);
+  CHECK(!pool.take_block(600 * MB) && pool.take_block(400 * MB));
+  return 0;
+}
+
+// On a full device buffers come out of the idle block, which is whole again
+// (and only then can be had) with the last of them back.
+static int block_is_carved() {
+  device_size = 1000 * MB;
+  Pool pool;
+  void *a = pool.take_block(600 * MB);
+  pool.return_block();
+  void *b = pool.get(400 * MB), *c = pool.get(300 * MB), *d = pool.get(100 * MB);
+  CHECK(b && c == a && frees == 0 && device_used == 1000 * MB);
+  CHECK(!pool.take_block(600 * MB));
+  pool.put(c);
+  CHECK(pool.get(300 * MB) == c && !pool.take_block(600 * MB));
+  pool.put(c);
+  pool.put(d);
+  CHECK(pool.take_block(600 * MB) == a);
+  CHECK(fails(pool, 700 * MB));  // takes the block, too small all the same
+  CHECK(pool.block_lost());
+  return 0;
+}
+
+// Buffers that a captured graph uses hold the block.
+static int block_and_captures() {
+  device_size = 1000 * MB;
+  Pool pool;
+  pool.take_block(600 * MB);
+  pool.return_block();
+  pool.get(400 * MB);
+  pool.begin_capture();
+  void *c = pool.get(300 * MB);
+  pool.put(c);
+  std::vector<void *> held = pool.end_capture();
+  CHECK(held.size() == 1 && held[0] == c && !pool.take_block(600 * MB));
+  void *d = pool.get(300 * MB);
+  CHECK(d != c);
+  pool.put(d);
+  pool.release(held);
+  CHECK(pool.take_block(600 * MB) == c);
+  return 0;
+}
+
+// A buffer carved before a capture and given back in it: whole at its end.
+static int block_given_back_in_a_capture() {
+  device_size = 1000 * MB;
+  Pool pool;
+  void *a = pool.take_block(600 * MB);
+  pool.return_block();
+  pool.get(400 * MB);
+  void *c = pool.get(300 * MB);
+  pool.begin_capture();
+  pool.put(c);
+  pool.release(pool.end_capture());
+  CHECK(pool.take_block(600 * MB) == a);
+  return 0;
+}
+
+// Another pool's allocation takes the block, lent or idle, and waits for the
+// end of its use.
+static int block_yields_to_other_pools() {
+  device_size = 1000 * MB;
+  Pool a, b;
+  CHECK(a.take_block(600 * MB));
+  a.return_block();
+  void *p = b.get(500 * MB);
+  CHECK(p && !a.block_lost() && device_used == 500 * MB);
+  b.put(p);
+  b.trim();
+  CHECK(a.take_block(600 * MB));
+  p = b.get(500 * MB);
+  CHECK(p && a.block_lost());
+  b.put(p);
+  b.trim();
+  a.return_block();
+  CHECK(a.take_block(600 * MB));
+  a.begin_use();
+  CHECK(fails(b, 500 * MB));
+  std::thread t([&] {
+    std::this_thread::sleep_for(std::chrono::milliseconds(100));
+    a.end_use();
+  });
+  p = b.get(500 * MB);
+  t.join();
+  CHECK(p && a.block_lost());
+  return 0;
+}
+
+// Threads that use, give up and take blocks on a device that holds less than
+// all of them want.
+static int block_from_threads() {
+  device_size = 1500 * MB;
+  std::atomic<int> used{0}, lost{0}, refused{0};
+  auto run = [&](int seed) {
+    Pool pool;
+    unsigned r = unsigned(seed);
+    std::vector<void *> mine;
+    bool lent = false;
+    for (int k = 0; k < 3000; ++k) {
+      r = r * 1664525u + 1013904223u;
+      pool.begin_use();
+      if (lent && pool.block_lost()) {
+        pool.return_block();
+        lent = false;
+        ++lost;
+      }
+      if (!lent) lent = pool.take_block(400 * MB) != nullptr;
+      if (lent) ++used;
+      pool.end_use();
+      try {
+        if (mine.size() < 3) mine.push_back(pool.get((100 + (r >> 24)) * MB));
+      } catch (const sisi::Error &) {
+        ++refused;
+      }
+      if (mine.size() == 3 || (r & 64)) {
+        for (void *p : mine) pool.put(p);
+        mine.clear();
+        if (r & 128) pool.trim();
+      }
+      if (lent && (r & 256)) {
+        pool.return_block();
+        lent = false;
+      }
+    }
+  };
+  std::vector<std::thread> t;
+  for (int k = 0; k < 3; ++k) t.emplace_back(run, k + 1);
+  for (auto &x : t) x.join();
+  printf("used %d lost %d refused %d\n", used.load(), lost.load(), refused.load());
+  CHECK(used > 0 && device_used == 0);
+  return 0;
+}
+
 int main(int argc, char **argv) {
   struct {
     const char *name;
     int (*f)();
   } tests[] = {{"cached_is_trimmable", cached_is_trimmable},
-               {"slab_tails_are_used", slab_tails_are_used}};
+               {"slab_tails_are_used", slab_tails_are_used},
+               {"block_is_kept", block_is_kept},
+               {"block_yields_to_its_pool", block_yields_to_its_pool},
+               {"block_is_carved", block_is_carved},
+               {"block_and_captures", block_and_captures},
+               {"block_given_back_in_a_capture", block_given_back_in_a_capture},
+               {"block_yields_to_other_pools", block_yields_to_other_pools},
+               {"block_from_threads", block_from_threads}};
   for (auto &t : tests)
     if (argc == 2 && std::string(argv[1]) == t.name) return t.f();
   fprintf(stderr, "unknown test\n");

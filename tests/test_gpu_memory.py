@@ -1,0 +1,115 @@
+"""Runs on a device that is almost full: the kept pair integrals are memory
+that any other allocation may have."""
+
+import ctypes
+
+import numpy as np
+import pytest
+
+from conftest import announce
+from test_zz_no_alloc import _hip
+
+pytestmark = pytest.mark.gpu
+
+MB = 1 << 20
+SIZE = (6, 120, 400)  # 0.9 GB of pair integrals
+
+
+class Hog:
+    """Takes all device memory but `leave` bytes."""
+
+    def __init__(self, leave):
+        self.hip, self.p = _hip(), []
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert self.hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        n = free.value - leave
+        while n > 16 * MB:
+            q = ctypes.c_void_p()
+            if self.hip.hipMalloc(ctypes.byref(q), ctypes.c_size_t(n)) == 0:
+                self.p.append(q)
+                return
+            self.hip.hipGetLastError()
+            n -= 16 * MB
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *exc):
+        for q in self.p:
+            assert self.hip.hipFree(q) == 0
+
+
+def options(**kw):
+    from sisi4s_amd import engine
+    d = dict(mixer="DiisMixer", max_residua=6, max_iterations=9, level_shift=2.0,
+             energy_convergence=0.0, amplitudes_convergence=1e-12)
+    d.update(kw)
+    return engine.default_opts(**d)
+
+
+def engine_of(size, seed):
+    from sisi4s_amd import engine
+    e = engine.Engine(*size)
+    e.set_system(*engine.generate_system(seed, *size))
+    return e
+
+
+def same(x, y):
+    # kept and sliced ladder: FP64 sums in another order
+    assert np.abs(np.asarray(x) - y).max() <= 1e-10 * np.abs(y).max()
+
+
+def test_another_engine_takes_the_pair_integrals():
+    other = (8, 130, 600)
+    announce("pair integrals taken by another engine")
+    with engine_of(SIZE, 1) as e, engine_of(other, 2) as f:
+        e.ccsd_solve(options())
+        f.ccsd_solve(options())
+        ref, other_ref = e.energies(), f.energies()
+    with engine_of(SIZE, 1) as e:
+        e.ccsd_begin(options())
+        e.ccsd_iterate(4)
+        with Hog(96 * MB):
+            with engine_of(other, 2) as f:  # 180 MB of vertex alone
+                f.ccsd_solve(options())
+                same(f.energies(), other_ref)
+            e.ccsd_iterate(9)
+        same(e.energies(), ref)
+
+
+def test_triples_take_the_pair_integrals():
+    """(T) between two iterations of a run, then the rest of the run."""
+    announce("pair integrals taken by (T)")
+    with engine_of(SIZE, 1) as e:
+        e.ccsd_begin(options())
+        e.ccsd_iterate(4)
+        t = e.triples()
+        e.ccsd_iterate(9)
+        ref = e.energies()
+    with engine_of(SIZE, 1) as e:
+        e.ccsd_begin(options())
+        e.ccsd_iterate(4)
+        with Hog(96 * MB):
+            same([e.triples()], np.array([t]))
+            e.ccsd_iterate(9)
+        same(e.energies(), ref)
+
+
+def test_next_run_on_one_engine_uses_the_idle_memory():
+    """A mixed run after an FP64 run has the memory of the FP64 run's pair
+    integrals; the FP64 run after it has them again."""
+    announce("mixed run in the idle pair integrals")
+    mixed = dict(precision="bf16x3", bulk_refine_interval=8, switch_threshold=1e-5)
+    with engine_of(SIZE, 1) as e:
+        e.ccsd_solve(options(**mixed))
+        ref_mixed = e.energies()
+        e.ccsd_solve(options())
+        ref = e.energies()
+    with engine_of(SIZE, 1) as e:
+        e.ccsd_solve(options())
+        with Hog(96 * MB):
+            e.ccsd_solve(options(**mixed))
+            # the reduced precision's ladder may keep its planes or not
+            assert np.abs(e.energies() - ref_mixed).max() <= 1e-4 * np.abs(ref_mixed).max()
+            e.ccsd_solve(options())
+            same(e.energies(), ref)
