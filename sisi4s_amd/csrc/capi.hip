@@ -602,6 +602,7 @@ int sisi_ccsd_solve_batched(int nsys, const sisi_dims *dims, const double *const
       for (int s = next++; s < nsys; s = next++) {
         const int rc = guarded([&] {
           Engine e(dims[s]);
+          e.ladder_share = 1.0 / workers;
           const size_t np = size_t(dims[s].No) + dims[s].Nv;
           SISI_REQUIRE(gammas[s] && eps_i[s] && eps_a[s], SISI_ERR_INVALID, "null system input");
           check_finite(gammas[s], size_t(dims[s].NG) * np * np, "CoulombVertex");

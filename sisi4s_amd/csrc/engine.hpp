@@ -255,6 +255,7 @@ class Engine {
   // around such a residual
   bool symmetric_run = false, use_kept_ladder = false, kept_ladder_failed = false;
   double *ladder = nullptr;  // in the pool's block
+  double ladder_share = 1.0;  // of the free memory (less with engines beside this one)
   void drop_ladder();
   std::vector<double> energies;
   // DIIS ring (DiisMixer.cxx:48-180)

@@ -12,8 +12,24 @@ namespace sisi {
 namespace {
 
 // Largest share of the free (or pool-cached) device memory the pair
-// integrals may take: 124 GB of about 240 free at No = 40, Nv = 400.
+// integrals may take: 124 GB of about 260 free at No = 40, Nv = 400.
 constexpr double kLadderShare = 0.55;
+
+// Device memory that the rest of a run will allocate, at most: the mixer's
+// slots not yet filled, the residual's intermediates and permuted copies
+// (about 14 doubles tensors and three vertex-sized ones), with a captured
+// residual a second set of these.
+double run_needs(const Engine &e) {
+  const double n2 = 8.0 * double(e.n1() + e.n2()), g = 8.0 * double(e.NG) * e.Nv * e.Nv;
+  const sisi_ccsd_opts &o = e.opts;
+  double slots = 2.0;
+  if (o.mixer == SISI_MIXER_DIIS) {
+    int filled = 0;
+    for (const DiisSlot &s : e.diis) filled += s.d2.get() != nullptr;
+    slots = std::max(0, std::min(o.max_residua, o.max_iterations - e.iteration + filled) - filled);
+  }
+  return 2.0 * n2 * slots + (o.graphs ? 2.0 : 1.0) * (14.0 * n2 + 3.0 * g);
+}
 
 constexpr int64_t kSlab = 4096;  // pairs per FP32 product of the ladder
 
@@ -300,8 +316,11 @@ bool kept_ladder_build(Engine &e) {
   const int64_t nb = std::min<int64_t>(v, std::max<int64_t>(1, most / (v * v * P)));
   size_t free_b = 0, total_b = 0;
   if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) return false;
-  const double room = kLadderShare * (double(free_b) + double(e.pool.cached_bytes()));
-  if (bytes + 8.0 * double(v * v * P * nb + G * v * P) > room || M >= (int64_t(1) << 31))
+  const double room = e.ladder_share * (double(free_b) + double(e.pool.cached_bytes()));
+  const double temporaries = 8.0 * double(v * v * P * nb + G * v * P);
+  if (bytes + temporaries > kLadderShare * room ||
+      bytes + temporaries + (e.run_active ? run_needs(e) : 0.0) > room ||
+      M >= (int64_t(1) << 31))
     return false;
   double *out = static_cast<double *>(e.pool.take_block(16 * size_t(M) * size_t(K)));
   if (!out) return false;

@@ -22,7 +22,8 @@ bool doubles_symmetric(Engine &e, const double *T2);
 
 // Build the pair integrals (in the pool's block) if the engine has none; false
 // when they do not fit (more than kLadderShare of the memory that is free or
-// cached in the pool, or an allocation fails).  Between begin_use() and
+// cached in the pool, less than the rest of the run needs left over, or an
+// allocation fails).  Between begin_use() and
 // end_use() of the pool.
 bool kept_ladder_build(Engine &e);
 // Device memory of an engine's pair integrals.

@@ -39,6 +39,12 @@ class Hog:
             assert self.hip.hipFree(q) == 0
 
 
+def free_memory():
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert _hip().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
 def options(**kw):
     from sisi4s_amd import engine
     d = dict(mixer="DiisMixer", max_residua=6, max_iterations=9, level_shift=2.0,
@@ -113,3 +119,26 @@ def test_next_run_on_one_engine_uses_the_idle_memory():
             assert np.abs(e.energies() - ref_mixed).max() <= 1e-4 * np.abs(ref_mixed).max()
             e.ccsd_solve(options())
             same(e.energies(), ref)
+
+
+@pytest.mark.parametrize("slots,kept", [(6, True), (200, False)])
+def test_pair_integrals_leave_what_the_run_needs(slots, kept):
+    """0.9 of 2 GB, but not when 200 DIIS slots of 8 MB are still to come."""
+    announce("pair integrals beside %d DIIS slots" % slots)
+    with engine_of(SIZE, 1) as e:
+        with Hog(2000 * MB):
+            before = free_memory()
+            e.ccsd_begin(options(max_residua=slots, max_iterations=300))
+            e.ccsd_iterate(3)
+            assert (before - free_memory() > 900 * MB) == kept
+
+
+def test_threaded_batch_in_little_memory():
+    """Three workers whose pair integrals do not fit together."""
+    from sisi4s_amd import engine
+    systems = [engine.generate_system(s, *SIZE) for s in (1, 2, 3)]
+    announce("threaded batch in little memory")
+    ref, _ = engine.ccsd_solve_batched(systems, options(), workers=1)
+    with Hog(2500 * MB):
+        E, _ = engine.ccsd_solve_batched(systems, options(), workers=3)
+    same(E, np.asarray(ref))
