@@ -96,7 +96,7 @@ class Pool {
       it->second.pop_back();
       hold(p, 1);
       live_.insert(p);
-      if (capturing_) captured_.push_back(p);
+      if (capturing_) captured_.insert(p);
       return p;
     }
     if (void *p = carve(bytes)) return handed_out(p, bytes);
@@ -223,12 +223,18 @@ class Pool {
   void trim() {
     std::lock_guard<std::recursive_mutex> lock(device_wide_mutex());
     (void)hipDeviceSynchronize();
-    // cached buffers, and the slabs none of whose buffers is in use
+    // cached buffers, and the slabs none of whose buffers is in use; not those
+    // that launches of the capture in progress use
+    std::set<size_t> captured;
+    for (void *p : captured_)
+      if (slab_of_.count(p)) captured.insert(slab_of_[p]);
+    auto held = [&](size_t slab) { return slabs_[slab].held > 0 || captured.count(slab); };
     for (auto &kv : free_) {
       std::vector<void *> keep;
       for (void *p : kv.second) {
         auto it = slab_of_.find(p);
-        if ((it != slab_of_.end() && slabs_[it->second].held > 0) || in_block_.count(p)) {
+        if ((it != slab_of_.end() && held(it->second)) || in_block_.count(p) ||
+            captured_.count(p)) {
           keep.push_back(p);
           continue;
         }
@@ -238,10 +244,10 @@ class Pool {
       }
       kv.second.swap(keep);
     }
-    for (auto &s : slabs_)
-      if (s.base && s.held == 0) {
-        (void)hipFree(s.base);
-        s = Slab();
+    for (size_t i = 0; i < slabs_.size(); ++i)
+      if (slabs_[i].base && !held(i)) {
+        (void)hipFree(slabs_[i].base);
+        slabs_[i] = Slab();
       }
     free_idle_block();
   }
@@ -353,7 +359,7 @@ class Pool {
   void free_idle_block() {
     std::lock_guard<std::recursive_mutex> device_lock(device_wide_mutex());
     std::lock_guard<std::mutex> lock(block_m_);
-    if (!block_.base || block_.lent || block_.held > 0) return;
+    if (!block_.base || block_.lent || !in_block_.empty()) return;
     (void)hipDeviceSynchronize();
     (void)hipFree(block_.base);
     block_ = Block();
@@ -397,7 +403,7 @@ class Pool {
   void *handed_out(void *p, size_t bytes) {
     size_[p] = bytes;
     live_.insert(p);
-    if (capturing_) captured_.push_back(p);
+    if (capturing_) captured_.insert(p);
     return p;
   }
   mutable std::mutex block_m_;     // block_: another pool may take it
@@ -412,7 +418,7 @@ class Pool {
   std::map<void *, size_t> size_;
   std::set<void *> reserved_;
   std::set<void *> live_;  // handed out and not yet given back
-  std::vector<void *> captured_;
+  std::set<void *> captured_;
   bool capturing_ = false;
 };
 

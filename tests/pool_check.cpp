@@ -186,6 +186,36 @@ static int block_given_back_in_a_capture() {
   return 0;
 }
 
+// A trim in the course of a capture leaves what captured launches use: a
+// buffer of its own, one in a slab, one in the block.
+static int trim_in_a_capture() {
+  device_size = 1000 * MB;
+  Pool pool;
+  pool.begin_capture();
+  void *a = pool.get(100 * MB), *b = pool.get(1 * MB);
+  pool.put(a);
+  pool.put(b);
+  CHECK(fails(pool, 950 * MB));
+  std::vector<void *> held = pool.end_capture();
+  CHECK(held.size() == 2 && device_used == 108 * MB);
+  CHECK(fails(pool, 950 * MB));
+  pool.release(held);
+  CHECK(pool.get(950 * MB));
+  pool.release_all();
+  void *c = pool.take_block(600 * MB);
+  pool.return_block();
+  pool.get(400 * MB);
+  pool.begin_capture();
+  CHECK(pool.get(300 * MB) == c);
+  pool.put(c);
+  CHECK(fails(pool, 550 * MB));
+  held = pool.end_capture();
+  CHECK(held.size() == 1 && device_used == 1000 * MB);
+  pool.release(held);
+  CHECK(pool.get(550 * MB));
+  return 0;
+}
+
 // Another pool's allocation takes the block, lent or idle, and waits for the
 // end of its use.
 static int block_yields_to_other_pools() {
@@ -272,6 +302,7 @@ int main(int argc, char **argv) {
                {"block_is_carved", block_is_carved},
                {"block_and_captures", block_and_captures},
                {"block_given_back_in_a_capture", block_given_back_in_a_capture},
+               {"trim_in_a_capture", trim_in_a_capture},
                {"block_yields_to_other_pools", block_yields_to_other_pools},
                {"block_from_threads", block_from_threads}};
   for (auto &t : tests)
