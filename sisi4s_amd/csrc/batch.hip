@@ -336,12 +336,10 @@ void record_residual(System &s, int p, int slice, int it, Tape &tape, std::vecto
   tape.upload(pool, stream);
 }
 
-}  // namespace
-
-void ccsd_solve_lockstep(int nsys, const sisi_dims *dims, const double *const *gammas,
-                         const double *const *eps_i, const double *const *eps_a,
-                         const sisi_ccsd_opts &o, double *energies, sisi_ccsd_report *reports,
-                         sisi_lockstep_stats *stats) {
+void solve_lockstep(int nsys, const sisi_dims *dims, const double *const *gammas,
+                    const double *const *eps_i, const double *const *eps_a,
+                    const sisi_ccsd_opts &o, double *energies, sisi_ccsd_report *reports,
+                    sisi_lockstep_stats *stats, bool keep_ladders) {
   SISI_REQUIRE(o.mixer == SISI_MIXER_LINEAR || o.mixer == SISI_MIXER_DIIS, SISI_ERR_INVALID,
                "Mixer not implemented");
   SISI_REQUIRE(o.mixer != SISI_MIXER_DIIS || (o.max_residua >= 1 && o.max_residua <= 30),
@@ -385,15 +383,6 @@ void ccsd_solve_lockstep(int nsys, const sisi_dims *dims, const double *const *g
   std::vector<System> sys(static_cast<size_t>(nsys));
   const int N = o.mixer == SISI_MIXER_DIIS ? o.max_residua : 0;
   const bool bulk_run = o.precision != SISI_FP64;
-  // kept pair integrals (ladder.hpp) for every system or for none: when all of
-  // them together leave most of the memory to the recorded residuals
-  bool keep_ladders = o.ppl != 0 && o.max_iterations >= 3;
-  if (keep_ladders) {
-    size_t free_b = 0, total_b = 0;
-    double need = 0.0;
-    for (int k = 0; k < nsys; ++k) need += kept_ladder_bytes(dims[k].No, dims[k].Nv);
-    keep_ladders = hipMemGetInfo(&free_b, &total_b) == hipSuccess && need <= 0.3 * double(free_b);
-  }
   // set-up: integrals per system (eager, on the system's own stream), fixed
   // buffers, recorded residuals
   for (int k = 0; k < nsys; ++k) {
@@ -740,6 +729,34 @@ void ccsd_solve_lockstep(int nsys, const sisi_dims *dims, const double *const *g
     if (sys[size_t(k)].status != SISI_OK)
       throw Error(sys[size_t(k)].status,
                   "system " + std::to_string(k) + ": " + sys[size_t(k)].error);
+}
+
+}  // namespace
+
+void ccsd_solve_lockstep(int nsys, const sisi_dims *dims, const double *const *gammas,
+                         const double *const *eps_i, const double *const *eps_a,
+                         const sisi_ccsd_opts &o, double *energies, sisi_ccsd_report *reports,
+                         sisi_lockstep_stats *stats) {
+  // kept pair integrals (ladder.hpp) for every system or for none: when all of
+  // them together leave most of the memory to the recorded residuals
+  bool keep_ladders = o.ppl != 0 && o.max_iterations >= 3;
+  if (keep_ladders) {
+    size_t free_b = 0, total_b = 0;
+    double need = 0.0;
+    for (int k = 0; k < nsys; ++k) need += kept_ladder_bytes(dims[k].No, dims[k].Nv);
+    keep_ladders = hipMemGetInfo(&free_b, &total_b) == hipSuccess && need <= 0.3 * double(free_b);
+  }
+  if (keep_ladders) {
+    try {
+      return solve_lockstep(nsys, dims, gammas, eps_i, eps_a, o, energies, reports, stats, true);
+    } catch (const Error &err) {
+      // the recorded residuals or the DIIS rings did not fit beside them: the
+      // same batch with sliced ladders
+      if (err.code != SISI_ERR_ALLOC) throw;
+      if (stats) *stats = sisi_lockstep_stats{};
+    }
+  }
+  solve_lockstep(nsys, dims, gammas, eps_i, eps_a, o, energies, reports, stats, false);
 }
 
 }  // namespace sisi

@@ -39,6 +39,14 @@ class Hog:
             assert self.hip.hipFree(q) == 0
 
 
+@pytest.fixture(scope="module", autouse=True)
+def small_device():
+    """4.5 GB for this file, once: pages that are freed are wiped (33 GB/s)
+    before they can be had again."""
+    with Hog(4500 * MB):
+        yield
+
+
 def free_memory():
     free, total = ctypes.c_size_t(), ctypes.c_size_t()
     assert _hip().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
@@ -142,3 +150,25 @@ def test_threaded_batch_in_little_memory():
     with Hog(2500 * MB):
         E, _ = engine.ccsd_solve_batched(systems, options(), workers=3)
     same(E, np.asarray(ref))
+
+
+def test_lockstep_batch_without_room_for_pair_integrals():
+    """In the memory that a batch needs with sliced ladders (two iterations
+    never keep pair integrals) a longer run, which would keep 134 MB of them,
+    ends with the same energies."""
+    from sisi4s_amd import engine
+    systems = [engine.generate_system(s, 16, 56, 224) for s in (1, 2)]
+    long, short = options(max_residua=2, max_iterations=4), options(max_residua=2, max_iterations=2)
+    ref, _, _ = engine.ccsd_solve_lockstep(systems, long)
+    for leave in range(200, 4000, 64):
+        announce("lockstep batch in %d MB" % leave)
+        with Hog(leave * MB):
+            try:
+                engine.ccsd_solve_lockstep(systems, short)
+            except engine.EngineError as err:
+                assert "allocation" in str(err)
+                continue
+            E, _, _ = engine.ccsd_solve_lockstep(systems, long)
+        same(E, np.asarray(ref))
+        return
+    raise AssertionError("no room at all")
