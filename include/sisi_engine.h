@@ -90,6 +90,8 @@ typedef struct {
   double energy_convergence;     /* energyConvergence, default 1e-6       */
   double level_shift;            /* levelShift, default 0                 */
   int slice_size;                /* integralsSliceSize, <= 0 means No     */
+                                 /* (below No: the ladder in slices only, */
+                                 /* no pair integrals are kept)           */
   int precision;                 /* bulk precision: SISI_FP64/_FP32/_BF16X3 */
   double switch_threshold;       /* |dT|/|T| at which a mixed run switches
                                     to FP64 iterations (default 1e-5)      */

@@ -738,8 +738,11 @@ void ccsd_solve_lockstep(int nsys, const sisi_dims *dims, const double *const *g
                          const sisi_ccsd_opts &o, double *energies, sisi_ccsd_report *reports,
                          sisi_lockstep_stats *stats) {
   // kept pair integrals (ladder.hpp) for every system or for none: when all of
-  // them together leave most of the memory to the recorded residuals
+  // them together leave most of the memory to the recorded residuals, and the
+  // slice width does not ask for less
   bool keep_ladders = o.ppl != 0 && o.max_iterations >= 3;
+  for (int k = 0; k < nsys; ++k)
+    keep_ladders = keep_ladders && !slices_bound_memory(o.slice_size, dims[k].No);
   if (keep_ladders) {
     size_t free_b = 0, total_b = 0;
     double need = 0.0;

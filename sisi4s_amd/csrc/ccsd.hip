@@ -1228,7 +1228,7 @@ struct LadderUse {
 // Residual of a plain iteration.  FP64 and FP32 iterations of a symmetric run
 // contract the ladder with the kept pair integrals when at least one more
 // iteration can use them (building them costs about what one sliced ladder
-// does) and they fit; everything else, and a run that finds no memory on the
+// does), they fit and the slice width does not ask for less; everything else, and a run that finds no memory on the
 // way or whose pair integrals were taken by another allocation, takes the
 // sliced ladder.
 void plain_residual(Engine &e, int prec, double *R1, double *R2) {
@@ -1243,7 +1243,7 @@ void plain_residual(Engine &e, int prec, double *R1, double *R2) {
     ccsd_residual(e, e.iteration, e.run_initial, o.slice_size, e.T1.get(), e.T2.get(), R1, R2);
   };
   if (!mp2 && e.symmetric_run && !e.kept_ladder_failed &&
-      (prec == SISI_FP64 || prec == SISI_FP32) &&
+      (prec == SISI_FP64 || prec == SISI_FP32) && !slices_bound_memory(o.slice_size, e.No) &&
       (e.ladder || o.max_iterations - e.iteration >= 2)) {
     {
       LadderUse use(e);

@@ -17,6 +17,13 @@
 
 namespace sisi {
 
+// A slice width below the default (No) asks for a ladder in less memory than
+// the doubles amplitudes take, (width x width x Nv x Nv): no pair integrals
+// are kept then.
+inline bool slices_bound_memory(int slice_size, int No) {
+  return slice_size > 0 && slice_size < No;
+}
+
 // Whether T2 (device) equals its transpose T_baji bit by bit.
 bool doubles_symmetric(Engine &e, const double *T2);
 

@@ -141,6 +141,16 @@ def test_pair_integrals_leave_what_the_run_needs(slots, kept):
             assert (before - free_memory() > 900 * MB) == kept
 
 
+@pytest.mark.parametrize("width,kept", [(0, True), (6, True), (5, False)])
+def test_slice_width_below_no_bounds_the_memory(width, kept):
+    announce("pair integrals and slice width %d" % width)
+    with engine_of(SIZE, 1) as e:
+        before = free_memory()
+        e.ccsd_begin(options(slice_size=width))
+        e.ccsd_iterate(3)
+        assert (before - free_memory() > 900 * MB) == kept
+
+
 def test_threaded_batch_in_little_memory():
     """Three workers whose pair integrals do not fit together."""
     from sisi4s_amd import engine
