@@ -1350,6 +1350,9 @@ void ccsd_iterate(Engine &e, int n) {
     // phase tolerates anyway, the refinement error scales with the change
     const bool bulk_refine = bulk && !e.coarse_active && o.bulk_refine_interval > 0;
     int prec = bulk ? (e.coarse_active ? o.coarse_precision : o.precision) : SISI_FP64;
+    // anchors and refinement residuals do not read the pair integrals, and the
+    // anchor's planes need memory (plain iterations after them build them again)
+    if ((bulk_refine || refine) && e.ladder) e.drop_residual_graph();
     DBuf R1(&e.pool, e.n1()), R2(&e.pool, e.n2());
     if (bulk_refine) {
       if (!e.anchor.valid || e.anchor.precision != prec ||

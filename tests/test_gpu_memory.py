@@ -2,6 +2,7 @@
 that any other allocation may have."""
 
 import ctypes
+import re
 
 import numpy as np
 import pytest
@@ -182,3 +183,17 @@ def test_lockstep_batch_without_room_for_pair_integrals():
         same(E, np.asarray(ref))
         return
     raise AssertionError("no room at all")
+
+
+def test_refinement_gives_up_the_pair_integrals(monkeypatch, capfd):
+    """FP32 iterations keep pair integrals, the refinement phase after them does
+    not read them: their 0.9 GB count as cached when the first anchor looks
+    for room for its planes."""
+    monkeypatch.setenv("SISI_VERBOSE", "1")
+    announce("refinement phase after plain FP32 iterations")
+    with engine_of(SIZE, 1) as e:
+        e.ccsd_begin(options(precision="fp32", switch_threshold=1e9, refine_interval=4,
+                             refine_precision="fp32"))
+        e.ccsd_iterate(4)
+    said = re.findall(r"([0-9.]+) GB cached", capfd.readouterr().err)
+    assert said and float(said[0]) > 0.9
