@@ -91,6 +91,7 @@ bool operand_ok(const Operand &o, const std::string &g1, const std::string &g2,
 
 // A view with the imaginary plane as one more index.
 View with_plane(View v, int64_t plane) {
+  SISI_REQUIRE(v.order < kMaxOrder, SISI_ERR_INVALID, "contract: complex operand of full order");
   v.len[v.order] = 2;
   v.stride[v.order] = plane;
   ++v.order;
