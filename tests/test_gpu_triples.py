@@ -67,3 +67,21 @@ def test_triples_after_no10_nv50_ccsd():
     et = e.triples()
     ref = triples.triples_energy(T1, T2, g, ei, ea)
     assert abs(et - ref) <= 1e-10 * abs(ref)
+
+
+@pytest.mark.parametrize("Nv", [65, 97, 129, 200])
+def test_triples_blocks_of_several_tiles(Nv):
+    """Blocks of every kind (i < j < k, i = j < k, i < j = k) at sizes where the
+    block products have several tiles along Nv and ragged last ones: two to
+    four of 64 rows in FP64 and FP32; in split-BF16x3 one of 96 (65) and of 128
+    (97), two of 96 (129) and of 128 (200).  Tolerances of the sums above."""
+    No, NG = 3, 12
+    e, g, ei, ea = make(52, No, Nv, NG)
+    T1, T2 = random_amplitudes(Nv, No, seed=Nv, scale=0.02)
+    inp = triples.TriplesInputs(T1, T2, g, ei, ea)
+    for b in ((0, 1, 2), (0, 0, 2), (0, 2, 2)):
+        announce("triples block %s Nv=%d" % (b, Nv))
+        ref = triples.block_energy(inp, b)
+        for prec, tol in (("fp64", 1e-11), ("fp32", 1e-5), ("bf16x3", 1e-4)):
+            x = e.triples(T1, T2, precision=prec, blocks=[b])
+            assert abs(x - ref) <= tol * abs(ref), (b, prec, x, ref)
