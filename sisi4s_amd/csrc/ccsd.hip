@@ -194,16 +194,18 @@ void ccsd_residual(Engine &e, int it, bool initial_doubles, int slice_size, cons
     ctr(e, 1.0, "Gai,Gck->akic", dGai, Gai, 0.0, Xakic, prec);  // cxx:234
     axpby(e, n2, 2.0, T2p, 0.0, Y2b.get());                     // cxx:248-249
     sum(e, -1.0, T2, "bckj", 1.0, Y2, "cbkj");
-    // Xakci (cxx:254-278)
-    DBuf dGabb(&e.pool, G * v * v), dGijb(&e.pool, G * o * o);
-    View dGab = V3(dGabb.get(), G, v, v), dGij = V3(dGijb.get(), G, o, o);
-    copy(e, dGab, Gab);
-    copy(e, dGij, Gij);
-    tctr(-1.0, "Gcl,al->Gac", Gai, T1, 1.0, dGab, prec);  // cxx:270
-    tctr(1.0, "Gdk,di->Gki", Gai, T1, 1.0, dGij, prec);   // cxx:273
-    e.record("dGab4", dGabb.get(), G * v * v);
-    e.record("dGij4", dGijb.get(), G * o * o);
-    ctr(e, 1.0, "Gac,Gki->akci", dGab, dGij, 0.0, Xakci, prec);  // cxx:277-278
+    {
+      // Xakci (cxx:254-278)
+      DBuf dGabb(&e.pool, G * v * v), dGijb(&e.pool, G * o * o);
+      View dGab = V3(dGabb.get(), G, v, v), dGij = V3(dGijb.get(), G, o, o);
+      copy(e, dGab, Gab);
+      copy(e, dGij, Gij);
+      tctr(-1.0, "Gcl,al->Gac", Gai, T1, 1.0, dGab, prec);  // cxx:270
+      tctr(1.0, "Gdk,di->Gki", Gai, T1, 1.0, dGij, prec);   // cxx:273
+      e.record("dGab4", dGabb.get(), G * v * v);
+      e.record("dGij4", dGijb.get(), G * o * o);
+      ctr(e, 1.0, "Gac,Gki->akci", dGab, dGij, 0.0, Xakci, prec);  // cxx:277-278
+    }
     if (!e.distinguishable) {
       e.frozen.push_back(Y2b.get());
       DBuf Qb(&e.pool, v * o * o * o);
@@ -217,7 +219,8 @@ void ccsd_residual(Engine &e, int it, bool initial_doubles, int slice_size, cons
       e.record("Xakci", Xcb.get(), v * o * v * o);
       tctr(1.0, "akic,cbkj->abij", Xakic, Y2, 1.0, R2, prec);
       e.unfreeze(Y2b.get());
-      DBuf Pb(&e.pool, n2);
+      Xkb.reset();
+      DBuf Pb(std::move(Y2b));
       View P = V4(Pb.get(), v, v, o, o);
       tctr(1.0, "akci,bckj->abij", Xakci, T2, 0.0, P, prec);
       axpby(e, n2, -0.5, Pb.get(), 1.0, R2p);
@@ -660,16 +663,18 @@ void ccsd_residual_delta(Engine &e, int slice_size, const double *T1c, const dou
     sum(e, -1.0, T2, "bckj", 1.0, Y2, "cbkj");
     axpby(e, n2, 2.0, d2b.get(), 0.0, dYb.get());
     sum(e, -1.0, d2, "bckj", 1.0, dY2, "cbkj");
-    // Xakci = (dressed Gamma_ab)(dressed Gamma_ij) - V T2 / 2
-    DBuf ddGab(&e.pool, G * v * v), ddGij(&e.pool, G * o * o), Gijn(&e.pool, G * o * o);
-    ctr(e, -1.0, "Gcl,al->Gac", Gai, d1, 0.0, V3(ddGab.get(), G, v, v), prec);
-    ctr(e, 1.0, "Gdk,di->Gki", Gai, d1, 0.0, V3(ddGij.get(), G, o, o), prec);
-    axpby(e, G * o * o, 1.0, A("dGij4"), 0.0, Gijn.get());
-    axpby(e, G * o * o, 1.0, ddGij.get(), 1.0, Gijn.get());
-    ctr(e, 1.0, "Gac,Gki->akci", V3(ddGab.get(), G, v, v), V3(Gijn.get(), G, o, o), 0.0, dXakci,
-        prec);
-    ctr(e, 1.0, "Gac,Gki->akci", V3(A("dGab4"), G, v, v), V3(ddGij.get(), G, o, o), 1.0, dXakci,
-        prec);
+    {
+      // Xakci = (dressed Gamma_ab)(dressed Gamma_ij) - V T2 / 2
+      DBuf ddGab(&e.pool, G * v * v), ddGij(&e.pool, G * o * o), Gijn(&e.pool, G * o * o);
+      ctr(e, -1.0, "Gcl,al->Gac", Gai, d1, 0.0, V3(ddGab.get(), G, v, v), prec);
+      ctr(e, 1.0, "Gdk,di->Gki", Gai, d1, 0.0, V3(ddGij.get(), G, o, o), prec);
+      axpby(e, G * o * o, 1.0, A("dGij4"), 0.0, Gijn.get());
+      axpby(e, G * o * o, 1.0, ddGij.get(), 1.0, Gijn.get());
+      ctr(e, 1.0, "Gac,Gki->akci", V3(ddGab.get(), G, v, v), V3(Gijn.get(), G, o, o), 0.0, dXakci,
+          prec);
+      ctr(e, 1.0, "Gac,Gki->akci", V3(A("dGab4"), G, v, v), V3(ddGij.get(), G, o, o), 1.0, dXakci,
+          prec);
+    }
     View XakciA = V4(A("Xakci"), v, o, v, o);
     if (!e.distinguishable) {
       e.frozen.push_back(dYb.get());
@@ -686,7 +691,8 @@ void ccsd_residual_delta(Engine &e, int slice_size, const double *T1c, const dou
       ctr(e, 1.0, "akic,cbkj->abij", dXakic, Y2, 1.0, dR2, prec);
       ctr(e, 1.0, "akic,cbkj->abij", V4(A("Bakic"), v, o, o, v), dY2, 1.0, dR2, prec);
       e.unfreeze(dYb.get());
-      DBuf dPb(&e.pool, n2);
+      dXkb.reset();
+      DBuf dPb(std::move(dYb));
       View dP = V4(dPb.get(), v, v, o, o);
       ctr(e, 1.0, "akci,bckj->abij", dXakci, T2, 0.0, dP, prec);
       ctr(e, 1.0, "akci,bckj->abij", XakciA, d2, 1.0, dP, prec);
