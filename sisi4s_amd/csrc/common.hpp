@@ -64,8 +64,8 @@ inline std::recursive_mutex &device_wide_mutex() {
 // A pool also holds at most one block: a large buffer whose contents its owner
 // can do without (the pair integrals of the ladder, 124 GB at No = 40, Nv =
 // 400).  It is there for whoever needs memory.  While it is not lent, the
-// pool's own buffers are carved out of it once hipMalloc fails; and an
-// allocation that would fail takes the block of its own pool or of another
+// pool's own buffers are carved out of it when less than a quarter of the
+// device is free; and an allocation that would fail takes the block of its own pool or of another
 // pool of the process, lent or not, back to the device (block_lost() then
 // tells the owner), except while the owner has work in hand that reads it
 // (begin_use() to end_use()).  Carving comes before freeing since pages that
@@ -100,7 +100,8 @@ class Pool {
       return p;
     }
     if (void *p = carve(bytes)) return handed_out(p, bytes);
-    void *p = device_malloc(bytes);
+    void *p = prefer_block(bytes) ? carve_block(bytes) : nullptr;
+    if (!p) p = device_malloc(bytes);
     if (!p) p = carve_block(bytes);
     if (!p) {
       // Drop cached buffers and retry, then take blocks.
@@ -152,6 +153,13 @@ class Pool {
     block_.lent = false;
     lost_ = false;
   }
+  // Size of the block if it can be had whole.
+  size_t idle_block() const {
+    std::lock_guard<std::mutex> lock(block_m_);
+    return block_.base && !block_.lent && block_.held == 0 ? block_.size : 0;
+  }
+  // Some of the pool's own buffers are carved out of it.
+  bool block_carved() const { return !in_block_.empty(); }
   // A lent block was taken by another allocation.
   bool block_lost() const { return lost_; }
   // The owner issues work that reads or writes the block.
@@ -216,9 +224,7 @@ class Pool {
         if (!slab_of_.count(p) && !in_block_.count(p)) b += kv.first;
     for (const auto &s : slabs_)
       if (s.base && s.held == 0) b += s.size;
-    std::lock_guard<std::mutex> lock(block_m_);
-    if (block_.base && !block_.lent && block_.held == 0) b += block_.size;
-    return b;
+    return b + idle_block();
   }
   void trim() {
     std::lock_guard<std::recursive_mutex> lock(device_wide_mutex());
@@ -346,6 +352,15 @@ class Pool {
   static std::vector<Pool *> &registry() {
     static auto *r = new std::vector<Pool *>;  // outlives every pool
     return *r;
+  }
+  // A quarter of the device stays free for others while there is an idle block.
+  bool prefer_block(size_t bytes) {
+    {
+      std::lock_guard<std::mutex> lock(block_m_);
+      if (!block_.base || block_.lent) return false;
+    }
+    size_t free_b = 0, total_b = 0;
+    return hipMemGetInfo(&free_b, &total_b) == hipSuccess && free_b < bytes + total_b / 4;
   }
   void *carve_block(size_t bytes) {
     std::lock_guard<std::mutex> lock(block_m_);

@@ -216,6 +216,9 @@ class Engine {
 
   void drop_triples_cache() {
     drop_eom();
+    drop_triples_operands();
+  }
+  void drop_triples_operands() {
     Vt.reset();
     Vt2.reset();
     VP.reset();

@@ -310,6 +310,9 @@ bool kept_ladder_build(Engine &e) {
   const int64_t K = rows.pairs(), M = rows.count();
   const double bytes = kept_ladder_bytes(o, v);
   if (o * o > 65535 || P > 65535) return false;  // grids of pack_pairs
+  // an earlier run's block may hold the operands that (T) caches; it builds
+  // them again in a fraction of an iteration
+  if (e.pool.block_carved()) e.drop_triples_operands();
   // a slice of b: a temporary of v^2 (o + v) doubles per b, at most an eighth
   // of the result and 2 GB (it stays in the engine's pool)
   const int64_t most = std::min<int64_t>(int64_t(1) << 28, M * K / 4);
@@ -318,7 +321,9 @@ bool kept_ladder_build(Engine &e) {
   if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) return false;
   const double room = e.ladder_share * (double(free_b) + double(e.pool.cached_bytes()));
   const double temporaries = 8.0 * double(v * v * P * nb + G * v * P);
-  if (bytes + temporaries > kLadderShare * room ||
+  // (a block kept from an earlier run has its share already)
+  const bool kept = double(e.pool.idle_block()) >= bytes;
+  if ((!kept && bytes + temporaries > kLadderShare * room) ||
       bytes + temporaries + (e.run_active ? run_needs(e) : 0.0) > room ||
       M >= (int64_t(1) << 31))
     return false;

@@ -39,6 +39,12 @@ hipError_t hipFree(void *p) {
   ++frees;
   return hipSuccess;
 }
+hipError_t hipMemGetInfo(size_t *free_b, size_t *total_b) {
+  std::lock_guard<std::mutex> lock(device_m);
+  *free_b = device_size - device_used;
+  *total_b = device_size;
+  return hipSuccess;
+}
 hipError_t hipDeviceSynchronize() { return hipSuccess; }
 hipError_t hipGetLastError() { return hipSuccess; }
 hipError_t hipGetDevice(int *d) {
@@ -131,14 +137,29 @@ static int block_yields_to_its_pool() {
   return 0;
 }
 
+// Buffers come from the device while a quarter of it stays free, then out of
+// the idle block, and when that has no room from the device again.
+static int quarter_stays_free() {
+  device_size = 1000 * MB;
+  Pool pool;
+  void *a = pool.take_block(300 * MB);
+  pool.get(100 * MB);
+  pool.return_block();
+  CHECK(pool.get(350 * MB) && device_used == 750 * MB);
+  CHECK(pool.get(200 * MB) == a && device_used == 750 * MB);
+  CHECK(pool.get(200 * MB) && device_used == 950 * MB);
+  return 0;
+}
+
 // On a full device buffers come out of the idle block, which is whole again
 // (and only then can be had) with the last of them back.
 static int block_is_carved() {
   device_size = 1000 * MB;
   Pool pool;
   void *a = pool.take_block(600 * MB);
+  void *b = pool.get(400 * MB);
   pool.return_block();
-  void *b = pool.get(400 * MB), *c = pool.get(300 * MB), *d = pool.get(100 * MB);
+  void *c = pool.get(300 * MB), *d = pool.get(100 * MB);
   CHECK(b && c == a && frees == 0 && device_used == 1000 * MB);
   CHECK(!pool.take_block(600 * MB));
   pool.put(c);
@@ -156,8 +177,8 @@ static int block_and_captures() {
   device_size = 1000 * MB;
   Pool pool;
   pool.take_block(600 * MB);
-  pool.return_block();
   pool.get(400 * MB);
+  pool.return_block();
   pool.begin_capture();
   void *c = pool.get(300 * MB);
   pool.put(c);
@@ -176,8 +197,8 @@ static int block_given_back_in_a_capture() {
   device_size = 1000 * MB;
   Pool pool;
   void *a = pool.take_block(600 * MB);
-  pool.return_block();
   pool.get(400 * MB);
+  pool.return_block();
   void *c = pool.get(300 * MB);
   pool.begin_capture();
   pool.put(c);
@@ -203,8 +224,8 @@ static int trim_in_a_capture() {
   CHECK(pool.get(950 * MB));
   pool.release_all();
   void *c = pool.take_block(600 * MB);
-  pool.return_block();
   pool.get(400 * MB);
+  pool.return_block();
   pool.begin_capture();
   CHECK(pool.get(300 * MB) == c);
   pool.put(c);
@@ -299,6 +320,7 @@ int main(int argc, char **argv) {
                {"slab_tails_are_used", slab_tails_are_used},
                {"block_is_kept", block_is_kept},
                {"block_yields_to_its_pool", block_yields_to_its_pool},
+               {"quarter_stays_free", quarter_stays_free},
                {"block_is_carved", block_is_carved},
                {"block_and_captures", block_and_captures},
                {"block_given_back_in_a_capture", block_given_back_in_a_capture},

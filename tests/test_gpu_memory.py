@@ -130,6 +130,26 @@ def test_next_run_on_one_engine_uses_the_idle_memory():
             same(e.energies(), ref)
 
 
+def test_next_run_after_triples_keeps_pair_integrals():
+    """(T) caches its operands in the idle pair integrals of the run before it;
+    the next run has them whole again (the same products as the first)."""
+    announce("run after (T) in the idle pair integrals")
+
+    def flops(e):
+        e.enable_stats(True)
+        e.reset_stats()
+        e.ccsd_solve(options())
+        return e.stats()["gemm_flops"][0], e.energies()
+    with engine_of(SIZE, 1) as e:
+        first, ref = flops(e)
+        with Hog(600 * MB):
+            e.triples()
+            second, E = flops(e)
+        same(E, ref)
+        # the build of the pair integrals included
+        assert second == first
+
+
 @pytest.mark.parametrize("slots,kept", [(6, True), (200, False)])
 def test_pair_integrals_leave_what_the_run_needs(slots, kept):
     """0.9 of 2 GB, but not when 200 DIIS slots of 8 MB are still to come."""
