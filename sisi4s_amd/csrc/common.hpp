@@ -100,7 +100,7 @@ class Pool {
       return p;
     }
     if (void *p = carve(bytes)) return handed_out(p, bytes);
-    void *p = prefer_block(bytes) ? carve_block(bytes) : nullptr;
+    void *p = bytes > kSlabMax && prefer_block(bytes) ? carve_block(bytes) : nullptr;
     if (!p) p = device_malloc(bytes);
     if (!p) p = carve_block(bytes);
     if (!p) {
@@ -126,7 +126,7 @@ class Pool {
   void *take_block(size_t bytes) {
     {
       std::lock_guard<std::mutex> lock(block_m_);
-      if (block_.base && (block_.lent || block_.held > 0)) return nullptr;
+      if (block_.base && (block_.lent || !block_.whole())) return nullptr;
       if (block_.base && block_.size >= bytes) {
         block_.lent = true;
         return block_.base;
@@ -143,6 +143,7 @@ class Pool {
     block_ = Block();
     block_.base = static_cast<char *>(p);
     block_.size = bytes;
+    block_.room[block_.base] = bytes;
     block_.lent = true;
     (void)hipGetDevice(&block_.device);
     return p;
@@ -156,7 +157,7 @@ class Pool {
   // Size of the block if it can be had whole.
   size_t idle_block() const {
     std::lock_guard<std::mutex> lock(block_m_);
-    return block_.base && !block_.lent && block_.held == 0 ? block_.size : 0;
+    return !block_.lent && block_.whole() ? block_.size : 0;
   }
   // Some of the pool's own buffers are carved out of it.
   bool block_carved() const { return !in_block_.empty(); }
@@ -173,8 +174,7 @@ class Pool {
     if (it == size_.end()) return;
     live_.erase(p);
     if (reserved_.count(p)) return;  // held by a captured graph
-    free_[it->second].push_back(p);
-    hold(p, -1);
+    recycle(p);
   }
   // Graph capture: every buffer handed out between begin_capture and
   // end_capture is referenced by the captured graph, so end_capture takes
@@ -192,31 +192,24 @@ class Pool {
       if (reserved_.count(p)) continue;
       reserved_.insert(p);
       held.push_back(p);
-      auto &fl = free_[size_[p]];
-      for (size_t k = 0; k < fl.size(); ++k)
-        if (fl[k] == p) {
-          fl.erase(fl.begin() + k);
-          hold(p, 1);
-          break;
-        }
+      if (unlist(p)) hold(p, 1);
     }
     captured_.clear();
-    std::lock_guard<std::mutex> lock(block_m_);
-    if (block_.held == 0) make_block_whole();
+    // what else of the block was given back in the course of the capture
+    const std::set<void *> carved = in_block_;
+    for (void *p : carved)
+      if (unlist(p)) recycle(p);
     return held;
   }
   void release(const std::vector<void *> &held) {
     for (void *p : held) {
       reserved_.erase(p);
-      auto it = size_.find(p);
-      if (it != size_.end() && !live_.count(p)) {
-        free_[it->second].push_back(p);
-        hold(p, -1);
-      }
+      if (size_.count(p) && !live_.count(p)) recycle(p);
     }
   }
-  // Device memory that trim() gives back: the free lists, of slabs those none
-  // of whose buffers is in use, and so the block when it is not lent.
+  // Device memory that can be had again: what trim() gives back (the free
+  // lists, of slabs those none of whose buffers is in use) and what is free of
+  // a block that is not lent.
   size_t cached_bytes() const {
     size_t b = 0;
     for (const auto &kv : free_)
@@ -224,7 +217,10 @@ class Pool {
         if (!slab_of_.count(p) && !in_block_.count(p)) b += kv.first;
     for (const auto &s : slabs_)
       if (s.base && s.held == 0) b += s.size;
-    return b + idle_block();
+    std::lock_guard<std::mutex> lock(block_m_);
+    if (block_.base && !block_.lent)
+      for (const auto &r : block_.room) b += r.second;
+    return b;
   }
   void trim() {
     std::lock_guard<std::recursive_mutex> lock(device_wide_mutex());
@@ -316,21 +312,27 @@ class Pool {
   void hold(void *p, int d) {
     auto it = slab_of_.find(p);
     if (it != slab_of_.end()) slabs_[it->second].held += d;
-    if (!in_block_.count(p)) return;
-    std::lock_guard<std::mutex> lock(block_m_);
-    block_.held += d;
-    if (block_.held == 0 && !capturing_) make_block_whole();
   }
-  // With the last of its buffers back (during a capture not before its end:
-  // the captured launches may use them) the block is one again.
-  void make_block_whole() {
-    for (void *q : in_block_) {
-      auto &fl = free_[size_[q]];
-      fl.erase(std::remove(fl.begin(), fl.end(), q), fl.end());
-      size_.erase(q);
+  // A buffer nobody owns: into its free list, or back into the block (in the
+  // course of a capture into the list: end_capture() reserves it there).
+  void recycle(void *p) {
+    if (in_block_.count(p) && !capturing_) {
+      std::lock_guard<std::mutex> lock(block_m_);
+      block_.give(static_cast<char *>(p), size_[p]);
+      in_block_.erase(p);
+      size_.erase(p);
+      return;
     }
-    in_block_.clear();
-    block_.used = 0;
+    free_[size_[p]].push_back(p);
+    hold(p, -1);
+  }
+  // Takes a buffer out of its free list; false when it is not in it.
+  bool unlist(void *p) {
+    auto &fl = free_[size_[p]];
+    auto it = std::find(fl.begin(), fl.end(), p);
+    if (it == fl.end()) return false;
+    fl.erase(it);
+    return true;
   }
   static void *device_malloc(size_t bytes) {
     void *p = nullptr;
@@ -340,9 +342,38 @@ class Pool {
   }
   struct Block {
     char *base = nullptr;
-    size_t size = 0, used = 0;
-    int held = 0, device = 0;
+    size_t size = 0;
+    int device = 0;
     bool lent = false;
+    std::map<char *, size_t> room;  // free ranges, none next to another
+    bool whole() const { return base && room.size() == 1 && room.begin()->second == size; }
+    // the smallest range that holds n bytes
+    char *take(size_t n) {
+      auto best = room.end();
+      for (auto it = room.begin(); it != room.end(); ++it)
+        if (it->second >= n && (best == room.end() || it->second < best->second)) best = it;
+      if (best == room.end()) return nullptr;
+      char *p = best->first;
+      const size_t rest = best->second - n;
+      room.erase(best);
+      if (rest > 0) room[p + n] = rest;
+      return p;
+    }
+    void give(char *p, size_t n) {
+      auto it = room.emplace(p, n).first;
+      auto next = std::next(it);
+      if (next != room.end() && p + n == next->first) {
+        it->second += next->second;
+        room.erase(next);
+      }
+      if (it != room.begin()) {
+        auto prev = std::prev(it);
+        if (prev->first + prev->second == p) {
+          prev->second += it->second;
+          room.erase(it);
+        }
+      }
+    }
   };
   static constexpr int kWaits = 50;  // of 20 ms, for blocks in use
   static std::mutex &registry_mutex() {
@@ -353,28 +384,29 @@ class Pool {
     static auto *r = new std::vector<Pool *>;  // outlives every pool
     return *r;
   }
-  // A quarter of the device stays free for others while there is an idle block.
+  // A quarter of the device stays free for others while there is an idle
+  // block; once it has come to that the block is asked first.
   bool prefer_block(size_t bytes) {
     {
       std::lock_guard<std::mutex> lock(block_m_);
-      if (!block_.base || block_.lent) return false;
+      if (!block_.base || block_.lent) return block_first_ = false;
     }
     size_t free_b = 0, total_b = 0;
-    return hipMemGetInfo(&free_b, &total_b) == hipSuccess && free_b < bytes + total_b / 4;
+    if (!block_first_)
+      block_first_ = hipMemGetInfo(&free_b, &total_b) == hipSuccess && free_b < bytes + total_b / 4;
+    return block_first_;
   }
   void *carve_block(size_t bytes) {
     std::lock_guard<std::mutex> lock(block_m_);
-    if (!block_.base || block_.lent || block_.size - block_.used < bytes) return nullptr;
-    void *p = block_.base + block_.used;
-    block_.used += bytes;
-    ++block_.held;
-    in_block_.insert(p);
+    if (!block_.base || block_.lent) return nullptr;
+    void *p = block_.take(bytes);
+    if (p) in_block_.insert(p);
     return p;
   }
   void free_idle_block() {
     std::lock_guard<std::recursive_mutex> device_lock(device_wide_mutex());
     std::lock_guard<std::mutex> lock(block_m_);
-    if (!block_.base || block_.lent || !in_block_.empty()) return;
+    if (block_.lent || !block_.whole()) return;
     (void)hipDeviceSynchronize();
     (void)hipFree(block_.base);
     block_ = Block();
@@ -383,7 +415,7 @@ class Pool {
   // busy_ (so that its owner is not using it) and the device-wide lock.
   bool surrender(int device) {
     std::lock_guard<std::mutex> lock(block_m_);
-    if (!block_.base || block_.held > 0 || block_.device != device) return false;
+    if (!block_.whole() || block_.device != device) return false;
     (void)hipDeviceSynchronize();
     (void)hipFree(block_.base);
     lost_ = block_.lent;
@@ -426,6 +458,7 @@ class Pool {
   std::set<void *> in_block_;      // buffers carved out of it
   std::atomic<bool> busy_{false};  // in use by its owner, or about to be freed
   std::atomic<bool> lost_{false};
+  bool block_first_ = false;
   std::vector<Slab> slabs_;
   std::map<void *, size_t> slab_of_;
   size_t next_slab_ = kSlabFirst;

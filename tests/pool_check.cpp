@@ -172,6 +172,31 @@ static int block_is_carved() {
   return 0;
 }
 
+// What comes back to the block joins: a buffer larger than each of them, and
+// all of it counts as cached.
+static int block_ranges_join() {
+  device_size = 1000 * MB;
+  Pool pool;
+  char *a = static_cast<char *>(pool.take_block(600 * MB));
+  pool.get(400 * MB);
+  pool.return_block();
+  void *b[4];
+  for (int k = 0; k < 4; ++k) b[k] = pool.get(150 * MB);
+  CHECK(b[3] == a + 450 * MB && pool.cached_bytes() == 0);
+  pool.put(b[2]);
+  pool.put(b[0]);
+  pool.put(b[1]);
+  CHECK(pool.cached_bytes() == 450 * MB);
+  void *c = pool.get(440 * MB), *d = pool.get(10 * MB);
+  CHECK(c == a && d && fails(pool, 100 * MB));
+  pool.put(c);
+  pool.put(b[3]);
+  CHECK(pool.block_carved() && pool.idle_block() == 0);
+  pool.put(d);
+  CHECK(pool.get(590 * MB) == a);
+  return 0;
+}
+
 // Buffers that a captured graph uses hold the block.
 static int block_and_captures() {
   device_size = 1000 * MB;
@@ -322,6 +347,7 @@ int main(int argc, char **argv) {
                {"block_yields_to_its_pool", block_yields_to_its_pool},
                {"quarter_stays_free", quarter_stays_free},
                {"block_is_carved", block_is_carved},
+               {"block_ranges_join", block_ranges_join},
                {"block_and_captures", block_and_captures},
                {"block_given_back_in_a_capture", block_given_back_in_a_capture},
                {"trim_in_a_capture", trim_in_a_capture},
