@@ -113,12 +113,25 @@ static int block_is_kept() {
   device_size = 1000 * MB;
   Pool pool;
   void *a = pool.take_block(600 * MB);
-  CHECK(a && !pool.take_block(1 * MB));
+  CHECK(a && !pool.take_block(100 * MB));
   pool.return_block();
   CHECK(pool.cached_bytes() == 600 * MB);
   CHECK(pool.take_block(500 * MB) == a && frees == 0);
   pool.return_block();
   CHECK(pool.take_block(700 * MB) && device_used == 700 * MB);
+  return 0;
+}
+
+// A block that fits a slab comes out of one and goes back to the free lists.
+static int small_blocks_are_buffers() {
+  device_size = 1000 * MB;
+  Pool pool;
+  pool.get(2 * MB);
+  const size_t used = device_used;
+  void *a = pool.take_block(4 * MB);
+  CHECK(a && device_used == used && !pool.block_lost() && !pool.block_carved());
+  pool.return_block();
+  CHECK(pool.get(4 * MB) == a && pool.idle_block() == 0);
   return 0;
 }
 
@@ -344,6 +357,7 @@ int main(int argc, char **argv) {
   } tests[] = {{"cached_is_trimmable", cached_is_trimmable},
                {"slab_tails_are_used", slab_tails_are_used},
                {"block_is_kept", block_is_kept},
+               {"small_blocks_are_buffers", small_blocks_are_buffers},
                {"block_yields_to_its_pool", block_yields_to_its_pool},
                {"quarter_stays_free", quarter_stays_free},
                {"block_is_carved", block_is_carved},

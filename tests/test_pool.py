@@ -23,7 +23,8 @@ def pool_check(tmp_path_factory):
 
 
 @pytest.mark.parametrize("name", [
-    "cached_is_trimmable", "slab_tails_are_used", "block_is_kept", "block_yields_to_its_pool",
+    "cached_is_trimmable", "slab_tails_are_used", "block_is_kept", "small_blocks_are_buffers",
+    "block_yields_to_its_pool",
     "quarter_stays_free", "block_is_carved", "block_ranges_join",
     "block_and_captures", "block_given_back_in_a_capture",
     "trim_in_a_capture", "block_yields_to_other_pools", "block_from_threads"])
