@@ -403,7 +403,7 @@ class Pool {
       if (!block_.base || block_.lent) return block_first_ = false;
     }
     size_t free_b = 0, total_b = 0;
-    if (!block_first_)
+    if (!block_first_ && !capturing_)
       block_first_ = hipMemGetInfo(&free_b, &total_b) == hipSuccess && free_b < bytes + total_b / 4;
     return block_first_;
   }

@@ -74,15 +74,17 @@ def same(x, y):
     assert np.abs(np.asarray(x) - y).max() <= 1e-10 * np.abs(y).max()
 
 
-def test_another_engine_takes_the_pair_integrals():
+@pytest.mark.parametrize("graphs", [0, 1])
+def test_another_engine_takes_the_pair_integrals(graphs):
+    """Between two iterations, also of a captured residual that reads them."""
     other = (8, 130, 600)
-    announce("pair integrals taken by another engine")
+    announce("pair integrals taken by another engine, graphs=%d" % graphs)
     with engine_of(SIZE, 1) as e, engine_of(other, 2) as f:
-        e.ccsd_solve(options())
+        e.ccsd_solve(options(graphs=graphs))
         f.ccsd_solve(options())
         ref, other_ref = e.energies(), f.energies()
     with engine_of(SIZE, 1) as e:
-        e.ccsd_begin(options())
+        e.ccsd_begin(options(graphs=graphs))
         e.ccsd_iterate(4)
         with Hog(96 * MB):
             with engine_of(other, 2) as f:  # 180 MB of vertex alone
